@@ -98,15 +98,15 @@ __global__ void k_group_maxlen(const int4* __restrict__ seg, DevHdr* hdr, int bo
 }
 
 // (node, live points, depth, parent) of the topmost violators, plus the node
-// count of the subtree before its rebuild
-__global__ void k_node_info(Pool pool, const int* __restrict__ top, int n, int4* __restrict__ out,
-                            int* __restrict__ nodes_before) {
+// count of the subtree before its rebuild (pend: what k_find_top added up)
+__global__ void k_node_info(Pool pool, const int* __restrict__ top, const int* __restrict__ pend, int n,
+                            int4* __restrict__ out, int* __restrict__ nodes_before) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     int u = top[2 * i];
     int4 c = pool.cnt[u];
     out[i] = make_int4(u, c.x - c.y, c.w, pool.par[u]);
-    nodes_before[i] = top[2 * i + 1];
+    nodes_before[i] = top[2 * i + 1] + pend[u];
 }
 
 
@@ -160,13 +160,13 @@ struct DevStatus {
     int top_before[TOPINFO_CAP];
 };
 constexpr size_t STATUS_SHORT = offsetof(DevStatus, top_info);  // header + root summary
-__global__ void k_top_info(Pool pool, const int* __restrict__ top, DevStatus* s) {
+__global__ void k_top_info(Pool pool, const int* __restrict__ top, const int* __restrict__ pend, DevStatus* s) {
     const int n = min(s->hdr.top_count, TOPINFO_CAP);
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         const int u = top[2 * i];
         const int4 c = pool.cnt[u];
         s->top_info[i] = make_int4(u, c.x - c.y, c.w, pool.par[u]);
-        s->top_before[i] = top[2 * i + 1];
+        s->top_before[i] = top[2 * i + 1] + pend[u];
     }
 }
 // Enumerate: the walk must have written exactly the live points the
@@ -948,7 +948,7 @@ int refit_finish(ikd_tree_t t) {
     CHK(ensure(t, B_PEND, std::max<long long>(t->cap, 16), &pend));
     CHK(ensure(t, B_START, cap, &start));
     launch_refit_up(t->pool, t->prm, dirty, pend, start, t->d_hdr, viol, defer, t->st);
-    launch_find_top(t->pool, viol, (int)cap, t->d_hdr, top, t->st);
+    launch_find_top(t->pool, viol, (int)cap, t->d_hdr, top, pend, t->st);
     launch_clear_viol(t->pool, viol, (int)cap, t->d_hdr, t->st);
     HIPCHK(hipGetLastError());
     return IKD_OK;
@@ -1033,8 +1033,9 @@ int rebuild_tops(ikd_tree_t t) {
         // the header, the root summary and the first subtrees to rebuild in one wait
         // (the refit's list; after a pass of rebuilds the list is empty)
         const int* top = iter == 0 ? reinterpret_cast<const int*>(t->b[B_TOP].p) : nullptr;
+        const int* pend = reinterpret_cast<const int*>(t->b[B_PEND].p);
         hipLaunchKernelGGL(k_root_info, dim3(1), dim3(1), 0, st, t->pool, t->d_root);
-        if (top) hipLaunchKernelGGL(k_top_info, dim3(1), dim3(256), 0, st, t->pool, top, t->d_status);
+        if (top) hipLaunchKernelGGL(k_top_info, dim3(1), dim3(256), 0, st, t->pool, top, pend, t->d_status);
         CHK(read_status(t, top ? sizeof(DevStatus) : STATUS_SHORT));
         int ntop = t->h_hdr->top_count;
         CHK(check_count(t, "rebuild: subtrees", ntop, 0, t->pool_used));
@@ -1051,7 +1052,7 @@ int rebuild_tops(ikd_tree_t t) {
             CHK(ensure(t, B_TOP, 2 * ntop, &topb));
             CHK(ensure(t, B_INFO, ntop, &info));
             CHK(ensure(t, B_SEEDS, ntop, &before));
-            hipLaunchKernelGGL(k_node_info, dim3(nblk(ntop)), dim3(BS), 0, st, t->pool, topb, ntop, info, before);
+            hipLaunchKernelGGL(k_node_info, dim3(nblk(ntop)), dim3(BS), 0, st, t->pool, topb, pend, ntop, info, before);
             HIPCHK(hipMemcpyAsync(hinfo.data(), info, ntop * sizeof(int4), hipMemcpyDeviceToHost, st));
             HIPCHK(hipMemcpyAsync(hbefore.data(), before, ntop * sizeof(int), hipMemcpyDeviceToHost, st));
             HIPCHK(wait_stream(t));

@@ -112,7 +112,7 @@ void launch_mark_dirty(Pool pool, const int* seeds, const int* nseeds_dev, int b
 void launch_defer_check(Pool pool, Params prm, const int* defer, int n, int4* info, int* before, int* keep,
                         hipStream_t s);
 void launch_defer_clear(Pool pool, const int* defer, int n, hipStream_t s);
-void launch_find_top(Pool pool, const int* viol, int bound, DevHdr* hdr, int* top, hipStream_t s);
+void launch_find_top(Pool pool, const int* viol, int bound, DevHdr* hdr, int* top, int* pend, hipStream_t s);
 void launch_clear_viol(Pool pool, const int* viol, int bound, DevHdr* hdr, hipStream_t s);
 // root statistics of a root the build just created (0 when it has <= 3 nodes)
 void launch_root_alpha_fresh(Pool pool, DevHdr* hdr, hipStream_t s);

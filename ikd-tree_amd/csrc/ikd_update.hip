@@ -283,24 +283,33 @@ void launch_defer_clear(Pool pool, const int* defer, int n, hipStream_t s) {
 
 // A violator is rebuilt only if no ancestor violates too: the reference
 // checks bottom-up on the way out of the recursion and ends up rebuilding
-// the highest violating node of the path (cpp:862-863, 706-707).
-__global__ void k_find_top(Pool pool, const int* __restrict__ viol, DevHdr* hdr, int* __restrict__ top) {
+// the highest violating node of the path (cpp:862-863, 706-707).  The refit
+// left post-rebuild counts in the violators below it, so the topmost one's
+// node count misses the nodes those still hold; they are added up in pend
+// (zero for every refit node by now), because a rebuild that records removed
+// points walks them all.
+__global__ void k_find_top(Pool pool, const int* __restrict__ viol, DevHdr* hdr, int* __restrict__ top,
+                           int* __restrict__ pend) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= hdr->viol_count) return;
     int v = viol[2 * i];
-    int u = v;
+    int u = v, topmost = -1;
     for (int step = 0; u != ROOT; ++step) {
         u = pool.par[u];
         if (step > WALK_LIMIT || u < ROOT) {
             atomicOr(&hdr->overflow, 16);
             return;
         }
-        if (pool.meta[u] & M_VIOL) return;
+        if (pool.meta[u] & M_VIOL) topmost = u;
+    }
+    if (topmost >= 0) {
+        atomicAdd(&pend[topmost], viol[2 * i + 1] - pool.cnt[v].x);
+        return;
     }
     atomicOr(&pool.meta[v], M_TOP);
     int pos = atomicAdd(&hdr->top_count, 1);
     top[2 * pos] = v;
-    top[2 * pos + 1] = viol[2 * i + 1];  // nodes in the subtree before the rebuild
+    top[2 * pos + 1] = viol[2 * i + 1];  // nodes in the subtree before the rebuild, without pend's
 }
 
 __global__ void k_clear_viol(Pool pool, const int* __restrict__ viol, DevHdr* hdr) {
@@ -340,9 +349,9 @@ void launch_mark_dirty(Pool pool, const int* seeds, const int* nseeds_dev, int b
     hipLaunchKernelGGL(k_mark_dirty, dim3(blocks_for(bound, 256)), dim3(256), 0, s, pool, seeds, nseeds_dev, bound,
                        stop_at_tdel, dirty, pend, hdr);
 }
-void launch_find_top(Pool pool, const int* viol, int bound, DevHdr* hdr, int* top, hipStream_t s) {
+void launch_find_top(Pool pool, const int* viol, int bound, DevHdr* hdr, int* top, int* pend, hipStream_t s) {
     if (bound <= 0) return;
-    hipLaunchKernelGGL(k_find_top, dim3(blocks_for(bound, 256)), dim3(256), 0, s, pool, viol, hdr, top);
+    hipLaunchKernelGGL(k_find_top, dim3(blocks_for(bound, 256)), dim3(256), 0, s, pool, viol, hdr, top, pend);
 }
 void launch_clear_viol(Pool pool, const int* viol, int bound, DevHdr* hdr, hipStream_t s) {
     if (bound <= 0) return;
