@@ -21,6 +21,7 @@
 // Cold arrays: id[n] (payload id), par[n] (parent), cnt[n] = {TreeSize,
 // invalid_point_num, down_del_num, depth}, meta[n] (axis + lazy labels).
 #pragma once
+#include <math.h>
 #include <stdint.h>
 
 #ifdef __HIPCC__
@@ -102,16 +103,20 @@ IKD_HD float calc_dist(float ax, float ay, float az, float bx, float by, float b
     return d;
 }
 
-// calc_box_dist, ikd_Tree.cpp:1380-1391: b = {lo x,y,z, hi x,y,z}; the six
-// terms are added in x-lo, x-hi, y-lo, y-hi, z-lo, z-hi order.
+// calc_box_dist, ikd_Tree.cpp:1380-1391: b = {lo x,y,z, hi x,y,z}; the
+// reference adds the square of p - lo (p < lo) and of p - hi (p > hi) per axis
+// in x, y, z order.  At most one of the two is positive as lo - p and p - hi,
+// the square of a difference does not depend on its sign, and adding +0
+// changes nothing, so one square of max(lo - p, p - hi, 0) per axis gives the
+// same bits (a NaN on either side drops out of fmaxf as it fails the
+// reference's comparisons): 14 vector instructions instead of about 40.
 IKD_HD float calc_box_dist(const float* b, float px, float py, float pz) {
-    float s = 0.0f;
-    if (px < b[0]) { float t = px - b[0]; s = s + t * t; }
-    if (px > b[3]) { float t = px - b[3]; s = s + t * t; }
-    if (py < b[1]) { float t = py - b[1]; s = s + t * t; }
-    if (py > b[4]) { float t = py - b[4]; s = s + t * t; }
-    if (pz < b[2]) { float t = pz - b[2]; s = s + t * t; }
-    if (pz > b[5]) { float t = pz - b[5]; s = s + t * t; }
+    const float tx = fmaxf(fmaxf(b[0] - px, px - b[3]), 0.0f);
+    const float ty = fmaxf(fmaxf(b[1] - py, py - b[4]), 0.0f);
+    const float tz = fmaxf(fmaxf(b[2] - pz, pz - b[5]), 0.0f);
+    float s = tx * tx;
+    s = s + ty * ty;
+    s = s + tz * tz;
     return s;
 }
 

@@ -49,6 +49,17 @@ __device__ __forceinline__ bool after(const NodeHot* hot, const uint32_t* ids, f
     return tie_less(hot, ids, n, en);
 }
 
+// The median and the smaller of values that are not NaN (a squared distance, a
+// list slot), each one instruction.
+__device__ __forceinline__ float med3(float a, float b, float c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_fmed3f(a, b, c);
+#else
+    return fmaxf(fminf(a, b), fminf(fmaxf(a, b), c));
+#endif
+}
+__device__ __forceinline__ float fminf_raw(float a, float b) { return b < a ? b : a; }
+
 // Sorted best-k list of one lane: bd_[0] is the current k-th candidate,
 // slots past k hold (-inf, -2) padding.
 template <int KM>
@@ -62,33 +73,38 @@ struct BestList {
             n[i] = i < k ? -1 : -2;
         }
     }
-    // offer (dist, node); keeps the k smallest in (d2, x, y, z, id) order.
-    // Without an exact distance tie in the list the ranks are plain float
-    // comparisons (branch-free selects); a tie takes the full comparator.
+    // offer (dist, node) with dist <= d[0]; keeps the k smallest in (d2, x, y,
+    // z, id) order.  Slots farther than the candidate move up by one and the
+    // candidate takes the slot they leave: for the distances that is the median
+    // of a slot, the next one and dist, whatever the ties.  On an exact tie the
+    // candidate now stands above the run of its equals (or outside the list,
+    // when the run starts it) and passes those that rank after it.
     __device__ __forceinline__ void offer(const NodeHot* hot, const uint32_t* ids, float dist, int node) {
-        if (dist > d[0]) return;  // strictly worse than the k-th: the common case
-        bool tie = false;
-#pragma unroll
-        for (int i = 0; i < KM; ++i) tie = tie || d[i] == dist;
-        bool gnext[KM];
-        if (!tie) {
-#pragma unroll
-            for (int i = 0; i < KM; ++i) gnext[i] = (i + 1 < KM) ? d[i + 1] > dist : false;
-        } else {
-            if (!after(hot, ids, d[0], n[0], dist, node)) return;
-#pragma unroll
-            for (int i = 0; i < KM; ++i)
-                gnext[i] = (i + 1 < KM) ? after(hot, ids, d[i + 1], n[i + 1], dist, node) : false;
-        }
+        bool tie = d[0] == dist;
+        const bool first = tie;
+        int below = d[0] > dist ? node : n[0];  // what slot i takes if slot i + 1 stays
 #pragma unroll
         for (int i = 0; i < KM; ++i) {
-            bool gcur = (i == 0) ? true : gnext[i - 1];
-            if (gnext[i]) {
-                d[i] = d[i + 1 < KM ? i + 1 : i];
-                n[i] = n[i + 1 < KM ? i + 1 : i];
-            } else if (gcur) {
-                d[i] = dist;
-                n[i] = node;
+            if (i + 1 < KM) {
+                const bool far1 = d[i + 1] > dist;
+                tie = tie | (d[i + 1] == dist);
+                const int n1 = n[i + 1];
+                n[i] = far1 ? n1 : below;
+                below = far1 ? node : n1;
+                d[i] = med3(d[i], d[i + 1], dist);
+            } else {
+                n[i] = below;
+                d[i] = fminf_raw(d[i], dist);
+            }
+        }
+        if (tie) {
+            if (first && after(hot, ids, d[0], n[0], dist, node)) n[0] = node;
+#pragma unroll
+            for (int i = 0; i + 1 < KM; ++i) {
+                if (n[i] == node && d[i + 1] == dist && after(hot, ids, d[i + 1], n[i + 1], dist, node)) {
+                    n[i] = n[i + 1];
+                    n[i + 1] = node;
+                }
             }
         }
     }
@@ -162,37 +178,42 @@ __device__ __forceinline__ void finish_query(const KnnArgs& a, const QueryCtx& c
     if (a.boxes) a.boxes[c.qo] = boxes;
 }
 
-// One visit of node n: offer its point, then compute both children's box
-// distances.  Returns the near child (or -1) and, through far/df, the far one.
-template <int KM>
-__device__ __forceinline__ void visit_node(const QueryCtx& c, BestList<KM>& best, int n, int& near_n, float& dn,
-                                           int& far_n, float& df, unsigned int& boxes) {
+// One visit of node n: offers its point, then computes both children's box
+// distances.  lim is the walk's bound, min(cap, k-th distance) with cap = min(
+// max_dist's threshold, a team's bound): nothing above it is offered or
+// descended into, and an offer tightens it.  near_n / far_n: the children
+// within the bound (near first, left on ties), or -1.  COUNT: also counts the
+// child boxes (instrumentation).
+//
+// A visit is one 64-byte gather per lane and its arithmetic.  The distances of
+// absent children are computed like the others and masked instead of branched
+// around, and an offer is medians and selects: about 85 vector instructions a
+// visit where it was 154, with the vector units 86 % busy (2M points, 1.18M
+// queries, k = 5: one launch alone 492 -> 447 us; what is left is the latency
+// of gathers that miss L1 (18 %) and L2 (19 %)).
+template <int KM, bool COUNT>
+__device__ __forceinline__ void visit_node(const QueryCtx& c, BestList<KM>& best, int n, float cap, float& lim,
+                                           int& near_n, float& dn, int& far_n, float& df, unsigned int& boxes) {
     const gv4* rec = reinterpret_cast<const gv4*>(c.hot[n].f);
     const gv4 r0 = gload4(rec), r1 = gload4(rec + 1), r2 = gload4(rec + 2), r3 = gload4(rec + 3);
     const uint32_t lk = fbits(r0.w);
-    if (!(lk & LK_PDEL)) {
-        float d = calc_dist(c.qx, c.qy, c.qz, r0.x, r0.y, r0.z);
-        if (d <= c.thr) best.offer(c.hot, c.ids, d, n);
+    const float d = calc_dist(c.qx, c.qy, c.qz, r0.x, r0.y, r0.z);
+    if (!(lk & LK_PDEL) && d <= lim) {
+        best.offer(c.hot, c.ids, d, n);
+        lim = fminf_raw(cap, best.d[0]);
     }
-    const int pair = (int)lk_pair(lk);
-    const bool hl = (lk & LK_HASL) != 0, hr = (lk & LK_HASR) != 0;
-    boxes += (hl ? 1u : 0u) + (hr ? 1u : 0u);
-    const bool el = hl && !(lk & LK_TDL), er = hr && !(lk & LK_TDR);
-    float bl[6] = {r1.x, r1.y, r1.z, r1.w, r2.x, r2.y};
-    float br[6] = {r2.z, r2.w, r3.x, r3.y, r3.z, r3.w};
-    const float dl = el ? calc_box_dist(bl, c.qx, c.qy, c.qz) : INFINITY;
-    const float dr = er ? calc_box_dist(br, c.qx, c.qy, c.qz) : INFINITY;
-    near_n = -1;
-    far_n = -1;
-    if (el || er) {
-        const bool near_left = el && (!er || dl <= dr);
-        near_n = near_left ? 2 * pair : 2 * pair + 1;
-        dn = near_left ? dl : dr;
-        if (near_left ? er : el) {
-            far_n = near_left ? 2 * pair + 1 : 2 * pair;
-            df = near_left ? dr : dl;
-        }
-    }
+    if (COUNT) boxes += ((lk & LK_HASL) ? 1u : 0u) + ((lk & LK_HASR) ? 1u : 0u);
+    const bool el = (lk & (LK_HASL | LK_TDL)) == LK_HASL, er = (lk & (LK_HASR | LK_TDR)) == LK_HASR;
+    const float bl[6] = {r1.x, r1.y, r1.z, r1.w, r2.x, r2.y};
+    const float br[6] = {r2.z, r2.w, r3.x, r3.y, r3.z, r3.w};
+    const float dl = calc_box_dist(bl, c.qx, c.qy, c.qz);
+    const float dr = calc_box_dist(br, c.qx, c.qy, c.qz);
+    const bool nl = el & (!er | (dl <= dr));
+    dn = nl ? dl : dr;
+    df = nl ? dr : dl;
+    const int near_c = (int)((lk >> (LK_PAIR_SHIFT - 1)) & ~1u) | (nl ? 0 : 1);
+    near_n = ((el | er) & (dn <= lim)) ? near_c : -1;
+    far_n = ((el & er) & (df <= lim)) ? (near_c ^ 1) : -1;
 }
 
 // ---- LDS traversal stacks --------------------------------------------------
@@ -244,7 +265,31 @@ __device__ __forceinline__ uint32_t compact_entry(int n, float d) {
 __device__ __forceinline__ float compact_dist(uint32_t e) { return bitsf((e & 0xffu) << 23); }
 static inline size_t lds_compact_bytes(int stack) { return (size_t)stack * 64 * sizeof(uint32_t); }
 
-template <int KM, bool COMPACT>
+// The node a lane starts at: the root, if it is live and within the bound.
+__device__ __forceinline__ int knn_root(const QueryCtx& c) {
+    const uint32_t lk0 = fbits(c.hot[SENTINEL].f[3]);
+    if (!(lk0 & LK_HASL) || (lk0 & LK_TDL)) return -1;
+    return calc_box_dist(c.hot[SENTINEL].f + 4, c.qx, c.qy, c.qz) <= c.thr ? ROOT : -1;
+}
+
+// The lane's next deferred child that can still improve (-1: none left).
+// Entries were within max_dist's threshold when they were pushed, and a stored
+// distance never exceeds the exact one.
+template <bool COMPACT>
+__device__ __forceinline__ int knn_pop(const LdsStack& st, const uint32_t* cst, int lane, int& sp, float kth) {
+    while (sp > 0) {
+        --sp;
+        if (COMPACT) {
+            const uint32_t e = cst[sp * 64 + lane];
+            if (compact_dist(e) <= kth) return (int)(e >> 8);
+        } else {
+            if (dist_val(st.d[sp * 64 + lane]) <= kth) return st.n[sp * 64 + lane];
+        }
+    }
+    return -1;
+}
+
+template <int KM, bool COMPACT, bool COUNT>
 __global__ __launch_bounds__(64) void k_knn(KnnArgs a) {
     const LdsStack st = lds_stack(a.stack);
     extern __shared__ int lds_dyn[];
@@ -257,67 +302,35 @@ __global__ __launch_bounds__(64) void k_knn(KnnArgs a) {
     BestList<KM> best;
     best.init(c.k);
     unsigned int visits = 0, boxes = 0;
-
-    const uint32_t lk0 = fbits(c.hot[SENTINEL].f[3]);
+    float lim = fminf_raw(c.thr, best.d[0]);
     int sp = 0;
-    int n = -1;
-    float bd = 0.0f;
-    if ((lk0 & LK_HASL) && !(lk0 & LK_TDL)) {
-        n = ROOT;
-        bd = calc_box_dist(c.hot[SENTINEL].f + 4, c.qx, c.qy, c.qz);
-    }
-    while (true) {
-        if ((int)visits > a.max_steps) {
-            atomicOr(a.overflow, 2);
-            break;
-        }
-        if (n >= 0 && bd <= c.thr) {
-            ++visits;
-            int nn, fn;
-            float dn = 0.0f, df = 0.0f;
-            visit_node<KM>(c, best, n, nn, dn, fn, df, boxes);
-            const float top = best.d[0];
-            if (fn >= 0 && df <= top && df <= c.thr) {
-                if (sp < a.stack) {
-                    if (COMPACT) {
-                        cst[sp * 64 + lane] = compact_entry(fn, df);
-                    } else {
-                        st.n[sp * 64 + lane] = fn;
-                        st.d[sp * 64 + lane] = dist_key(df);
-                    }
-                    ++sp;
+    int n = knn_root(c);
+    int round = 0;
+    while (n >= 0) {  // every lane still here visits one node per round
+        if (COUNT) ++visits;
+        int nn, fn;
+        float dn, df;
+        visit_node<KM, COUNT>(c, best, n, c.thr, lim, nn, dn, fn, df, boxes);
+        if (fn >= 0) {
+            if (sp < a.stack) {
+                if (COMPACT) {
+                    cst[sp * 64 + lane] = compact_entry(fn, df);
                 } else {
-                    atomicOr(a.overflow, 1);
+                    st.n[sp * 64 + lane] = fn;
+                    st.d[sp * 64 + lane] = dist_key(df);
                 }
-            }
-            if (nn >= 0 && dn <= top && dn <= c.thr) {
-                n = nn;
-                bd = dn;
-                continue;
-            }
-        }
-        // backtrack to the deepest deferred child that can still improve
-        n = -1;
-        while (sp > 0) {
-            --sp;
-            if (COMPACT) {
-                const uint32_t e = cst[sp * 64 + lane];
-                const float d = compact_dist(e);
-                if (d <= best.d[0]) {
-                    n = (int)(e >> 8);
-                    bd = d;
-                    break;
-                }
+                ++sp;
             } else {
-                const float d = dist_val(st.d[sp * 64 + lane]);
-                if (d <= best.d[0]) {
-                    n = st.n[sp * 64 + lane];
-                    bd = d;
-                    break;
-                }
+                atomicOr(a.overflow, 1);
             }
         }
-        if (n < 0) break;
+        n = nn;
+        if (++round > a.max_steps) {
+            atomicOr(a.overflow, 2);
+            sp = 0;
+            n = -1;
+        }
+        if (n < 0) n = knn_pop<COMPACT>(st, cst, lane, sp, best.d[0]);
     }
 
     finish_query<KM>(a, c, best, visits, boxes);
@@ -606,16 +619,16 @@ __global__ __launch_bounds__(64) void k_knn_team(KnnArgs a) {
         }
 
         if (n >= 0) {
-            float bound = fminf(B, best.d[0]);
-            if (bd > c.thr || bd > bound) {
+            const float cap = fminf(B, c.thr);
+            float bound = fminf(cap, best.d[0]);
+            if (bd > bound) {
                 n = -1;
             } else {
                 ++visits;
                 int nn, fn;
-                float dn = 0.0f, df = 0.0f;
-                visit_node<KM>(c, best, n, nn, dn, fn, df, boxes);
-                bound = fminf(B, best.d[0]);
-                if (fn >= 0 && df <= bound && df <= c.thr) {
+                float dn, df;
+                visit_node<KM, true>(c, best, n, cap, bound, nn, dn, fn, df, boxes);
+                if (fn >= 0) {
                     if (tail - head < a.stack) {
                         const int s = tail & smask;
                         slot_put<COMPACT>(st, cst, s * 64 + lane, fn, df);
@@ -624,12 +637,8 @@ __global__ __launch_bounds__(64) void k_knn_team(KnnArgs a) {
                         atomicOr(a.overflow, 1);
                     }
                 }
-                if (nn >= 0 && dn <= bound && dn <= c.thr) {
-                    n = nn;
-                    bd = dn;
-                } else {
-                    n = -1;
-                }
+                n = nn;
+                bd = dn;
             }
         }
         float v = best.d[0];
@@ -700,7 +709,6 @@ __global__ __launch_bounds__(64) void k_knn_persist(KnnArgs a, int* __restrict__
     BestList<KM> best;
     bool has = false;
     int n = -1, sp = 0;
-    float bd = 0.0f;
     unsigned int visits = 0, boxes = 0;
     bool drained = false;
     while (true) {
@@ -722,12 +730,7 @@ __global__ __launch_bounds__(64) void k_knn_persist(KnnArgs a, int* __restrict__
                     best.init(c.k);
                     visits = boxes = 0;
                     sp = 0;
-                    n = -1;
-                    const uint32_t lk0 = fbits(c.hot[SENTINEL].f[3]);
-                    if ((lk0 & LK_HASL) && !(lk0 & LK_TDL)) {
-                        n = ROOT;
-                        bd = calc_box_dist(c.hot[SENTINEL].f + 4, c.qx, c.qy, c.qz);
-                    }
+                    n = knn_root(c);
                     has = true;
                 }
             }
@@ -738,13 +741,13 @@ __global__ __launch_bounds__(64) void k_knn_persist(KnnArgs a, int* __restrict__
             n = -1;
             sp = 0;
         }
-        if (n >= 0 && bd <= c.thr) {
+        if (n >= 0) {
             ++visits;
             int nn, fn;
-            float dn = 0.0f, df = 0.0f;
-            visit_node<KM>(c, best, n, nn, dn, fn, df, boxes);
-            const float top = best.d[0];
-            if (fn >= 0 && df <= top && df <= c.thr) {
+            float dn, df;
+            float lim = fminf_raw(c.thr, best.d[0]);
+            visit_node<KM, true>(c, best, n, c.thr, lim, nn, dn, fn, df, boxes);
+            if (fn >= 0) {
                 if (sp < a.stack) {
                     if (COMPACT) {
                         cst[sp * 64 + lane] = compact_entry(fn, df);
@@ -757,32 +760,10 @@ __global__ __launch_bounds__(64) void k_knn_persist(KnnArgs a, int* __restrict__
                     atomicOr(a.overflow, 1);
                 }
             }
-            if (nn >= 0 && dn <= top && dn <= c.thr) {
-                n = nn;
-                bd = dn;
-                continue;
-            }
+            n = nn;
+            if (n >= 0) continue;
         }
-        n = -1;
-        while (sp > 0) {
-            --sp;
-            if (COMPACT) {
-                const uint32_t e = cst[sp * 64 + lane];
-                const float d = compact_dist(e);
-                if (d <= best.d[0]) {
-                    n = (int)(e >> 8);
-                    bd = d;
-                    break;
-                }
-            } else {
-                const float d = dist_val(st.d[sp * 64 + lane]);
-                if (d <= best.d[0]) {
-                    n = st.n[sp * 64 + lane];
-                    bd = d;
-                    break;
-                }
-            }
-        }
+        n = knn_pop<COMPACT>(st, cst, lane, sp, best.d[0]);
         if (n >= 0) continue;
         finish_query<KM>(a, c, best, visits, boxes);
         has = false;
@@ -801,6 +782,8 @@ static int device_cus() {
     }
     return v;
 }
+
+constexpr int KNN_STACK_FLOOR = 26;
 
 template <int KM>
 static int launch_knn_km(const KnnArgs& a0, int lanes, int stack, hipStream_t s, int* persist_next,
@@ -821,12 +804,21 @@ static int launch_knn_km(const KnnArgs& a0, int lanes, int stack, hipStream_t s,
                 hipLaunchKernelGGL((k_knn_staged<KM>), dim3(xcd_grid(blocks_for(a.nq, 64))), block, lds_t, s, a);
                 return 0;
             }
-            if (a.compact_stack) {
-                hipLaunchKernelGGL((k_knn<KM, true>), dim3(xcd_grid(blocks_for(a.nq, 64))), block,
-                                   lds_compact_bytes(stack), s, a);
+            if (a.visits) {
+                hipLaunchKernelGGL((k_knn<KM, false, true>), dim3(xcd_grid(blocks_for(a.nq, 64))), block, lds, s, a);
                 return 0;
             }
-            hipLaunchKernelGGL((k_knn<KM, false>), dim3(xcd_grid(blocks_for(a.nq, 64))), block, lds, s, a);
+            if (a.compact_stack) {
+                // At least KNN_STACK_FLOOR entries of LDS, so that a CU holds at most 24
+                // wavefronts: with 28 the walks of three 2M-point maps in turn (1.18M
+                // queries each, k = 5) evict each other's nodes from L2, 446 us a launch
+                // against 433; one map alone takes 447 against 452.
+                const size_t lb = lds_compact_bytes(std::max(stack, KNN_STACK_FLOOR));
+                hipLaunchKernelGGL((k_knn<KM, true, false>), dim3(xcd_grid(blocks_for(a.nq, 64))), block,
+                                   lb, s, a);
+                return 0;
+            }
+            hipLaunchKernelGGL((k_knn<KM, false, false>), dim3(xcd_grid(blocks_for(a.nq, 64))), block, lds, s, a);
             return 0;
         case 0: {  // persistent lanes; the 8 per-XCD query counters were zeroed by the caller
             // as many single-wavefront workgroups as the LDS stacks let each CU hold
