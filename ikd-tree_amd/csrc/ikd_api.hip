@@ -283,7 +283,7 @@ enum Buf {
     B_PFLAG, B_PSCAN, B_ISEG, B_ISEGD, B_IO0, B_IO1, B_IO2, B_IO3, B_IO4, B_VSTART, B_DELBOX, B_DELFL, B_INSPT,
     B_INSFL, B_CBOX, B_CPTS, B_MISC, B_MORTK, B_MORTV, B_MORTK2, B_MORTV2, B_CNT64, B_OFF64, B_ADDX, B_ADDI, B_PNEXT, B_SPAIRS, B_SPSCAN,
     B_DEFER, B_DINFO, B_DBEFORE, B_DKEEP, B_PTS3, B_PEND, B_START, B_INV0, B_LASTP, B_PSEED, B_DBELOW, B_MAXDEL,
-    B_SLISTS, B_ENUMROOT, B_ENUMGRP, B_TOPT, B_TOPI, B_TCNT64, B_TOFF64, B_RTASKS, B_ICNT64, B_EMPTYL, B_COUNT
+    B_SLISTS, B_ENUMROOT, B_ENUMGRP, B_TOPT, B_TOPI, B_TCNT64, B_TOFF64, B_RTASKS, B_ICNT64, B_EMPTYL, B_RAW, B_COUNT
 };
 static_assert(B_COUNT <= 96, "scratch table");
 
@@ -797,9 +797,12 @@ constexpr long long ENUM_BLOCK_MAX = 1024;
 // larger one walks one level per launch over the whole grid instead).
 constexpr long long ENUM_GROUP_NODES = 2048;
 constexpr long long ENUM_GROUP_ROOT_MAX = 16384;
-// Range search: subtrees a query covers whole with at most this many nodes are
-// written by one lane each after the walks (the walks stop there).
-constexpr int RANGE_TASK_NODES = 256;
+// Range search: subtrees of at most this many nodes are counted and written by
+// one lane each after the walks (the walks stop there).
+constexpr int RANGE_TASK_NODES = 32;
+// Items the first walk of a range search keeps for all queries together (16 MB):
+// 200 boxes keep up to 20k each, half a million balls 7.
+constexpr int RANGE_RAW_ITEMS = 1 << 22;
 
 // Room for `extra` more records beyond the current count (fresh in h_hdr):
 // the record survives the growth, unlike scratch.
@@ -1537,13 +1540,13 @@ int knn_dev(ikd_tree_t t, const float* d_q, int nq, int k, double max_dist, floa
 // output position; *total and *ntask come back to the host (two waits: the
 // item count sizes the lists, the total sizes the output).  slots: scratch
 // slots for the per-query item counts and offsets, the items, the item
-// counts and the item offsets.
+// counts and offsets, and the items the first walk keeps.
 hipError_t owner_wait(ikd_tree_t t) { return wait_stream(t); }
 template <class Owner>
 hipError_t owner_wait(Owner* b) { return hipStreamSynchronize(b->st); }
 
 template <class Owner>
-int range_plan(Owner* t, RangeArgs& a, int nq, long long* d_offsets, const int (&slots)[5], long long pool_bound,
+int range_plan(Owner* t, RangeArgs& a, int nq, long long* d_offsets, const int (&slots)[6], long long pool_bound,
                long long* total, long long* ntask_out) {
     hipStream_t st = t->st;
     long long *tcnt, *toff, *icnt, *ioff;
@@ -1553,6 +1556,8 @@ int range_plan(Owner* t, RangeArgs& a, int nq, long long* d_offsets, const int (
     launch_fill_i32(reinterpret_cast<int*>(tcnt + nq), 0, 2, st);  // the scan's trailing zero
     a.task_nodes = RANGE_TASK_NODES;
     a.tcounts = tcnt;
+    a.raw_cap = (int)std::max<long long>(1, std::min<long long>(pool_bound, RANGE_RAW_ITEMS / nq));
+    CHK(ensure(t, slots[5], (long long)nq * a.raw_cap, &a.raw));
     launch_range_top(a, 0, st);
     CHK(exscan_i64(t, tcnt, toff, nq + 1));
     long long ntask = 0;
@@ -1596,7 +1601,7 @@ int range_dev(ikd_tree_t t, int mode, const float* d_boxes, const float* d_cente
     a.overflow = &t->d_hdr->overflow;
     a.stack = std::min(t->max_depth + 2, MAX_DEPTH);
     long long total = 0, ntask = 0;
-    static const int slots[5] = {B_TCNT64, B_TOFF64, B_RTASKS, B_CNT64, B_ICNT64};
+    static const int slots[6] = {B_TCNT64, B_TOFF64, B_RTASKS, B_CNT64, B_ICNT64, B_RAW};
     CHK(range_plan(t, a, nq, off, slots, std::max<long long>(t->pool_used, 1), &total, &ntask));
     HIPCHK(hipMemcpyAsync(h_offsets, off, (nq + 1) * sizeof(long long), hipMemcpyDeviceToHost, st));
     CHK(sync_hdr(t));
@@ -2320,7 +2325,7 @@ const char* ikd_last_error(ikd_tree_t t) {
 
 // ------------------------------------------------------------ multi-tree batches
 enum BatchBuf { BB_TMP = 0, BB_TREES, BB_THR, BB_NEXT, BB_FLAG, BB_CNT, BB_POOLS, BB_TCNT, BB_TOFF, BB_TASKS,
-                BB_ICNT, BB_COUNT };
+                BB_ICNT, BB_RAW, BB_COUNT };
 static_assert(BB_COUNT <= 16, "batch scratch table");
 
 // ------------------------------------- allocation-free multi-tree kNN scratch
@@ -2834,7 +2839,7 @@ int ikd_batch_radius_search_device(ikd_batch_t b, const ikd_tree_t* trees, int n
     a.max_steps = steps;
     a.stack = std::min(depth + 2, MAX_DEPTH);
     long long total = 0, ntask = 0;
-    static const int slots[5] = {BB_TCNT, BB_TOFF, BB_TASKS, BB_CNT, BB_ICNT};
+    static const int slots[6] = {BB_TCNT, BB_TOFF, BB_TASKS, BB_CNT, BB_ICNT, BB_RAW};
     CHK(range_plan(b, a, (int)nq, reinterpret_cast<long long*>(d_out_offsets), slots, std::max<long long>(steps, 1),
                    &total, &ntask));
     *out_total = total;

@@ -246,7 +246,7 @@ struct RangeArgs {
     uint32_t* out_ids;
     int* overflow;
     long long max_steps;
-    int stack;            // LDS stack entries per lane (>= tree depth + 2)
+    int stack;            // item walks: LDS stack entries per lane (>= tree depth + 2)
     const Pool* pools;    // multi-tree launch: pool table with qtree[q] per query (else null)
     const int* qtree;
     int ntrees;           // a query naming no valid tree finds nothing
@@ -256,11 +256,13 @@ struct RangeArgs {
     // node, query, kind) and written from item_offsets[i]
     int task_nodes;
     long long* tcounts;
+    int* raw;             // the first raw_cap items of each query, as stack entries
+    int raw_cap;
     const long long* toffsets;
     int4* tasks;
     const long long* item_offsets;
 };
-// list 0: tcounts[q] = items of query q; list 1: the items at toffsets[q]
+// list 0: tcounts[q] = items of query q, the first of them kept in raw; list 1: the items at toffsets[q]
 void launch_range_top(const RangeArgs& a, int list, hipStream_t s);
 // counts[i] = points of item i
 void launch_range_item_count(const RangeArgs& a, long long ntask, long long* counts, hipStream_t s);

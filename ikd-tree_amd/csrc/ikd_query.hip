@@ -972,25 +972,28 @@ __device__ __forceinline__ int classify(const RangeArgs& a, int qi, const float*
     return 2;
 }
 
-// Range search in items.  A walk per query (one lane each, depth-first
-// stack in LDS as [stack][64] entries) goes down only through subtrees of
-// more than task_nodes nodes; everything at or below that size, and the own
-// point of every node it walks, becomes an item of the query's list, in
-// pre-order:
+// Range search in items.  One wavefront walks each query; the walk goes down
+// only through subtrees of more than task_nodes nodes, and everything at or
+// below that size, and the own point of every node it walks, becomes an item
+// of the query's list, in pre-order:
 //   RANGE_OWN   the node's own point (the walk checked the predicate),
 //   RANGE_COVER a subtree the query covers whole,
 //   RANGE_PART  a subtree the query cuts.
-// The count walk (k_range_top, list 0) counts each query's items, the list
-// walk (list 1) writes them; one lane per item then counts its points
-// (k_range_item_count: 1, the subtree's live count, or a walk of the cut
-// subtree with covered parts counted from their stored counts), a scan over
-// the items gives every item its output offset and every query its first,
-// and one lane per item writes its points (k_range_item_fill) in pre-order.
-// The output is the pre-order sequence of one walk per query.
+// The first walk (k_range_top, list 0) counts each query's items and keeps the
+// first raw_cap of them; a scan gives every query its place in the item list,
+// and list 1 copies the kept items there (a query with more walks again).  One
+// lane per item then counts its points (k_range_item_count: 1, the subtree's
+// live count, or a walk of the cut subtree with covered parts counted from
+// their stored counts), a scan over the items gives every item its output
+// offset and every query its first, and one lane per item writes its points
+// (k_range_item_fill) in pre-order.  The output is the pre-order sequence of
+// one walk per query.
 //
 // Stack entries: node index (< 2^28) with bit 31 = covered whole, bit 30 =
-// an item left for its pop (so items keep pre-order), bit 29 = the item is
-// a cut subtree.
+// an item (so items keep pre-order), bit 29 = the item is a cut subtree; an
+// item with bit 31 is the node's own point.  Whether a node is small enough to
+// be an item is read with its record, when its entry is taken, so a round waits
+// for one gather and not for the record and then the children's sizes.
 constexpr int RANGE_WHOLE = (int)0x80000000;
 constexpr int RANGE_TASK = 0x40000000;
 constexpr int RANGE_CUT = 0x20000000;
@@ -1006,6 +1009,11 @@ __device__ __forceinline__ Pool range_pool(const RangeArgs& a, int qi, bool* ok)
         return a.pool;
     }
     return a.pools[ti];
+}
+
+__device__ __forceinline__ void range_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 struct RangeQuery {
@@ -1027,76 +1035,146 @@ __device__ __forceinline__ bool range_takes(const RangeArgs& a, int qi, const Ra
     return calc_dist(f[0], f[1], f[2], q.qx, q.qy, q.qz) <= q.r2;
 }
 
-__global__ __launch_bounds__(64) void k_range_top(RangeArgs a, int list) {
+// One wavefront per query.  The pending sequence, in pre-order, is a stack in
+// LDS with its first entry on top.  A round takes up to 64 entries off the
+// top, one a lane: an item stays itself, a node of at most task_nodes nodes
+// becomes one, a larger one becomes its own point (if taken), its left and its
+// right child.  What now leads the sequence up to the first node still to be
+// walked is final and is written; the rest goes back in order, found by prefix
+// counts over ballots.
+//
+// A walk is a chain of dependent gathers: with one lane a query, 200 boxes over
+// 1M points kept 200 lanes of the whole device busy for 705 us a walk; a
+// wavefront takes its frontier 64 nodes at a time (about 120 us).
+//
+// The stack never overflows: a round of b entries adds at most 2 b, b is cut to
+// half the room above a reserve of RANGE_RESERVE entries, and below that the
+// walk is plain depth-first (b = 1), which adds at most one entry per level
+// of the tree (at most MAX_DEPTH) before it is back where it was.
+constexpr int RANGE_RESERVE = MAX_DEPTH + 4;
+constexpr int RANGE_FEW_QUERIES = 2048;
+
+__device__ __forceinline__ int lanes_below(unsigned long long m, int lane) {
+    return __popcll(m & ((1ull << lane) - 1ull));
+}
+__device__ __forceinline__ int4 range_item_of(int e, int qi) {
+    return make_int4(e & RANGE_NODE, qi, (e & RANGE_WHOLE) ? RANGE_OWN : ((e & RANGE_CUT) ? RANGE_PART : RANGE_COVER),
+                     0);
+}
+
+__global__ __launch_bounds__(64) void k_range_top(RangeArgs a, int list, int qbase) {
     extern __shared__ int lds_dyn[];
     int* stk = lds_dyn;
     const int lane = threadIdx.x;
-    const int qi = blockIdx.x * 64 + lane;
-    if (qi >= a.nq) return;
+    const int qi = qbase + (int)blockIdx.x;
     bool ok;
     const Pool P = range_pool(a, qi, &ok);
     if (!ok) {
-        if (!list) a.tcounts[qi] = 0;
+        if (!list && lane == 0) a.tcounts[qi] = 0;
         return;
+    }
+    // where this walk writes its items, and how many it may
+    int* const raw = a.raw + (size_t)qi * a.raw_cap;
+    int4* dst = nullptr;
+    long long cap = a.raw_cap;
+    if (list) {
+        dst = a.tasks + a.toffsets[qi];
+        cap = a.toffsets[qi + 1] - a.toffsets[qi];
+        if (cap <= a.raw_cap) {
+            for (int i = lane; i < (int)cap; i += 64) dst[i] = range_item_of(raw[i], qi);
+            return;
+        }
     }
     const NodeHot* __restrict__ hot = P.hot;
     const int G = a.task_nodes;
     const RangeQuery q = range_query(a, qi);
     long long items = 0;
-    long long tpos = list ? a.toffsets[qi] : 0;
-    const long long tlim = list ? a.toffsets[qi + 1] : 0;
-    auto item = [&](int u, int kind) {
-        if (!list) {
-            ++items;
-        } else if (tpos < tlim) {
-            a.tasks[tpos++] = make_int4(u, qi, kind, 0);
-        } else {
-            atomicOr(a.overflow, 8);
-        }
-    };
-    // an entry for child c of class cls (1 covered, 2 cut)
-    auto entry = [&](int c, int cls) -> int {
-        if (P.cnt[c].x <= G) return c | RANGE_TASK | (cls == 2 ? RANGE_CUT : 0);
-        return c | (cls == 1 ? RANGE_WHOLE : 0);
-    };
+    int sp = 0;
     const uint32_t lk0 = fbits(hot[SENTINEL].f[3]);
     if ((lk0 & LK_HASL) && !(lk0 & LK_TDL)) {
-        int sp = 0;
         const int c0 = classify(a, qi, hot[SENTINEL].f + 4, q.qx, q.qy, q.qz, q.r);
         if (c0 != 0) {
-            stk[lane] = entry(ROOT, c0);
+            if (lane == 0) stk[0] = ROOT | (c0 == 1 ? RANGE_WHOLE : 0);
             sp = 1;
         }
-        long long steps = 0;
-        while (sp > 0) {
-            if (++steps > a.max_steps) {
-                atomicOr(a.overflow, 8);
-                break;
-            }
-            const int e = stk[--sp * 64 + lane];
-            const int u = e & RANGE_NODE;
+    }
+    range_lds_fence();
+    long long rounds = 0;
+    while (sp > 0) {
+        if (++rounds > 4 * a.max_steps) {
+            if (lane == 0) atomicOr(a.overflow, 8);
+            break;
+        }
+        const int b = min(min(sp, 64), max(1, (a.stack - RANGE_RESERVE - sp) >> 1));
+        // this lane's part of the sequence: m entries, the first r of them items
+        int e0 = 0, e1 = 0, e2 = 0, m = 0, r = 0;
+        if (lane < b) {
+            const int e = stk[sp - 1 - lane];
             if (e & RANGE_TASK) {
-                item(u, (e & RANGE_CUT) ? RANGE_PART : RANGE_COVER);
-                continue;
-            }
-            const bool whole = (e & RANGE_WHOLE) != 0;
-            float f[16];
-            load_record(hot[u].f, f);
-            const uint32_t lk = fbits(f[3]);
-            if (!(lk & LK_PDEL) && (whole || range_takes(a, qi, q, f))) item(u, RANGE_OWN);
-            const int pair = (int)lk_pair(lk);
+                e0 = e;
+                m = r = 1;
+            } else {
+                const int u = e & RANGE_NODE;
+                const bool whole = (e & RANGE_WHOLE) != 0;
+                float f[16];
+                load_record(hot[u].f, f);
+                if (P.cnt[u].x <= G) {
+                    e0 = u | RANGE_TASK | (whole ? 0 : RANGE_CUT);
+                    m = r = 1;
+                } else {
+                    const uint32_t lk = fbits(f[3]);
+                    const int pair = (int)lk_pair(lk);
+                    int c[2] = {0, 0};
 #pragma unroll
-            for (int s = 1; s >= 0; --s) {
-                if (!(lk & lk_has(s)) || (lk & lk_td(s))) continue;
-                const int c = 2 * pair + s;
-                const int cls = whole ? 1 : classify(a, qi, f + 4 + 6 * s, q.qx, q.qy, q.qz, q.r);
-                if (cls == 0) continue;
-                if (sp < a.stack) stk[sp++ * 64 + lane] = entry(c, cls);
-                else atomicOr(a.overflow, 8);
+                    for (int s = 0; s < 2; ++s) {
+                        if ((lk & lk_has(s)) && !(lk & lk_td(s)))
+                            c[s] = whole ? 1 : classify(a, qi, f + 4 + 6 * s, q.qx, q.qy, q.qz, q.r);
+                    }
+                    // own, left, right without the absent ones; no entry is 0 (node 0 is the sentinel)
+                    const int el = c[0] ? 2 * pair | (c[0] == 1 ? RANGE_WHOLE : 0) : 0;
+                    const int er = c[1] ? (2 * pair + 1) | (c[1] == 1 ? RANGE_WHOLE : 0) : 0;
+                    const bool own = !(lk & LK_PDEL) && (whole || range_takes(a, qi, q, f));
+                    e0 = own ? (u | RANGE_TASK | RANGE_WHOLE) : (el ? el : er);
+                    e1 = own ? (el ? el : er) : (el ? er : 0);
+                    e2 = (own && el) ? er : 0;
+                    m = (own ? 1 : 0) + (el ? 1 : 0) + (er ? 1 : 0);
+                    r = own ? 1 : 0;
+                }
             }
         }
+        sp -= b;
+        const unsigned long long open = __ballot(r < m);
+        const int first = open ? __ffsll((long long)open) - 1 : 64;
+        const int out = lane < first ? m : (lane == first ? r : 0);  // at most 1: an entry's items come first
+        const int rem = m - out;
+        const unsigned long long om = __ballot(out != 0);
+        const unsigned long long m1 = __ballot((rem & 1) != 0), m2 = __ballot((rem & 2) != 0);
+        const long long oat = items + lanes_below(om, lane);
+        if (out) {
+            if (list) {
+                if (oat < cap) dst[oat] = range_item_of(e0, qi);
+                else atomicOr(a.overflow, 8);  // more items than the first walk counted
+            } else if (oat < cap) {
+                raw[oat] = e0;
+            }
+        }
+        items += __popcll(om);
+        const int total = __popcll(m1) + 2 * __popcll(m2);
+        // the entry of order o goes to sp + total - 1 - o
+        int at = sp + total - 1 - (lanes_below(m1, lane) + 2 * lanes_below(m2, lane));
+        range_lds_fence();  // every lane has read its entry
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            if (i < out || i >= m) continue;
+            if (at < a.stack) stk[at] = i == 0 ? e0 : (i == 1 ? e1 : e2);
+            else atomicOr(a.overflow, 8);
+            --at;
+        }
+        sp += total;
+        if (sp > a.stack) break;  // flagged above
+        range_lds_fence();
     }
-    if (!list) a.tcounts[qi] = items;
+    if (!list && lane == 0) a.tcounts[qi] = items;
 }
 
 // The points one item holds: counted (fill false) or written from pos on in
@@ -1198,8 +1276,14 @@ __global__ __launch_bounds__(64) void k_range_item_fill(RangeArgs a, long long n
 
 void launch_range_top(const RangeArgs& a, int list, hipStream_t s) {
     if (a.nq <= 0) return;
-    hipLaunchKernelGGL(k_range_top, dim3(blocks_for(a.nq, 64)), dim3(64), (size_t)a.stack * 64 * sizeof(int), s, a,
-                       list);
+    // 16 KB of stack a wavefront while the queries do not fill the device (the
+    // widest frontiers then still go 64 at a time), 4 KB when occupancy counts
+    RangeArgs b = a;
+    b.stack = a.nq <= RANGE_FEW_QUERIES ? 4096 : 1024;
+    constexpr int STEP = 1 << 25;  // a grid holds fewer than 2^32 lanes
+    for (int q0 = 0; q0 < a.nq; q0 += std::min(STEP, a.nq - q0))
+        hipLaunchKernelGGL(k_range_top, dim3(std::min(STEP, a.nq - q0)), dim3(64), (size_t)b.stack * sizeof(int), s, b,
+                           list, q0);
 }
 void launch_range_item_count(const RangeArgs& a, long long ntask, long long* counts, hipStream_t s) {
     if (ntask <= 0) return;
