@@ -1443,13 +1443,17 @@ int add_points_dev(ikd_tree_t t, const float* d_xyz, const uint32_t* d_ids, int 
     return compact_if_needed(t, false, true);
 }
 
-// Lanes per query so that a launch has about 2^17 lanes in flight: a small
-// batch (one scan) shares each query among a team of lanes, a large batch
-// keeps one lane per query (the most work-efficient form).
+// Lanes per query.  A small batch is bound by its longest walk, which a team
+// splits; a large one by the work of a visit, which is least with one lane.
+// Measured crossings on LiDAR and uniform maps of 0.1-1M points (us, k = 5 on
+// the 1M LiDAR map, lanes 16 / 8 / 4 / 2 / 1): 10k queries 48/58/68/98/97, 20k
+// 68/59/70/105/100, 40k 101/84/80/114/127, 80k 163/119/110/125/131, 160k
+// 292/196/158/162/142; the same side wins for k = 1, 10 and 20 and in
+// multi-map launches.
 int auto_lanes(int nq) {
-    int lanes = 1;
-    while (lanes < 16 && (long long)nq * lanes < (1ll << 17)) lanes *= 2;
-    return lanes;
+    if (nq <= (1 << 14)) return 16;
+    if (nq <= (1 << 15)) return 8;
+    return nq < (1 << 17) ? 4 : 1;
 }
 
 float max_dist_threshold(double max_dist) {

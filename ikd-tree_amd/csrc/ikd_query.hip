@@ -178,6 +178,24 @@ __device__ __forceinline__ void finish_query(const KnnArgs& a, const QueryCtx& c
     if (a.boxes) a.boxes[c.qo] = boxes;
 }
 
+// The children of a visited node within the bound (near first, left on ties),
+// or -1, and their box distances.  link: the record's link word.
+__device__ __forceinline__ void children(const QueryCtx& c, float link, const gv4& r1, const gv4& r2, const gv4& r3,
+                                         float lim, int& near_n, float& dn, int& far_n, float& df) {
+    const uint32_t lk = fbits(link);
+    const bool el = (lk & (LK_HASL | LK_TDL)) == LK_HASL, er = (lk & (LK_HASR | LK_TDR)) == LK_HASR;
+    const float bl[6] = {r1.x, r1.y, r1.z, r1.w, r2.x, r2.y};
+    const float br[6] = {r2.z, r2.w, r3.x, r3.y, r3.z, r3.w};
+    const float dl = calc_box_dist(bl, c.qx, c.qy, c.qz);
+    const float dr = calc_box_dist(br, c.qx, c.qy, c.qz);
+    const bool nl = el & (!er | (dl <= dr));
+    dn = nl ? dl : dr;
+    df = nl ? dr : dl;
+    const int near_c = (int)((lk >> (LK_PAIR_SHIFT - 1)) & ~1u) | (nl ? 0 : 1);
+    near_n = ((el | er) & (dn <= lim)) ? near_c : -1;
+    far_n = ((el & er) & (df <= lim)) ? (near_c ^ 1) : -1;
+}
+
 // One visit of node n: offers its point, then computes both children's box
 // distances.  lim is the walk's bound, min(cap, k-th distance) with cap = min(
 // max_dist's threshold, a team's bound): nothing above it is offered or
@@ -203,17 +221,7 @@ __device__ __forceinline__ void visit_node(const QueryCtx& c, BestList<KM>& best
         lim = fminf_raw(cap, best.d[0]);
     }
     if (COUNT) boxes += ((lk & LK_HASL) ? 1u : 0u) + ((lk & LK_HASR) ? 1u : 0u);
-    const bool el = (lk & (LK_HASL | LK_TDL)) == LK_HASL, er = (lk & (LK_HASR | LK_TDR)) == LK_HASR;
-    const float bl[6] = {r1.x, r1.y, r1.z, r1.w, r2.x, r2.y};
-    const float br[6] = {r2.z, r2.w, r3.x, r3.y, r3.z, r3.w};
-    const float dl = calc_box_dist(bl, c.qx, c.qy, c.qz);
-    const float dr = calc_box_dist(br, c.qx, c.qy, c.qz);
-    const bool nl = el & (!er | (dl <= dr));
-    dn = nl ? dl : dr;
-    df = nl ? dr : dl;
-    const int near_c = (int)((lk >> (LK_PAIR_SHIFT - 1)) & ~1u) | (nl ? 0 : 1);
-    near_n = ((el | er) & (dn <= lim)) ? near_c : -1;
-    far_n = ((el & er) & (df <= lim)) ? (near_c ^ 1) : -1;
+    children(c, r0.w, r1, r2, r3, lim, near_n, dn, far_n, df);
 }
 
 // ---- LDS traversal stacks --------------------------------------------------
@@ -504,12 +512,19 @@ __global__ __launch_bounds__(64) void k_knn_staged(KnnArgs a) {
 // deferred far children (a ring buffer in LDS holding at most one entry per
 // level of its current walk, so never more than the tree depth).  Whenever a
 // lane is idle, a busy teammate donates the bottom (shallowest) entry of its
-// deque.  Each lane keeps its own best-k list; the pruning bound is the
-// smallest k-th distance of the team, which is never below the true k-th
-// distance, so nothing of the answer is pruned.  At the end the T lists are
-// merged by rank in the total order.  Every node is reached through exactly
-// one parent, so no point is offered twice and the merge sees distinct
-// candidates.
+// deque.  The team keeps ONE best-k list, ascending over its lanes (lane i
+// holds the positions [i S, (i + 1) S)): a candidate is broadcast, every lane
+// ranks its slots against it and the later ones move up by one, the last slot
+// of a lane to its neighbour.  So every lane prunes with the team's k-th
+// distance, nothing is merged at the end, and a lane needs k / T registers of
+// list.  Every node is reached through exactly one parent, so no point is
+// offered twice.
+//
+// A list per lane, merged by rank at the end, took 250 us of one 10-nearest
+// search with 16 lanes (each of 160 candidates against the other 159) and 800
+// us of a 20-nearest one, where the walk itself takes 30; now 10k
+// queries on a 100k map, 16 lanes each, take 71 us (k = 10) and 112 (k = 20)
+// where they took 303 and 1793.
 __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -536,7 +551,16 @@ __device__ __forceinline__ int slot_get(const LdsStack& st, const uint32_t* cst,
     return st.n[i];
 }
 
-template <int KM, int T, bool COMPACT>
+// the value of the lane before (any value on the first lane of a team)
+__device__ __forceinline__ int lane_before(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_mov_dpp(v, 0x111, 0xf, 0xf, true);  // row_shr:1, teams never cross a row of 16
+#else
+    return __shfl(v, (int)((threadIdx.x + 63u) & 63u));
+#endif
+}
+
+template <int S, int T, bool COMPACT>
 __global__ __launch_bounds__(64) void k_knn_team(KnnArgs a) {
     constexpr int TEAMS = 64 / T;
     const LdsStack st = lds_stack(a.stack);
@@ -545,43 +569,33 @@ __global__ __launch_bounds__(64) void k_knn_team(KnnArgs a) {
     const int smask = a.stack - 1;  // team launches use a power-of-two stack
     __shared__ int dn_n[TEAMS][T];
     __shared__ float dn_d[TEAMS][T];
-    __shared__ float mg_d[TEAMS][T * KM];
-    __shared__ int mg_n[TEAMS][T * KM];
     const int lane = threadIdx.x;
     const int team = lane / T, tl = lane % T;
-    const unsigned long long team_mask = (T == 64) ? ~0ull : (((1ull << T) - 1ull) << (team * T));
+    const unsigned long long team_mask = ((1ull << T) - 1ull) << (team * T);
     const unsigned long long below = (1ull << lane) - 1ull;
     const int qi = xcd_chunk(blockIdx.x, (a.nq + TEAMS - 1) / TEAMS) * TEAMS + team;
     const bool valid = qi < a.nq;
-    QueryCtx c = load_query(a, valid ? qi : 0);
-    if (!valid) c.k = 1;
-    BestList<KM> best;
-    best.init(c.k);
-    unsigned int visits = 0, boxes = 0;
-    int head = 0, tail = 0;  // deque [head, tail) modulo a.stack
-
-    int n = -1;
-    float bd = 0.0f;
-    if (valid && tl == 0) {
-        const uint32_t lk0 = fbits(c.hot[SENTINEL].f[3]);
-        if ((lk0 & LK_HASL) && !(lk0 & LK_TDL)) {
-            n = ROOT;
-            bd = calc_box_dist(c.hot[SENTINEL].f + 4, c.qx, c.qy, c.qz);
-        }
+    const QueryCtx c = load_query(a, valid ? qi : 0);
+    float sd[S];
+    int sn[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+        sd[i] = INFINITY;
+        sn[i] = -1;
     }
-    float B = INFINITY;  // team bound: min over the team's k-th distances
+    const int klast = c.k > 0 ? c.k - 1 : 0;  // the k-th slot: lane klast / S, its slot klast % S
+    const int kslot = klast % S, klane = team * T + klast / S;
+    float lim = (valid && c.k > 0) ? c.thr : -INFINITY;  // min(max_dist's threshold, the k-th distance)
+    int head = 0, tail = 0;  // deque [head, tail) modulo a.stack
+    int n = (valid && tl == 0 && c.k > 0) ? knn_root(c) : -1;
     int iter = 0;
     while (true) {
         // an idle lane resumes the deepest entry of its own deque
         while (n < 0 && tail != head) {
             --tail;
-            const int s = tail & smask;
             float d;
-            const int e = slot_get<COMPACT>(st, cst, s * 64 + lane, &d);
-            if (d <= fminf(B, best.d[0])) {
-                n = e;
-                bd = d;
-            }
+            const int e = slot_get<COMPACT>(st, cst, (tail & smask) * 64 + lane, &d);
+            if (d <= lim) n = e;
         }
         // lanes still idle receive the bottom entry of a busy teammate
         const unsigned long long imask = __ballot(valid && n < 0) & team_mask;
@@ -595,9 +609,8 @@ __global__ __launch_bounds__(64) void k_knn_team(KnnArgs a) {
             if (donate && tail != head) {
                 const int r = __popcll(dmask & below);
                 if (r < ni) {
-                    const int s = head & smask;
                     float d;
-                    dn_n[team][r] = slot_get<COMPACT>(st, cst, s * 64 + lane, &d);
+                    dn_n[team][r] = slot_get<COMPACT>(st, cst, (head & smask) * 64 + lane, &d);
                     dn_d[team][r] = d;
                     ++head;
                 }
@@ -605,10 +618,7 @@ __global__ __launch_bounds__(64) void k_knn_team(KnnArgs a) {
             wave_lds_fence();
             if (donate && valid && n < 0) {
                 const int r = __popcll(imask & below);
-                if (r < nd) {
-                    n = dn_n[team][r];
-                    bd = dn_d[team][r];
-                }
+                if (r < nd && dn_d[team][r] <= lim) n = dn_n[team][r];
             }
             wave_lds_fence();
         }
@@ -618,73 +628,77 @@ __global__ __launch_bounds__(64) void k_knn_team(KnnArgs a) {
             break;
         }
 
+        gv4 r0, r1, r2, r3;
+        float d = 0.0f;
+        bool cand = false;
         if (n >= 0) {
-            const float cap = fminf(B, c.thr);
-            float bound = fminf(cap, best.d[0]);
-            if (bd > bound) {
-                n = -1;
-            } else {
-                ++visits;
-                int nn, fn;
-                float dn, df;
-                visit_node<KM, true>(c, best, n, cap, bound, nn, dn, fn, df, boxes);
-                if (fn >= 0) {
-                    if (tail - head < a.stack) {
-                        const int s = tail & smask;
-                        slot_put<COMPACT>(st, cst, s * 64 + lane, fn, df);
-                        ++tail;
-                    } else {
-                        atomicOr(a.overflow, 1);
-                    }
-                }
-                n = nn;
-                bd = dn;
-            }
+            const gv4* rec = reinterpret_cast<const gv4*>(c.hot[n].f);
+            r0 = gload4(rec);
+            r1 = gload4(rec + 1);
+            r2 = gload4(rec + 2);
+            r3 = gload4(rec + 3);
+            d = calc_dist(c.qx, c.qy, c.qz, r0.x, r0.y, r0.z);
+            cand = !(fbits(r0.w) & LK_PDEL) && d <= lim;
         }
-        float v = best.d[0];
+        // the round's candidates enter the lists, one per team at a time
+        unsigned long long cm = __ballot(cand);
+        while (cm != 0) {
+            const unsigned long long mine = cm & team_mask;
+            const int src = mine ? __ffsll((long long)mine) - 1 : lane;
+            const float cd = __shfl(d, src);
+            const int cn = __shfl(n, src);
+            const float pd = bitsf((uint32_t)lane_before((int)fbits(sd[S - 1])));
+            const int pn = lane_before(sn[S - 1]);
+            if (mine) {
+                bool up = tl > 0 && after(c.hot, c.ids, pd, pn, cd, cn);  // the slot before this one is later
+                float bd = pd;
+                int bn = pn;
 #pragma unroll
-        for (int off = T / 2; off >= 1; off >>= 1) v = fminf(v, __shfl_xor(v, off, T));
-        B = v;
+                for (int i = 0; i < S; ++i) {
+                    const float od = sd[i];
+                    const int on = sn[i];
+                    const bool later = after(c.hot, c.ids, od, on, cd, cn);
+                    sd[i] = later ? (up ? bd : cd) : od;
+                    sn[i] = later ? (up ? bn : cn) : on;
+                    up = later;
+                    bd = od;
+                    bn = on;
+                }
+            }
+            float kd = sd[0];
+#pragma unroll
+            for (int i = 1; i < S; ++i) kd = i == kslot ? sd[i] : kd;
+            kd = __shfl(kd, klane);
+            if (mine) lim = fminf_raw(c.thr, kd);
+            cand = cand && lane != src && d <= lim;
+            cm = __ballot(cand);
+        }
+        if (n >= 0) {
+            int nn, fn;
+            float dn, df;
+            children(c, r0.w, r1, r2, r3, lim, nn, dn, fn, df);
+            if (fn >= 0) {
+                if (tail - head < a.stack) {
+                    slot_put<COMPACT>(st, cst, (tail & smask) * 64 + lane, fn, df);
+                    ++tail;
+                } else {
+                    atomicOr(a.overflow, 1);
+                }
+            }
+            n = nn;
+        }
     }
 
-    // ---- merge the team's lists by rank in (d2, x, y, z, id) order
+    int found = 0;
 #pragma unroll
-    for (int i = 0; i < KM; ++i) {
-        mg_d[team][tl * KM + i] = best.d[i];
-        mg_n[team][tl * KM + i] = best.n[i];
-    }
-    wave_lds_fence();
-    int real = 0;
-    for (int cidx = tl; cidx < T * KM; cidx += T) real += mg_n[team][cidx] >= 0 ? 1 : 0;
-#pragma unroll
-    for (int off = T / 2; off >= 1; off >>= 1) real += __shfl_xor(real, off, T);
-    unsigned int vsum = visits, bsum = boxes;
-#pragma unroll
-    for (int off = T / 2; off >= 1; off >>= 1) {
-        vsum += __shfl_xor(vsum, off, T);
-        bsum += __shfl_xor(bsum, off, T);
-    }
+    for (int i = 0; i < S; ++i) found += __popcll(__ballot(sn[i] >= 0) & team_mask);
     if (!valid) return;
-    const int found = min(real, c.k);
-    for (int cidx = tl; cidx < T * KM; cidx += T) {
-        const int node = mg_n[team][cidx];
-        if (node < 0) continue;
-        const float d = mg_d[team][cidx];
-        int rank = 0;
-        for (int j = 0; j < T * KM; ++j) {
-            const int nj = mg_n[team][j];
-            if (nj < 0 || j == cidx) continue;
-            const float dj = mg_d[team][j];
-            if (dj < d || (dj == d && tie_less(c.hot, c.ids, nj, node))) ++rank;
-        }
-        if (rank < c.k) write_slot(a, c, rank, d, node);
-    }
+    found = min(found, c.k);
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+        if (tl * S + i < found) write_slot(a, c, tl * S + i, sd[i], sn[i]);
     for (int j = found + tl; j < a.out_stride; j += T) write_slot(a, c, j, INFINITY, -1);
-    if (tl == 0) {
-        a.out_counts[c.qo] = found;
-        if (a.visits) a.visits[c.qo] = vsum;
-        if (a.boxes) a.boxes[c.qo] = bsum;
-    }
+    if (tl == 0) a.out_counts[c.qo] = found;
 }
 
 // ---- persistent lanes -----------------------------------------------------
@@ -790,11 +804,6 @@ static int launch_knn_km(const KnnArgs& a0, int lanes, int stack, hipStream_t s,
                          int persist_waves) {
     KnnArgs a = a0;
     dim3 block(64);
-    if (lanes >= 2) {  // team deques are ring buffers: round the stack up to a power of two
-        int p = 1;
-        while (p < stack) p <<= 1;
-        stack = p;
-    }
     a.stack = stack;
     const size_t lds = lds_stack_bytes(stack);
     switch (lanes) {
@@ -831,46 +840,51 @@ static int launch_knn_km(const KnnArgs& a0, int lanes, int stack, hipStream_t s,
                 hipLaunchKernelGGL((k_knn_persist<KM, false>), dim3(xcd_grid(waves)), block, lb, s, a, persist_next);
             return 0;
         }
-        case 2:
-            if (a.compact_stack)
-                hipLaunchKernelGGL((k_knn_team<KM, 2, true>), dim3(xcd_grid(blocks_for(a.nq, 32))), block,
-                                   lds_compact_bytes(stack), s, a);
-            else
-                hipLaunchKernelGGL((k_knn_team<KM, 2, false>), dim3(xcd_grid(blocks_for(a.nq, 32))), block, lds,
-                                   s, a);
-            return 0;
-        case 4:
-            if (a.compact_stack)
-                hipLaunchKernelGGL((k_knn_team<KM, 4, true>), dim3(xcd_grid(blocks_for(a.nq, 16))), block,
-                                   lds_compact_bytes(stack), s, a);
-            else
-                hipLaunchKernelGGL((k_knn_team<KM, 4, false>), dim3(xcd_grid(blocks_for(a.nq, 16))), block, lds,
-                                   s, a);
-            return 0;
-        case 8:
-            if (a.compact_stack)
-                hipLaunchKernelGGL((k_knn_team<KM, 8, true>), dim3(xcd_grid(blocks_for(a.nq, 8))), block,
-                                   lds_compact_bytes(stack), s, a);
-            else
-                hipLaunchKernelGGL((k_knn_team<KM, 8, false>), dim3(xcd_grid(blocks_for(a.nq, 8))), block, lds,
-                                   s, a);
-            return 0;
-        case 16:
-            if (a.compact_stack)
-                hipLaunchKernelGGL((k_knn_team<KM, 16, true>), dim3(xcd_grid(blocks_for(a.nq, 4))), block,
-                                   lds_compact_bytes(stack), s, a);
-            else
-                hipLaunchKernelGGL((k_knn_team<KM, 16, false>), dim3(xcd_grid(blocks_for(a.nq, 4))), block, lds,
-                                   s, a);
-            return 0;
         default:
             return -1;
     }
 }
 
+template <int S, int T>
+static int launch_knn_team(const KnnArgs& a0, int stack, hipStream_t s) {
+    KnnArgs a = a0;
+    a.stack = 1;  // the deques are ring buffers: a power of two
+    while (a.stack < stack) a.stack <<= 1;
+    const dim3 grid(xcd_grid(blocks_for(a.nq, 64 / T))), block(64);
+    if (a.compact_stack)
+        hipLaunchKernelGGL((k_knn_team<S, T, true>), grid, block, lds_compact_bytes(a.stack), s, a);
+    else
+        hipLaunchKernelGGL((k_knn_team<S, T, false>), grid, block, lds_stack_bytes(a.stack), s, a);
+    return 0;
+}
+
+template <int T>
+static int launch_knn_teams(const KnnArgs& a, int kmax, int stack, hipStream_t s) {
+    const int need = (kmax + T - 1) / T;  // list slots per lane
+    if (need <= 1) return launch_knn_team<1, T>(a, stack, s);
+    if (need <= 2) return launch_knn_team<2, T>(a, stack, s);
+    if (need <= 3) return launch_knn_team<3, T>(a, stack, s);
+    if (need <= 5) return launch_knn_team<5, T>(a, stack, s);
+    if constexpr (T <= 8)
+        if (need <= 8) return launch_knn_team<8, T>(a, stack, s);
+    if constexpr (T <= 4)
+        if (need <= 16) return launch_knn_team<16, T>(a, stack, s);
+    if constexpr (T <= 2)
+        if (need <= 32) return launch_knn_team<32, T>(a, stack, s);
+    return -1;
+}
+
 int launch_knn(const KnnArgs& a, int kmax, int lanes, int stack, hipStream_t s, int* persist_next,
                int persist_waves) {
     if (a.nq <= 0) return 0;
+    if (kmax > 64) return -1;
+    switch (lanes) {
+        case 2: return launch_knn_teams<2>(a, kmax, stack, s);
+        case 4: return launch_knn_teams<4>(a, kmax, stack, s);
+        case 8: return launch_knn_teams<8>(a, kmax, stack, s);
+        case 16: return launch_knn_teams<16>(a, kmax, stack, s);
+        default: break;
+    }
     if (lanes == 0) launch_fill_i32(persist_next, 0, NUM_XCD, s);
 #define IKD_KNN(KMV) return launch_knn_km<KMV>(a, lanes, stack, s, persist_next, persist_waves)
     if (kmax <= 1) IKD_KNN(1);
@@ -883,9 +897,7 @@ int launch_knn(const KnnArgs& a, int kmax, int lanes, int stack, hipStream_t s, 
     if (kmax <= 20) IKD_KNN(20);
     if (kmax <= 32) IKD_KNN(32);
 #undef IKD_KNN
-    if (kmax <= 64) return launch_knn_km<64>(a, lanes <= 1 ? lanes : (lanes > 4 ? 4 : lanes), stack, s, persist_next,
-                                             persist_waves);
-    return -1;
+    return launch_knn_km<64>(a, lanes, stack, s, persist_next, persist_waves);
 }
 
 // ------------------------------------------------ per-query max_dist thresholds
