@@ -38,7 +38,8 @@ __global__ void k_reset_counters(DevHdr* h, int which) {
     if (which & 2) h->rec_count = 0;
     if (which & 4) h->conflicts = 0;
     if (which & 8) { h->split_index = INT_MAX; h->added = 0; h->ins_count = 0; }
-    if (which & 16) h->group_count = 0;
+    if (which & 16) { h->group_count = 0; h->ins_maxlen = 0; }
+    if (which & 32) h->vox_bad = 0;
 }
 
 __global__ void k_link_defer_flags(Pool pool, const int* __restrict__ defer, int n) {
@@ -91,10 +92,10 @@ __global__ void k_seeds_from_attach(const int* __restrict__ attach, DevHdr* hdr,
     seeds[g] = g < hdr->group_count ? (attach[g] >> 1) : -1;
 }
 
-__global__ void k_group_maxlen(const int4* __restrict__ seg, DevHdr* hdr, int bound, int* __restrict__ out) {
+__global__ void k_group_maxlen(const int4* __restrict__ seg, DevHdr* hdr, int bound) {
     int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= bound || g >= hdr->group_count) return;
-    atomicMax(out, seg[g].y - seg[g].x + 1);
+    atomicMax(&hdr->ins_maxlen, seg[g].y - seg[g].x + 1);
 }
 
 // (node, live points, depth, parent) of the topmost violators, plus the node
@@ -106,7 +107,7 @@ __global__ void k_node_info(Pool pool, const int* __restrict__ top, const int* _
     int u = top[2 * i];
     int4 c = pool.cnt[u];
     out[i] = make_int4(u, c.x - c.y, c.w, pool.par[u]);
-    nodes_before[i] = top[2 * i + 1] + pend[u];
+    nodes_before[i] = top[2 * i + 1] + (pend ? pend[u] : 0);
 }
 
 
@@ -150,32 +151,30 @@ struct RootInfo {
 // Subtrees to rebuild whose summaries come back with the header in one copy
 // (more than this: a second read).
 constexpr int TOPINFO_CAP = 1024;
+// Host searches whose queries and results fit this go through page-locked
+// memory without a copy (above it, one DMA each way costs less than the
+// kernel's small writes over PCIe).
+constexpr int64_t HOST_IO_BYTES = 64 << 10;
 // What one host wait brings back: the header, the root summary and, after a
 // refit, (node, live points, depth, parent) and the node count of the first
-// TOPINFO_CAP topmost violators.  One device block and its pinned mirror.
+// TOPINFO_CAP topmost violators.  In page-locked host memory that kernels write.
 struct DevStatus {
     DevHdr hdr;
     RootInfo root;
     int4 top_info[TOPINFO_CAP];
     int top_before[TOPINFO_CAP];
+    long long count;  // a published count
 };
-constexpr size_t STATUS_SHORT = offsetof(DevStatus, top_info);  // header + root summary
-__global__ void k_top_info(Pool pool, const int* __restrict__ top, const int* __restrict__ pend, DevStatus* s) {
-    const int n = min(s->hdr.top_count, TOPINFO_CAP);
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const int u = top[2 * i];
-        const int4 c = pool.cnt[u];
-        s->top_info[i] = make_int4(u, c.x - c.y, c.w, pool.par[u]);
-        s->top_before[i] = top[2 * i + 1] + pend[u];
-    }
+// The three kernels below write what the host waits for straight into its
+// page-locked mirror: a wait costs its kernel, not a copy engine's turn (and a
+// second launch for the root summary) behind it.
+__device__ __forceinline__ void publish_hdr(const DevHdr* hdr, DevStatus* host) {
+    const int* src = reinterpret_cast<const int*>(hdr);
+    int* dst = reinterpret_cast<int*>(&host->hdr);
+    for (int i = threadIdx.x; i < (int)(sizeof(DevHdr) / sizeof(int)); i += blockDim.x) dst[i] = src[i];
 }
-// Enumerate: the walk must have written exactly the live points the
-// subtrees' counts promise (overflow bit 32 otherwise, reported by the next
-// header read).
-__global__ void k_enum_check(DevHdr* hdr, int expect) {
-    if (hdr->rec_count != expect) atomicOr(&hdr->overflow, 32);
-}
-__global__ void k_root_info(Pool pool, RootInfo* out) {
+__device__ __forceinline__ void publish_root(const Pool& pool, DevStatus* host) {
+    if (threadIdx.x != 0) return;
     RootInfo r = {};
     uint32_t lk0 = fbits(pool.hot[SENTINEL].f[3]);
     r.child.z = (int)lk0;
@@ -187,9 +186,34 @@ __global__ void k_root_info(Pool pool, RootInfo* out) {
         r.child.y = (lk & LK_HASR) ? pool.cnt[2 * pair + 1].x : -1;
         for (int i = 0; i < 6; ++i) r.box[i] = pool.hot[SENTINEL].f[4 + i];
     }
-    *out = r;
+    host->root = r;
 }
-
+__global__ void k_publish_count(const long long* src, long long* host) { *host = *src; }
+__global__ void k_publish_hdr(const DevHdr* hdr, DevStatus* host) { publish_hdr(hdr, host); }
+__global__ void k_publish_root(Pool pool, const DevHdr* hdr, DevStatus* host, int with_hdr) {
+    publish_root(pool, host);
+    if (with_hdr) publish_hdr(hdr, host);
+}
+// top null: no list (the header's count is 0)
+__global__ void k_publish_tops(Pool pool, const DevHdr* hdr, const int* __restrict__ top,
+                               const int* __restrict__ pend, DevStatus* host) {
+    publish_root(pool, host);
+    publish_hdr(hdr, host);
+    if (!top) return;
+    const int n = min(hdr->top_count, TOPINFO_CAP);
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        const int u = top[2 * i];
+        const int4 c = pool.cnt[u];
+        host->top_info[i] = make_int4(u, c.x - c.y, c.w, pool.par[u]);
+        host->top_before[i] = top[2 * i + 1] + (pend ? pend[u] : 0);
+    }
+}
+// Enumerate: the walk must have written exactly the live points the
+// subtrees' counts promise (overflow bit 32 otherwise, reported by the next
+// header read).
+__global__ void k_enum_check(DevHdr* hdr, int expect) {
+    if (hdr->rec_count != expect) atomicOr(&hdr->overflow, 32);
+}
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
@@ -216,12 +240,12 @@ struct ikd_tree_s {
     // node pool
     long long cap = 0;
     Pool pool{};
-    DevStatus* d_status = nullptr;  // header, root summary, rebuild list
-    DevStatus* h_status = nullptr;  // its pinned mirror
-    DevHdr* d_hdr = nullptr;        // &d_status->hdr
-    DevHdr* h_hdr = nullptr;
-    RootInfo* d_root = nullptr;  // &d_status->root
-    RootInfo* h_root = nullptr;
+    DevHdr* d_hdr = nullptr;
+    DevStatus* h_status = nullptr;  // page-locked: header, root summary, rebuild list as last published
+    DevHdr* h_hdr = nullptr;        // &h_status->hdr
+    RootInfo* h_root = nullptr;     // &h_status->root
+    long long* h_count = nullptr;   // &h_status->count
+    char* h_io = nullptr;           // page-locked queries and results of small host searches (HOST_IO_BYTES)
     uint32_t next_id = 0;
     long long rebuilds = 0;
     bool compact_due = false;  // a sparse pool left to ikd_rebuild_deferred
@@ -264,7 +288,8 @@ struct ikd_batch_s {
     int knn_lanes = -1;
     int knn_stack = 0;
     int knn_compact = 1;
-    int* h_flag = nullptr;  // pinned mirror of the overflow flags (the batch's, the scratch one)
+    long long* h_count = nullptr;  // page-locked: a published count
+    int* h_flag = nullptr;  // behind h_count: pinned mirror of the overflow flags (the batch's, the scratch one)
     char* na_scratch = nullptr;  // this device's allocation-free scratch (ikd_batch_nearest_search_noalloc)
     int* na_flag = nullptr;      // its overflow flag, once the entry point ran on this batch
     ikd_counters_t ctr{};   // only scratch_grows and host_waits move
@@ -281,7 +306,7 @@ enum Buf {
     B_SID2, B_SIDE, B_SEG0, B_SEG1, B_SEGD0, B_SEGD1, B_SEGAX, B_SEGMID, B_SEGCH, B_SEGFL, B_SEGSC, B_POSFL, B_POSSC,
     B_SEEDS, B_DIRTY, B_VIOL, B_TOP, B_INFO, B_FRONT0, B_FRONT1, B_EKEY0, B_EKEY1, B_RECS, B_GFLAG, B_GSCAN, B_ATTACH,
     B_PFLAG, B_PSCAN, B_ISEG, B_ISEGD, B_IO0, B_IO1, B_IO2, B_IO3, B_IO4, B_VSTART, B_DELBOX, B_DELFL, B_INSPT,
-    B_INSFL, B_CBOX, B_CPTS, B_MISC, B_MORTK, B_MORTV, B_MORTK2, B_MORTV2, B_CNT64, B_OFF64, B_ADDX, B_ADDI, B_PNEXT, B_SPAIRS, B_SPSCAN,
+    B_INSFL, B_CBOX, B_CPTS, B_MORTK, B_MORTV, B_MORTK2, B_MORTV2, B_CNT64, B_OFF64, B_ADDX, B_ADDI, B_PNEXT, B_SPAIRS, B_SPSCAN,
     B_DEFER, B_DINFO, B_DBEFORE, B_DKEEP, B_PTS3, B_PEND, B_START, B_INV0, B_LASTP, B_PSEED, B_DBELOW, B_MAXDEL,
     B_SLISTS, B_ENUMROOT, B_ENUMGRP, B_TOPT, B_TOPI, B_TCNT64, B_TOFF64, B_RTASKS, B_ICNT64, B_EMPTYL, B_RAW, B_COUNT
 };
@@ -439,9 +464,9 @@ int check_count(Owner* t, const char* what, long long v, long long lo, long long
     return IKD_ERR_INTERNAL;
 }
 
-// Copies the first `bytes` of the status block back and waits.
-int read_status(ikd_tree_t t, size_t bytes) {
-    HIPCHK(hipMemcpyAsync(t->h_status, t->d_status, bytes, hipMemcpyDeviceToHost, t->st));
+// Waits for a published status (the publishing kernel is queued) and takes it over.
+int take_status(ikd_tree_t t) {
+    HIPCHK(hipGetLastError());
     HIPCHK(wait_stream(t));
     t->pool_used = 2ll * t->h_hdr->pair_used;
     t->max_depth = t->h_hdr->max_depth;
@@ -455,18 +480,21 @@ int read_status(ikd_tree_t t, size_t bytes) {
     }
     return IKD_OK;
 }
-int sync_hdr(ikd_tree_t t) { return read_status(t, sizeof(DevHdr)); }
+int sync_hdr(ikd_tree_t t) {
+    hipLaunchKernelGGL(k_publish_hdr, dim3(1), dim3(64), 0, t->st, t->d_hdr, t->h_status);
+    return take_status(t);
+}
 
 int read_root(ikd_tree_t t) {
-    hipLaunchKernelGGL(k_root_info, dim3(1), dim3(1), 0, t->st, t->pool, t->d_root);
-    HIPCHK(hipMemcpyAsync(t->h_root, t->d_root, sizeof(RootInfo), hipMemcpyDeviceToHost, t->st));
+    hipLaunchKernelGGL(k_publish_root, dim3(1), dim3(64), 0, t->st, t->pool, t->d_hdr, t->h_status, 0);
+    HIPCHK(hipGetLastError());
     HIPCHK(wait_stream(t));
     return IKD_OK;
 }
-// Header and root summary in one copy and one host wait.
+// Header and root summary in one kernel and one host wait.
 int refresh(ikd_tree_t t) {
-    hipLaunchKernelGGL(k_root_info, dim3(1), dim3(1), 0, t->st, t->pool, t->d_root);
-    return read_status(t, STATUS_SHORT);
+    hipLaunchKernelGGL(k_publish_root, dim3(1), dim3(64), 0, t->st, t->pool, t->d_hdr, t->h_status, 1);
+    return take_status(t);
 }
 bool has_root(ikd_tree_t t) { return (t->h_root->child.z & (int)LK_HASL) != 0; }
 long long live_count(ikd_tree_t t) {
@@ -1036,10 +1064,10 @@ int rebuild_tops(ikd_tree_t t) {
         // the header, the root summary and the first subtrees to rebuild in one wait
         // (the refit's list; after a pass of rebuilds the list is empty)
         const int* top = iter == 0 ? reinterpret_cast<const int*>(t->b[B_TOP].p) : nullptr;
-        const int* pend = reinterpret_cast<const int*>(t->b[B_PEND].p);
-        hipLaunchKernelGGL(k_root_info, dim3(1), dim3(1), 0, st, t->pool, t->d_root);
-        if (top) hipLaunchKernelGGL(k_top_info, dim3(1), dim3(256), 0, st, t->pool, top, pend, t->d_status);
-        CHK(read_status(t, top ? sizeof(DevStatus) : STATUS_SHORT));
+        // only a recording rebuild walks the nodes that lower violators hide
+        const int* pend = t->record_removed ? reinterpret_cast<const int*>(t->b[B_PEND].p) : nullptr;
+        hipLaunchKernelGGL(k_publish_tops, dim3(1), dim3(256), 0, st, t->pool, t->d_hdr, top, pend, t->h_status);
+        CHK(take_status(t));
         int ntop = t->h_hdr->top_count;
         CHK(check_count(t, "rebuild: subtrees", ntop, 0, t->pool_used));
         if (ntop == 0) return IKD_OK;
@@ -1165,17 +1193,12 @@ int insert_points(ikd_tree_t t, const float4* pts, int m, const int* extra_seeds
     launch_insert_segments2(t->pool, kb, gscan, gflag, m, seg, segd, segof, attach, pflag, t->d_hdr, st);
     CHK(exscan_i32(t, pflag, pscan, m));
     launch_insert_pairs(t->pool, attach, pflag, pscan, t->d_hdr, m, seg, st);
-    int* misc;
-    CHK(ensure(t, B_MISC, 4, &misc));
-    launch_fill_i32(misc, 0, 1, st);
-    hipLaunchKernelGGL(k_group_maxlen, dim3(nblk(m)), dim3(BS), 0, st, seg, t->d_hdr, m, misc);
+    hipLaunchKernelGGL(k_group_maxlen, dim3(nblk(m)), dim3(BS), 0, st, seg, t->d_hdr, m);
     float4* spts;
     CHK(ensure(t, B_PTS2, m, &spts));
     hipLaunchKernelGGL(k_gather_pts, dim3(nblk(m)), dim3(BS), 0, st, pts, vb, m, spts);
-    int maxlen = 0;
-    HIPCHK(hipMemcpyAsync(&maxlen, misc, sizeof(int), hipMemcpyDeviceToHost, st));
     CHK(sync_hdr(t));
-    int S = t->h_hdr->group_count;
+    const int S = t->h_hdr->group_count, maxlen = t->h_hdr->ins_maxlen;
     CHK(check_count(t, "insert: attach groups", S, 1, m));
     CHK(check_count(t, "insert: largest group", maxlen, 1, m));
     CHK(run_build(t, spts, segof, m, seg, segd, S, maxlen));
@@ -1304,7 +1327,8 @@ int add_points_ds_chunk(ikd_tree_t t, const float* d_xyz, const uint32_t* d_ids,
     unsigned long long *ka, *kb;
     uint32_t *va, *vb;
     float4* pts;
-    int *flag, *scan, *vstart, *bad;
+    int *flag, *scan, *vstart;
+    int* const bad = &t->d_hdr->vox_bad;
     CHK(ensure(t, B_MORTK, n, &ka));
     CHK(ensure(t, B_MORTK2, n, &kb));
     CHK(ensure(t, B_MORTV, n, &va));
@@ -1313,13 +1337,11 @@ int add_points_ds_chunk(ikd_tree_t t, const float* d_xyz, const uint32_t* d_ids,
     CHK(ensure(t, B_GFLAG, n, &flag));
     CHK(ensure(t, B_GSCAN, n, &scan));
     CHK(ensure(t, B_VSTART, n + 1, &vstart));
-    CHK(ensure(t, B_MISC, 4, &bad));
-    launch_fill_i32(bad, 0, 4, st);
+    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(1), 0, st, t->d_hdr, 2 | 8 | 16 | 32);
     launch_voxel_keys2(d_xyz, d_ids, id_base, n, t->prm.box_length, ka, va, pts, bad, st);
     CHK(sort_pairs(t, ka, kb, va, vb, n, 63));
     launch_voxel_flags(kb, n, flag, st);
     CHK(exscan_i32(t, flag, scan, n));
-    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(1), 0, st, t->d_hdr, 16);
     launch_voxel_starts(flag, scan, n, vstart, t->d_hdr, st);
     float* delbox;
     float4* inspt;
@@ -1345,14 +1367,12 @@ int add_points_ds_chunk(ikd_tree_t t, const float* d_xyz, const uint32_t* d_ids,
     }
     for (int pass = 0; pass < passes; ++pass) {
         const bool deleting = apply && pass == passes - 1;
-        hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(1), 0, st, t->d_hdr, 2 | 8);
+        if (pass > 0) hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(1), 0, st, t->d_hdr, 2 | 8);
         launch_voxel_fold2(t->pool, pts, vb, kb, vstart, n, n, t->prm.box_length, check, delbox, delfl, inspt, insfl,
                            t->d_hdr, t->pool_used + 16, deleting ? dseeds : nullptr, (int)dcap, fold_stack, fold_lanes,
                            bad, st);
-        int hbad = 0;
-        HIPCHK(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, st));
         CHK(sync_hdr(t));
-        if (hbad) {
+        if (t->h_hdr->vox_bad) {
             t->err = "Add_Points: a voxel index floor(p/box_length) is beyond +-2^20";
             return IKD_ERR_UNSUPPORTED;
         }
@@ -1542,7 +1562,8 @@ int knn_dev(ikd_tree_t t, const float* d_q, int nq, int k, double max_dist, floa
 // Range search plan on the owner's stream (count walk, item lists, item
 // counts, offsets): d_offsets (device, nq + 1) gets every query's first
 // output position; *total and *ntask come back to the host (two waits: the
-// item count sizes the lists, the total sizes the output).  slots: scratch
+// item count sizes the lists, the total sizes the output; h_offsets, when given,
+// takes all offsets in the second).  slots: scratch
 // slots for the per-query item counts and offsets, the items, the item
 // counts and offsets, and the items the first walk keeps.
 hipError_t owner_wait(ikd_tree_t t) { return wait_stream(t); }
@@ -1551,7 +1572,7 @@ hipError_t owner_wait(Owner* b) { return hipStreamSynchronize(b->st); }
 
 template <class Owner>
 int range_plan(Owner* t, RangeArgs& a, int nq, long long* d_offsets, const int (&slots)[6], long long pool_bound,
-               long long* total, long long* ntask_out) {
+               long long* h_offsets, long long* total, long long* ntask_out) {
     hipStream_t st = t->st;
     long long *tcnt, *toff, *icnt, *ioff;
     int4* items;
@@ -1564,9 +1585,10 @@ int range_plan(Owner* t, RangeArgs& a, int nq, long long* d_offsets, const int (
     CHK(ensure(t, slots[5], (long long)nq * a.raw_cap, &a.raw));
     launch_range_top(a, 0, st);
     CHK(exscan_i64(t, tcnt, toff, nq + 1));
-    long long ntask = 0;
-    HIPCHK(hipMemcpyAsync(&ntask, toff + nq, sizeof(long long), hipMemcpyDeviceToHost, st));
+    hipLaunchKernelGGL(k_publish_count, dim3(1), dim3(1), 0, st, toff + nq, t->h_count);
+    HIPCHK(hipGetLastError());
     HIPCHK(owner_wait(t));
+    const long long ntask = *t->h_count;
     CHK(check_count(t, "range search: items", ntask, 0, std::min<long long>((long long)nq * pool_bound, INT_MAX - 1)));
     CHK(ensure(t, slots[2], std::max<long long>(ntask, 1), &items));
     CHK(ensure(t, slots[3], ntask + 1, &icnt));
@@ -1579,8 +1601,11 @@ int range_plan(Owner* t, RangeArgs& a, int nq, long long* d_offsets, const int (
     CHK(exscan_i64(t, icnt, ioff, (int)ntask + 1));
     launch_range_query_offsets(toff, ioff, nq, d_offsets, st);
     a.item_offsets = ioff;
-    HIPCHK(hipMemcpyAsync(total, d_offsets + nq, sizeof(long long), hipMemcpyDeviceToHost, st));
+    if (h_offsets) HIPCHK(hipMemcpyAsync(h_offsets, d_offsets, (nq + 1) * sizeof(long long), hipMemcpyDeviceToHost, st));
+    else hipLaunchKernelGGL(k_publish_count, dim3(1), dim3(1), 0, st, d_offsets + nq, t->h_count);
+    HIPCHK(hipGetLastError());
     HIPCHK(owner_wait(t));
+    *total = h_offsets ? h_offsets[nq] : *t->h_count;
     *ntask_out = ntask;
     return IKD_OK;
 }
@@ -1606,9 +1631,11 @@ int range_dev(ikd_tree_t t, int mode, const float* d_boxes, const float* d_cente
     a.stack = std::min(t->max_depth + 2, MAX_DEPTH);
     long long total = 0, ntask = 0;
     static const int slots[6] = {B_TCNT64, B_TOFF64, B_RTASKS, B_CNT64, B_ICNT64, B_RAW};
-    CHK(range_plan(t, a, nq, off, slots, std::max<long long>(t->pool_used, 1), &total, &ntask));
-    HIPCHK(hipMemcpyAsync(h_offsets, off, (nq + 1) * sizeof(long long), hipMemcpyDeviceToHost, st));
-    CHK(sync_hdr(t));
+    static_assert(sizeof(int64_t) == sizeof(long long), "offsets");
+    CHK(range_plan(t, a, nq, off, slots, std::max<long long>(t->pool_used, 1), reinterpret_cast<long long*>(h_offsets),
+                   &total, &ntask));
+    // without results to deliver the walks' flags are read now, else with the last wait
+    if (!h_xyz || capacity < total || total == 0) CHK(sync_hdr(t));
     CHK(check_count(t, "range search: results", total, 0, (long long)nq * std::max<long long>(t->pool_used, 1)));
     if (!h_xyz) return IKD_OK;
     if (capacity < total) {
@@ -1657,15 +1684,14 @@ int ikd_create(float delete_param, float balance_param, float box_length, ikd_tr
     }
     t->mp = library_pool(dev);
     if (hipStreamCreateWithFlags(&t->st, hipStreamNonBlocking) != hipSuccess ||
-        hipMalloc(&t->d_status, sizeof(DevStatus)) != hipSuccess ||
+        hipMalloc(&t->d_hdr, sizeof(DevHdr)) != hipSuccess ||
         hipHostMalloc(&t->h_status, sizeof(DevStatus), hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&t->ev, hipEventDisableTiming) != hipSuccess) {
         ikd_destroy(t);
         return IKD_ERR_HIP;
     }
-    t->d_hdr = &t->d_status->hdr;
     t->h_hdr = &t->h_status->hdr;
-    t->d_root = &t->d_status->root;
+    t->h_count = &t->h_status->count;
     t->h_root = &t->h_status->root;
     // a zero header first: the pool's initialisation keeps only the record count
     launch_fill_i32(reinterpret_cast<int*>(t->d_hdr), 0, sizeof(DevHdr) / sizeof(int), t->st);
@@ -1693,8 +1719,9 @@ int ikd_destroy(ikd_tree_t t) {
         hipStreamSynchronize(t->st);
     }
     stage_release(t);
-    if (t->d_status) hipFree(t->d_status);
+    if (t->d_hdr) hipFree(t->d_hdr);
     if (t->h_status) hipHostFree(t->h_status);
+    if (t->h_io) hipHostFree(t->h_io);
     if (t->ev) hipEventDestroy(t->ev);
     if (t->st) hipStreamDestroy(t->st);
     delete t;
@@ -1771,15 +1798,39 @@ int ikd_nearest_search(ikd_tree_t t, const float* q, int64_t nq, int k, double m
         return IKD_ERR_ARG;
     }
     if (nq == 0) return IKD_OK;
-    float *dq, *dx, *dd;
-    uint32_t* di;
-    int* dc;
+    const int64_t nk = nq * k;
+    if (nq <= HOST_IO_BYTES / 16 && 12 * nq + 20 * nk + 4 * nq <= HOST_IO_BYTES) {
+        // A few queries: the kernel reads them from page-locked memory and writes
+        // its results there.  One query of a 100k-point map took 6 copies of 3 us
+        // each on the device and their gaps, 97 us in all, and now 53.
+        if (!t->h_io) HIPCHK(hipHostMalloc((void**)&t->h_io, HOST_IO_BYTES, hipHostMallocDefault));
+        float* hq = reinterpret_cast<float*>(t->h_io);
+        float* hx = hq + 3 * nq;
+        float* hd = hx + 3 * nk;
+        uint32_t* hi = reinterpret_cast<uint32_t*>(hd + nk);
+        int32_t* hc = reinterpret_cast<int32_t*>(hi + nk);
+        std::memcpy(hq, q, 12 * nq);
+        CHK(knn_dev(t, hq, (int)nq, k, max_dist, hx, hd, hi, hc, nullptr, nullptr));
+        CHK(sync_hdr(t));
+        std::memcpy(out_xyz, hx, 12 * nk);
+        std::memcpy(out_d2, hd, 4 * nk);
+        std::memcpy(out_ids, hi, 4 * nk);
+        std::memcpy(out_counts, hc, 4 * nq);
+        return IKD_OK;
+    }
+    float *dq, *dx;
+    // one block, so that results in one block on the host (xyz, d2, ids, counts
+    // in that order) come back in one copy
     CHK(upload(t, B_IO0, q, 3 * nq, &dq));
-    CHK(ensure(t, B_IO1, 3 * nq * k, &dx));
-    CHK(ensure(t, B_IO2, nq * k, &dd));
-    CHK(ensure(t, B_IO3, nq * k, &di));
-    CHK(ensure(t, B_IO4, nq, &dc));
+    CHK(ensure(t, B_IO1, 5 * nk + nq, &dx));
+    float* dd = dx + 3 * nk;
+    uint32_t* di = reinterpret_cast<uint32_t*>(dd + nk);
+    int* dc = reinterpret_cast<int*>(di + nk);
     CHK(knn_dev(t, dq, (int)nq, k, max_dist, dx, dd, di, dc, nullptr, nullptr));
+    if (out_d2 == out_xyz + 3 * nk && (void*)out_ids == (void*)(out_d2 + nk) && (void*)out_counts == (void*)(out_ids + nk)) {
+        HIPCHK(hipMemcpyAsync(out_xyz, dx, 20 * nk + 4 * nq, hipMemcpyDeviceToHost, t->st));
+        return sync_hdr(t);
+    }
     HIPCHK(hipMemcpyAsync(out_xyz, dx, 3 * nq * k * sizeof(float), hipMemcpyDeviceToHost, t->st));
     HIPCHK(hipMemcpyAsync(out_d2, dd, nq * k * sizeof(float), hipMemcpyDeviceToHost, t->st));
     HIPCHK(hipMemcpyAsync(out_ids, di, nq * k * sizeof(uint32_t), hipMemcpyDeviceToHost, t->st));
@@ -2314,7 +2365,7 @@ int ikd_get_counters(ikd_tree_t t, ikd_counters_t* out) {
 int ikd_device_bytes(ikd_tree_t t, int64_t* out_bytes) {
     CHECK_T();
     if (!out_bytes) return IKD_ERR_ARG;
-    int64_t b = (int64_t)sizeof(DevStatus);
+    int64_t b = (int64_t)sizeof(DevHdr);
     b += t->cap * (int64_t)(sizeof(NodeHot) + sizeof(uint32_t) + sizeof(int32_t) + sizeof(int4) + sizeof(uint32_t));
     for (const DevBuf& d : t->b) b += (int64_t)d.bytes;
     b += t->removed_cap * (int64_t)sizeof(float4);
@@ -2423,10 +2474,11 @@ int ikd_batch_create(ikd_batch_t* out) {
     b->mp = library_pool(dev);
     if (hipStreamCreateWithFlags(&b->st, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreateWithFlags(&b->ev, hipEventDisableTiming) != hipSuccess ||
-        hipHostMalloc(&b->h_flag, 2 * sizeof(int), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc(&b->h_count, sizeof(long long) + 2 * sizeof(int), hipHostMallocDefault) != hipSuccess) {
         ikd_batch_destroy(b);
         return IKD_ERR_HIP;
     }
+    b->h_flag = reinterpret_cast<int*>(b->h_count + 1);
     // set-up of the allocation-free entry point on this device (its absence
     // only disables that entry point)
     b->na_scratch = noalloc_scratch(dev);
@@ -2451,7 +2503,7 @@ int ikd_batch_destroy(ikd_batch_t b) {
         hipStreamSynchronize(b->st);
     }
     stage_release(b);
-    if (b->h_flag) hipHostFree(b->h_flag);
+    if (b->h_count) hipHostFree(b->h_count);
     if (b->ev) hipEventDestroy(b->ev);
     if (b->st) hipStreamDestroy(b->st);
     delete b;
@@ -2845,7 +2897,7 @@ int ikd_batch_radius_search_device(ikd_batch_t b, const ikd_tree_t* trees, int n
     long long total = 0, ntask = 0;
     static const int slots[6] = {BB_TCNT, BB_TOFF, BB_TASKS, BB_CNT, BB_ICNT, BB_RAW};
     CHK(range_plan(b, a, (int)nq, reinterpret_cast<long long*>(d_out_offsets), slots, std::max<long long>(steps, 1),
-                   &total, &ntask));
+                   nullptr, &total, &ntask));
     *out_total = total;
     if (total < 0) {
         b->err = "batch: device result count out of range";

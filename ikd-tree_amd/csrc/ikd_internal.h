@@ -34,6 +34,8 @@ struct DevHdr {
     int removed_count;  // points rebuilds removed since the last acquire (kept across calls)
     float alpha_bal;    // the root's alpha_bal / alpha_del as of its last Update (cpp:1315-1321)
     float alpha_del;
+    int vox_bad;        // downsample: a voxel index of the batch is out of range
+    int ins_maxlen;     // insert: points of the largest attach group
     int small_lists[2]; // small build: segments listed for the 64- and 256-thread workgroup builds
 };
 static_assert(sizeof(DevHdr) % sizeof(int) == 0, "the header is cleared as ints");

@@ -645,7 +645,7 @@ __global__ __launch_bounds__(64) void k_knn_team(KnnArgs a) {
         while (cm != 0) {
             const unsigned long long mine = cm & team_mask;
             const int src = mine ? __ffsll((long long)mine) - 1 : lane;
-            const float cd = __shfl(d, src);
+            const float cd = bitsf((uint32_t)__shfl((int)fbits(d), src));
             const int cn = __shfl(n, src);
             const float pd = bitsf((uint32_t)lane_before((int)fbits(sd[S - 1])));
             const int pn = lane_before(sn[S - 1]);
@@ -668,7 +668,7 @@ __global__ __launch_bounds__(64) void k_knn_team(KnnArgs a) {
             float kd = sd[0];
 #pragma unroll
             for (int i = 1; i < S; ++i) kd = i == kslot ? sd[i] : kd;
-            kd = __shfl(kd, klane);
+            kd = bitsf((uint32_t)__shfl((int)fbits(kd), klane));
             if (mine) lim = fminf_raw(c.thr, kd);
             cand = cand && lane != src && d <= lim;
             cm = __ballot(cand);
