@@ -308,7 +308,7 @@ enum Buf {
     B_PFLAG, B_PSCAN, B_ISEG, B_ISEGD, B_IO0, B_IO1, B_IO2, B_IO3, B_IO4, B_VSTART, B_DELBOX, B_DELFL, B_INSPT,
     B_INSFL, B_CBOX, B_CPTS, B_MORTK, B_MORTV, B_MORTK2, B_MORTV2, B_CNT64, B_OFF64, B_ADDX, B_ADDI, B_PNEXT, B_SPAIRS, B_SPSCAN,
     B_DEFER, B_DINFO, B_DBEFORE, B_DKEEP, B_PTS3, B_PEND, B_START, B_INV0, B_LASTP, B_PSEED, B_DBELOW, B_MAXDEL,
-    B_SLISTS, B_ENUMROOT, B_ENUMGRP, B_TOPT, B_TOPI, B_TCNT64, B_TOFF64, B_RTASKS, B_ICNT64, B_EMPTYL, B_RAW, B_COUNT
+    B_SLISTS, B_ENUMROOT, B_ENUMGRP, B_TOPT, B_TOPI, B_TCNT64, B_TOFF64, B_RTASKS, B_ICNT64, B_EMPTYL, B_RAW, B_SORTK, B_SORTV, B_COUNT
 };
 static_assert(B_COUNT <= 96, "scratch table");
 
@@ -512,9 +512,19 @@ int prim_tmp(Owner* t, size_t bytes, void** out) {
     return IKD_OK;
 }
 
+// kout, vout: the keys ascending and their indices (vin[i] = i), equal keys in input order.
 int sort_pairs(ikd_tree_t t, const unsigned long long* kin, unsigned long long* kout, const uint32_t* vin,
                uint32_t* vout, int n, int end_bit) {
     if (n <= 0) return IKD_OK;
+    if (n <= RANK_SORT_MAX) {
+        unsigned long long* tk;
+        uint32_t* tv;
+        CHK(ensure(t, B_SORTK, n, &tk));
+        CHK(ensure(t, B_SORTV, n, &tv));
+        launch_rank_sort(kin, n, tk, tv, kout, vout, t->st);
+        HIPCHK(hipGetLastError());
+        return IKD_OK;
+    }
     size_t bytes = 0;
     HIPCHK(prim_sort_pairs_u64(nullptr, bytes, kin, kout, vin, vout, n, 0, end_bit, t->st));
     void* tmp;
@@ -731,8 +741,15 @@ int run_build(ikd_tree_t t, const float4* pts, const int* seg_of, int m, const i
     CHK(ensure(t, B_POSFL, 3ll * m, &posfl));
     CHK(ensure(t, B_POSSC, 3ll * m, &possc));
 
-    int end_bit = 32 + bits_for(S);
-    for (int a = 0; a < 3; ++a) {
+    const int end_bit = 32 + bits_for(S);
+    if (m <= RANK_SORT_MAX) {
+        unsigned long long* tk;
+        uint32_t* tv;
+        CHK(ensure(t, B_SORTK, 3ll * m, &tk));
+        CHK(ensure(t, B_SORTV, 3ll * m, &tv));
+        launch_build_sort3(pts, seg_of, m, tk, tv, perm[0], sid[0], st);
+    }
+    for (int a = 0; m > RANK_SORT_MAX && a < 3; ++a) {
         launch_build_keys(pts, seg_of, m, a, keya, vala, st);
         CHK(sort_pairs(t, keya, keyb, vala, perm[0][a], m, end_bit));
         if (a == 0) launch_build_init_sid(keyb, m, sid[0], st);

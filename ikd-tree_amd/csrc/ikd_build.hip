@@ -39,6 +39,238 @@ __global__ void k_build_init_sid(const unsigned long long* __restrict__ k0, int 
     sid[i] = (int)(k0[i] >> 32);
 }
 
+// ---- stable sort of up to RANK_SORT_MAX keys in two launches ---------------
+// Tiles of 2048 keys are sorted in registers (bitonic network over (key,
+// index), so the order is stable), then every key finds its final place in one
+// pass: its place in its own tile plus, for every other tile, how many of that
+// tile's keys come before it (equal keys of earlier tiles do).  A workgroup's
+// 256 keys are neighbours in their tile's order, so they search one short
+// stretch of every other tile, found once per workgroup.  Several lists of
+// the same length are sorted by the same two launches (grid y).
+//
+// At these sizes a sort is a chain of dependent launches: the library's merge
+// sort takes one per doubling (29k keys: 8 launches, about 75 us with their
+// gaps; here 18 + 33 us for three lists at once), and the build ran three of
+// them behind one another.  The searches grow with the square of the length, so
+// longer lists go to the library: a Build of 30k points takes 383 us for 452,
+// one of 65536 459 for 516.
+constexpr int TILE_SB = 512, TILE_E = 4, TILE_KEYS = TILE_SB * TILE_E;
+constexpr int MERGE_SB = 256;
+static_assert(RANK_SORT_MAX % TILE_KEYS == 0 && TILE_KEYS % MERGE_SB == 0, "whole tiles");
+
+// lane ^ M's value; the exchanges inside 16 lanes are register moves
+template <int M>
+__device__ __forceinline__ int lane_xor(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (M == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true);   // quad_perm 1,0,3,2
+    if constexpr (M == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true);   // quad_perm 2,3,0,1
+    if constexpr (M == 4)  // row_half_mirror is ^ 7, quad_perm 3,2,1,0 is ^ 3
+        return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, true), 0x1B, 0xf, 0xf, true);
+    if constexpr (M == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xf, 0xf, true);  // row_ror:8
+#endif
+    return __shfl_xor(v, M);
+}
+__device__ __forceinline__ bool pair_less(unsigned long long ka, uint32_t va, unsigned long long kb, uint32_t vb) {
+    return ka < kb || (ka == kb && va < vb);
+}
+
+// One stage of the network: every entry and its partner (index ^ J) are put in
+// order, ascending where the bit KK of the index is clear.  Entry 4 t + e is
+// in k[e], v[e] of thread t: partners are in the thread's registers (J < 4),
+// in its wavefront (J < 256), or exchanged through LDS.
+template <int KK, int J>
+__device__ __forceinline__ void sort_stage(unsigned long long (&k)[TILE_E], uint32_t (&v)[TILE_E],
+                                           unsigned long long* xk, uint32_t* xv) {
+    const int t = threadIdx.x;
+    if constexpr (J < TILE_E) {
+#pragma unroll
+        for (int e = 0; e < TILE_E; ++e) {
+            if (e & J) continue;
+            const bool up = (((TILE_E * t + e) & KK) == 0);
+            if (pair_less(k[e | J], v[e | J], k[e], v[e]) == up) {
+                const unsigned long long tk = k[e];
+                const uint32_t tv = v[e];
+                k[e] = k[e | J];
+                v[e] = v[e | J];
+                k[e | J] = tk;
+                v[e | J] = tv;
+            }
+        }
+    } else {
+        unsigned long long ok[TILE_E];
+        uint32_t ov[TILE_E];
+        if constexpr (J < 64 * TILE_E) {
+#pragma unroll
+            for (int e = 0; e < TILE_E; ++e) {
+                const unsigned lo = (unsigned)lane_xor<J / TILE_E>((int)(unsigned)k[e]);
+                const unsigned hi = (unsigned)lane_xor<J / TILE_E>((int)(unsigned)(k[e] >> 32));
+                ok[e] = ((unsigned long long)hi << 32) | lo;
+                ov[e] = (uint32_t)lane_xor<J / TILE_E>((int)v[e]);
+            }
+        } else {
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < TILE_E; ++e) {
+                xk[e * TILE_SB + t] = k[e];
+                xv[e * TILE_SB + t] = v[e];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < TILE_E; ++e) {
+                ok[e] = xk[e * TILE_SB + (t ^ (J / TILE_E))];
+                ov[e] = xv[e * TILE_SB + (t ^ (J / TILE_E))];
+            }
+        }
+        const bool keep_min = ((TILE_E * t) & J) == 0 ? ((TILE_E * t) & KK) == 0 : ((TILE_E * t) & KK) != 0;
+#pragma unroll
+        for (int e = 0; e < TILE_E; ++e) {
+            if (pair_less(ok[e], ov[e], k[e], v[e]) == keep_min) {
+                k[e] = ok[e];
+                v[e] = ov[e];
+            }
+        }
+    }
+}
+template <int KK, int J>
+__device__ __forceinline__ void sort_stages(unsigned long long (&k)[TILE_E], uint32_t (&v)[TILE_E],
+                                            unsigned long long* xk, uint32_t* xv) {
+    sort_stage<KK, J>(k, v, xk, xv);
+    if constexpr (J > 1) sort_stages<KK, J / 2>(k, v, xk, xv);
+    else if constexpr (KK < TILE_KEYS) sort_stages<2 * KK, KK>(k, v, xk, xv);
+}
+
+// keys: the list itself, or null for the build's keys (segment, coordinate of
+// axis blockIdx.y).  okey, oval: lists of n entries one behind the other.
+__global__ __launch_bounds__(TILE_SB) void k_tile_sort(const unsigned long long* __restrict__ keys,
+                                                       const float4* __restrict__ pts,
+                                                       const int* __restrict__ seg_of, int n,
+                                                       unsigned long long* __restrict__ okey,
+                                                       uint32_t* __restrict__ oval) {
+    __shared__ unsigned long long xk[TILE_KEYS];
+    __shared__ uint32_t xv[TILE_KEYS];
+    const int axis = blockIdx.y, first = blockIdx.x * TILE_KEYS + TILE_E * (int)threadIdx.x;
+    unsigned long long k[TILE_E];
+    uint32_t v[TILE_E];
+#pragma unroll
+    for (int e = 0; e < TILE_E; ++e) {
+        const int i = first + e;
+        v[e] = (uint32_t)i;
+        k[e] = ~0ull;  // padding ranks last
+        if (i < n) {
+            if (keys) {
+                k[e] = keys[i];
+            } else {
+                const float4 p = pts[i];
+                k[e] = ((unsigned long long)(uint32_t)seg_of[i] << 32) |
+                       float_key(axis == 0 ? p.x : (axis == 1 ? p.y : p.z));
+            }
+        }
+    }
+    sort_stages<2, 1>(k, v, xk, xv);
+    const size_t off = (size_t)blockIdx.y * n;
+#pragma unroll
+    for (int e = 0; e < TILE_E; ++e) {
+        if (first + e < n) {
+            okey[off + first + e] = k[e];
+            oval[off + first + e] = v[e];
+        }
+    }
+}
+
+// The number of keys below k in the ascending key[lo, hi), plus lo.
+__device__ __forceinline__ int key_bound(const unsigned long long* __restrict__ key, int lo, int hi,
+                                         unsigned long long k) {
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (key[mid] < k) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// val_out[l]: list l's order; key_out (nullable): the sorted keys of list 0;
+// seg_out (nullable): their upper halves.
+struct RankOut {
+    uint32_t* val[3];
+    unsigned long long* key;
+    int* seg;
+};
+__global__ __launch_bounds__(MERGE_SB) void k_rank_merge(const unsigned long long* __restrict__ keys,
+                                                        const uint32_t* __restrict__ vals, int n, RankOut out) {
+    constexpr int TILES = RANK_SORT_MAX / TILE_KEYS;
+    static_assert(2 * TILES <= MERGE_SB, "two searches per tile");
+    __shared__ int lo[TILES], hi[TILES];
+    const size_t off = (size_t)blockIdx.y * n;
+    const unsigned long long* __restrict__ key = keys + off;
+    const int t = threadIdx.x, first = blockIdx.x * MERGE_SB, last = min(first + MERGE_SB, n) - 1;
+    const int tiles = (n + TILE_KEYS - 1) / TILE_KEYS, own = first / TILE_KEYS;
+    if (t < 2 * tiles) {
+        const int q = t >> 1, a = q * TILE_KEYS, b = min(a + TILE_KEYS, n);
+        // keys are below 2^64 - 1: k + 1 does not wrap
+        const int at = q == own ? a : key_bound(key, a, b, (t & 1) ? key[last] + 1 : key[first]);
+        if (t & 1) hi[q] = at;
+        else lo[q] = at;
+    }
+    __syncthreads();
+    const int i = first + t;
+    if (i > last) return;
+    const unsigned long long k = key[i];
+    int rank = i - own * TILE_KEYS;
+    // four tiles at a time (their searches do not wait for each other; eight measured 21 us for 18)
+    constexpr int W = 4;
+    for (int j = 0; j < tiles; j += W) {
+        int at[W], len[W], any = 0;
+        unsigned long long kj[W];
+#pragma unroll
+        for (int u = 0; u < W; ++u) {
+            const int q = min(j + u, tiles - 1);
+            const bool use = j + u < tiles && q != own;
+            at[u] = use ? lo[q] : q * TILE_KEYS;
+            len[u] = use ? hi[q] - lo[q] : 0;
+            kj[u] = k + (q < own ? 1 : 0);  // an earlier tile's equal keys come first
+            rank -= q * TILE_KEYS;
+            any |= len[u];
+        }
+        while (any != 0) {
+            any = 0;
+#pragma unroll
+            for (int u = 0; u < W; ++u) {
+                const int half = len[u] >> 1;
+                const bool below = len[u] > 0 && key[at[u] + half] < kj[u];
+                at[u] = below ? at[u] + half + 1 : at[u];
+                len[u] = below ? len[u] - half - 1 : half;
+                any |= len[u];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < W; ++u) rank += at[u];
+    }
+    out.val[blockIdx.y][rank] = vals[off + i];
+    if (blockIdx.y == 0) {
+        if (out.key) out.key[rank] = k;
+        if (out.seg) out.seg[rank] = (int)(k >> 32);
+    }
+}
+
+static inline int tiles_for(int n, int per) { return (n + per - 1) / per; }
+
+void launch_rank_sort(const unsigned long long* keys, int n, unsigned long long* tmp_key, uint32_t* tmp_val,
+                      unsigned long long* key_out, uint32_t* val_out, hipStream_t s) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_tile_sort, dim3(tiles_for(n, TILE_KEYS)), dim3(TILE_SB), 0, s, keys, (const float4*)nullptr,
+                       (const int*)nullptr, n, tmp_key, tmp_val);
+    RankOut out{{val_out, nullptr, nullptr}, key_out, nullptr};
+    hipLaunchKernelGGL(k_rank_merge, dim3(tiles_for(n, MERGE_SB)), dim3(MERGE_SB), 0, s, tmp_key, tmp_val, n, out);
+}
+void launch_build_sort3(const float4* pts, const int* seg_of, int n, unsigned long long* tmp_key, uint32_t* tmp_val,
+                        uint32_t* const (&perm)[3], int* sid, hipStream_t s) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_tile_sort, dim3(tiles_for(n, TILE_KEYS), 3), dim3(TILE_SB), 0, s,
+                       (const unsigned long long*)nullptr, pts, seg_of, n, tmp_key, tmp_val);
+    RankOut out{{perm[0], perm[1], perm[2]}, nullptr, sid};
+    hipLaunchKernelGGL(k_rank_merge, dim3(tiles_for(n, MERGE_SB), 3), dim3(MERGE_SB), 0, s, tmp_key, tmp_val, n, out);
+}
+
 __device__ __forceinline__ float coord_of(float4 p, int a) { return a == 0 ? p.x : (a == 1 ? p.y : p.z); }
 
 // Per segment: longest axis, mid, and what it allocates (one pair if it has a

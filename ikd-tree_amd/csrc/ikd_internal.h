@@ -83,6 +83,15 @@ struct BuildLevel {
 void launch_build_keys(const float4* pts, const int* seg_of, int m, int axis, unsigned long long* keys,
                        uint32_t* vals, hipStream_t s);
 void launch_build_init_sid(const unsigned long long* sorted_keys0, int m, int* sid, hipStream_t s);
+// Stable sorts of lists of at most RANK_SORT_MAX keys below 2^64 - 1, in two
+// launches (tmp_key, tmp_val: scratch as long as all lists together): the
+// order of `keys`, and the three lists of the build (by segment and coordinate)
+// with the segment of every position of the first.
+constexpr int RANK_SORT_MAX = 1 << 16;
+void launch_rank_sort(const unsigned long long* keys, int n, unsigned long long* tmp_key, uint32_t* tmp_val,
+                      unsigned long long* key_out, uint32_t* val_out, hipStream_t s);
+void launch_build_sort3(const float4* pts, const int* seg_of, int n, unsigned long long* tmp_key, uint32_t* tmp_val,
+                        uint32_t* const (&perm)[3], int* sid, hipStream_t s);
 void launch_build_seg_a(const BuildLevel& L, int bound, DevHdr* hdr, hipStream_t s);
 void launch_build_seg_b(const BuildLevel& L, int bound, Pool pool, DevHdr* hdr, hipStream_t s);
 void launch_build_side(const BuildLevel& L, DevHdr* hdr, hipStream_t s);
