@@ -685,6 +685,27 @@ int reset_pool(ikd_tree_t t) {
     return IKD_OK;
 }
 
+// Builds the S segments (count_dev: how many of them are live, or null), each of
+// at most SMALL_MAX points.
+int build_small(ikd_tree_t t, const float4* pts, const int4* seg, const int* seg_depth, int S, const int* count_dev,
+                const uint32_t* orig, const SmallLists& pre) {
+    int *pscan, *lists;
+    CHK(ensure(t, B_SPSCAN, S, &pscan));
+    CHK(ensure(t, B_SLISTS, 2ll * S, &lists));
+    if (small_plan_fits(S)) {
+        launch_small_plan(seg, S, count_dev, orig, pre, pscan, lists, t->d_hdr, t->st);
+    } else {
+        int* pairs;
+        CHK(ensure(t, B_SPAIRS, S, &pairs));
+        launch_small_pairs(seg, S, count_dev, orig, pre, pairs, lists, t->d_hdr, t->st);
+        CHK(exscan_i32(t, pairs, pscan, S));
+        launch_small_commit(pairs, pscan, S, t->d_hdr, t->st);
+    }
+    launch_build_small(pts, seg, seg_depth, pscan, S, count_dev, orig, pre, lists, t->pool, t->d_hdr, t->st);
+    HIPCHK(hipGetLastError());
+    return IKD_OK;
+}
+
 // -------------------------------------------------------------- the build
 // Builds S subtrees at once.  pts: m points grouped by segment (segment g at
 // positions [seg[g].x, seg[g].y]); seg_of: segment of each point; seg /
@@ -696,17 +717,7 @@ int run_build(ikd_tree_t t, const float4* pts, const int* seg_of, int m, const i
     hipStream_t st = t->st;
     if (maxlen <= SMALL_MAX && t->small_build) {
         // every subtree fits one workgroup: one launch builds them all
-        int *pairs, *pscan, *lists;
-        CHK(ensure(t, B_SPAIRS, S, &pairs));
-        CHK(ensure(t, B_SPSCAN, S, &pscan));
-        CHK(ensure(t, B_SLISTS, 2ll * S, &lists));
-        launch_small_pairs(d_seg, S, nullptr, pairs, t->d_hdr, st);
-        CHK(exscan_i32(t, pairs, pscan, S));
-        launch_build_small(pts, d_seg, d_seg_depth, pscan, S, nullptr, nullptr, SmallLists{}, lists, t->pool,
-                           t->d_hdr, st);
-        launch_small_commit(pairs, pscan, S, t->d_hdr, st);
-        HIPCHK(hipGetLastError());
-        return IKD_OK;
+        return build_small(t, pts, d_seg, d_seg_depth, S, nullptr, nullptr, SmallLists{});
     }
     unsigned long long *keya, *keyb;
     uint32_t* vala;
@@ -806,25 +817,17 @@ int run_build(ikd_tree_t t, const float4* pts, const int* seg_of, int m, const i
         const int cur = Ls & 1;
         const int bound = (int)std::min<long long>((long long)S << std::min(Ls, 30), m);
         float4* gpts;
-        int *pairs, *pscan, *lists;
         CHK(ensure(t, B_PTS3, m, &gpts));
-        CHK(ensure(t, B_SPAIRS, bound, &pairs));
-        CHK(ensure(t, B_SPSCAN, bound, &pscan));
-        CHK(ensure(t, B_SLISTS, 2ll * bound, &lists));
         int* inv0;
         CHK(ensure(t, B_INV0, m, &inv0));
         launch_gather_list(pts, perm[cur][0], sid[cur], m, gpts, inv0, st);
         const int* count_dev = &t->d_hdr->seg_count[cur];
-        launch_small_pairs(seg[cur], bound, count_dev, pairs, t->d_hdr, st);
-        CHK(exscan_i32(t, pairs, pscan, bound));
         // the level-synchronous lists are already sorted per segment
         SmallLists pre;
         pre.list1 = perm[cur][1];
         pre.list2 = perm[cur][2];
         pre.inv0 = inv0;
-        launch_build_small(gpts, seg[cur], segd[cur], pscan, bound, count_dev, perm[cur][0], pre, lists, t->pool,
-                           t->d_hdr, st);
-        launch_small_commit(pairs, pscan, bound, t->d_hdr, st);
+        CHK(build_small(t, gpts, seg[cur], segd[cur], bound, count_dev, perm[cur][0], pre));
     }
     HIPCHK(hipGetLastError());
     return IKD_OK;

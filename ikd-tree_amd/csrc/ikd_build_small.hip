@@ -19,14 +19,16 @@
 namespace ikd {
 
 // Three shapes: one lane per segment of at most MICRO_MAX points (most insert
-// groups hold one to a few points), a 64-thread workgroup for segments of at
-// most TINY_MAX points, a 256-thread one for the rest up to SMALL_MAX.  The
-// lane kernel also lists the larger segments for the two workgroup kernels,
-// which loop over their list, so no workgroup is launched only to find its
-// segment belongs to the other shape.
+// groups hold one to a few points), one wavefront per segment of at most
+// TINY_MAX points, one workgroup for the rest up to SMALL_MAX.  The plan lists
+// the segments of the two larger shapes, and one launch builds all three side
+// by side: each is a chain of LDS and gather latencies that leaves the device
+// almost idle, and one behind the other they took 25 + 38 + 47 us twice per
+// mapped scan (now 69 together, at 20 scans 18.2 -> 16.5 ms).
 constexpr int MICRO_MAX = 8;
 constexpr int TINY_MAX = 128;
-constexpr int SMALL_SB = 256;  // threads of the workgroup build of segments above TINY_MAX points
+constexpr int SMALL_SB = 256;  // threads of a workgroup
+constexpr int TINY_WAVES = SMALL_SB / 64;
 
 // Nodes with at least one child in the median-split tree of m points.  A node
 // of size x >= 2 leaves children of sizes (x-1)>>1 and x-1-((x-1)>>1), so a
@@ -58,24 +60,68 @@ __device__ int median_tree_pairs(int m) {
     return (int)internal;
 }
 
-// count_dev (optional) holds the number of live segments among the S slots;
-// slots past it take no pairs.
-__global__ void k_small_pairs(const int4* __restrict__ seg, int S, const int* __restrict__ count_dev,
-                              int* __restrict__ pairs, DevHdr* hdr) {
-    int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g == 0) {  // the size-class lists of this build start empty
-        hdr->small_lists[0] = 0;
-        hdr->small_lists[1] = 0;
+// Pairs of segment g, and its entry in the list of its shape.
+__device__ __forceinline__ int plan_segment(const int4* __restrict__ seg, int g, int S, int micro,
+                                            int* __restrict__ lists, DevHdr* hdr) {
+    const int m = seg[g].y - seg[g].x + 1;
+    if (m <= 0) return 0;
+    if (!micro || m > MICRO_MAX) {
+        if (m <= TINY_MAX) lists[atomicAdd(&hdr->small_lists[0], 1)] = g;
+        else lists[S + atomicAdd(&hdr->small_lists[1], 1)] = g;
     }
+    return median_tree_pairs(m);
+}
+
+// count_dev (optional) holds the number of live segments among the S slots;
+// slots past it take no pairs.  k_small_plan: one workgroup, for up to PLAN_MAX
+// segments; pair_scan gets every segment's first pair relative to the pairs this
+// build takes, which begin at hdr->pair_base.
+constexpr int PLAN_MAX = 8192;
+__global__ __launch_bounds__(1024) void k_small_plan(const int4* __restrict__ seg, int S,
+                                                     const int* __restrict__ count_dev, int micro,
+                                                     int* __restrict__ pair_scan, int* __restrict__ lists,
+                                                     DevHdr* hdr) {
+    __shared__ int wave_tot[16];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int count = min(count_dev ? *count_dev : S, S);
+    const int chunk = (S + 1023) >> 10;
+    const int b = min(t * chunk, S), e = min(b + chunk, S);
+    if (t < 2) hdr->small_lists[t] = 0;
+    __syncthreads();
+    int sum = 0;
+    for (int g = b; g < e; ++g) {
+        const int p = g < count ? plan_segment(seg, g, S, micro, lists, hdr) : 0;
+        pair_scan[g] = sum;  // within the thread's run for now
+        sum += p;
+    }
+    int inc = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl(inc, (lane - d) & 63);  // lanes below d ignore what they read
+        if (lane >= d) inc += o;
+    }
+    if (lane == 63) wave_tot[w] = inc;
+    __syncthreads();
+    int run = inc - sum;
+    for (int i = 0; i < w; ++i) run += wave_tot[i];
+    for (int g = b; g < e; ++g) pair_scan[g] += run;
+    if (t == 1023) {
+        hdr->pair_base = hdr->pair_used;
+        hdr->pair_used += run + sum;
+    }
+}
+
+__global__ void k_small_pairs(const int4* __restrict__ seg, int S, const int* __restrict__ count_dev, int micro,
+                              int* __restrict__ pairs, int* __restrict__ lists, DevHdr* hdr) {
+    int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= S) return;
     const int count = count_dev ? *count_dev : S;
-    pairs[g] = g < count ? median_tree_pairs(seg[g].y - seg[g].x + 1) : 0;
+    pairs[g] = g < count ? plan_segment(seg, g, S, micro, lists, hdr) : 0;
 }
-
 __global__ void k_small_commit(const int* __restrict__ pairs, const int* __restrict__ scan, int S, DevHdr* hdr) {
+    hdr->pair_base = hdr->pair_used;
     hdr->pair_used += scan[S - 1] + pairs[S - 1];
 }
-
 __device__ __forceinline__ void write_child_box_s(NodeHot* hot, int parent, int side, const float* b) {
     float* f = hot[parent].f;
     if (side == 0) {
@@ -87,14 +133,30 @@ __device__ __forceinline__ void write_child_box_s(NodeHot* hot, int parent, int 
     }
 }
 
-// Exclusive scan of one 64-bit value per thread across the workgroup
+// A build by SB threads: a wavefront of its own (SB = 64; the workgroup's other
+// wavefronts build other segments) or a whole workgroup.
+template <int SB>
+__device__ __forceinline__ int build_thread() {
+    return SB == 64 ? (int)(threadIdx.x & 63u) : (int)threadIdx.x;
+}
+template <int SB>
+__device__ __forceinline__ void build_sync() {
+    if (SB == 64) {
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+
+// Exclusive scan of one 64-bit value per thread across the building threads
 // (*total gets the sum): an inclusive scan inside each wavefront by
 // shuffles, then the wavefront totals through LDS (two barriers).  Several
 // small counters can ride in one value as bit fields that never overflow.
 template <int SB>
 __device__ unsigned long long block_exscan_u64(unsigned long long v, unsigned long long* wtot,
                                                unsigned long long* total) {
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int t = build_thread<SB>(), lane = t & 63, w = t >> 6;
     unsigned long long x = v;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -105,7 +167,7 @@ __device__ unsigned long long block_exscan_u64(unsigned long long v, unsigned lo
         if (lane >= off) x += y;
     }
     if (lane == 63) wtot[w] = x;
-    __syncthreads();
+    build_sync<SB>();
     unsigned long long base = 0, tot = 0;
 #pragma unroll
     for (int i = 0; i < SB / 64; ++i) {
@@ -113,7 +175,7 @@ __device__ unsigned long long block_exscan_u64(unsigned long long v, unsigned lo
         tot += wtot[i];
     }
     *total = tot;
-    __syncthreads();
+    build_sync<SB>();
     return base + x - v;
 }
 
@@ -124,7 +186,7 @@ __device__ unsigned long long block_exscan_u64(unsigned long long v, unsigned lo
 // LDS (xch, SB * E entries).  Keys must be distinct.
 template <int SB, int E>
 __device__ void reg_bitonic(unsigned long long (&x)[E], int P, unsigned long long* xch) {
-    const int t = threadIdx.x;
+    const int t = build_thread<SB>();
     for (int k = 2; k <= P; k <<= 1) {
         for (int j = k >> 1; j > 0; j >>= 1) {
             if (j >= SB) {
@@ -141,10 +203,10 @@ __device__ void reg_bitonic(unsigned long long (&x)[E], int P, unsigned long lon
                     }
                 }
             } else if (j >= 64) {
-                __syncthreads();
+                build_sync<SB>();
 #pragma unroll
                 for (int e = 0; e < E; ++e) xch[e * SB + t] = x[e];
-                __syncthreads();
+                build_sync<SB>();
 #pragma unroll
                 for (int e = 0; e < E; ++e) {
                     const int i = e * SB + t;
@@ -165,50 +227,48 @@ __device__ void reg_bitonic(unsigned long long (&x)[E], int P, unsigned long lon
             }
         }
     }
-    __syncthreads();  // xch may be reused at once
+    build_sync<SB>();  // xch may be reused at once
 }
 
 // orig (optional) gives each point's index in the caller's original input:
 // equal coordinates are then ordered by it, as the global build's stable
 // presorted lists order them; without it, by position in the segment.
 template <int SB, int SMAX>
-__global__ __launch_bounds__(SB) void k_build_small(const float4* __restrict__ pts, const int4* __restrict__ seg,
-                                                     const int* __restrict__ seg_depth,
-                                                     const int* __restrict__ pair_scan,
-                                                     const int* __restrict__ list,
-                                                     const int* __restrict__ list_count,
-                                                     const uint32_t* __restrict__ orig, SmallLists pre, Pool pool,
-                                                     DevHdr* hdr) {
-    constexpr int SMAX_SEG = SMAX / 2 + 1;
-    __shared__ float px[SMAX], py[SMAX], pz[SMAX];
-    __shared__ unsigned long long skey[SMAX];  // sort keys, then running counts
-    __shared__ unsigned short lst[2][3][SMAX];
-    __shared__ short sid[2][SMAX];
-    __shared__ unsigned char side[SMAX];
-    __shared__ short seg_l[2][SMAX_SEG], seg_r[2][SMAX_SEG];
-    __shared__ int seg_node[2][SMAX_SEG], seg_par[2][SMAX_SEG];
-    __shared__ unsigned char seg_axis[SMAX_SEG];
-    __shared__ short seg_mid[SMAX_SEG], seg_cl[SMAX_SEG], seg_cr[SMAX_SEG];
-    __shared__ unsigned long long wtot[SB / 64];
-    __shared__ unsigned short rnk[SMAX];
+struct BuildLds {
+    static constexpr int SEGS = SMAX / 2 + 1;
+    unsigned long long skey[SMAX];  // sort keys, then running counts
+    unsigned long long wtot[SB / 64];
+    float px[SMAX], py[SMAX], pz[SMAX];
+    int seg_node[2][SEGS], seg_par[2][SEGS];
+    unsigned short lst[2][3][SMAX];
+    unsigned short rnk[SMAX];
+    short sid[2][SMAX];
+    short seg_l[2][SEGS], seg_r[2][SEGS];
+    short seg_mid[SEGS], seg_cl[SEGS], seg_cr[SEGS];
+    unsigned char side[SMAX];
+    unsigned char seg_axis[SEGS];
+};
 
-    const int t = threadIdx.x;
-    const int nlist = *list_count;
-    for (int li = blockIdx.x; li < nlist; li += gridDim.x) {
-    const int g = list[li];
+// Segment g by SB threads.
+template <int SB, int SMAX>
+__device__ void build_segment(BuildLds<SB, SMAX>& L, int g, const float4* __restrict__ pts,
+                              const int4* __restrict__ seg, const int* __restrict__ seg_depth,
+                              const int* __restrict__ pair_scan, const uint32_t* __restrict__ orig,
+                              const SmallLists& pre, const Pool& pool, DevHdr* hdr) {
+    const int t = build_thread<SB>();
     const int4 sg = seg[g];
     const int l0 = sg.x;
     const int m = sg.y - sg.x + 1;
     // the list holds this shape's size class; the host guarantees m <= SMALL_MAX
-    if (m <= 0 || m > SMAX) continue;
+    if (m <= 0 || m > SMAX) return;
     const int depth0 = seg_depth[g];
-    int next_pair = hdr->pair_used + pair_scan[g];
+    int next_pair = hdr->pair_base + pair_scan[g];
 
     for (int i = t; i < m; i += SB) {
         float4 p = pts[l0 + i];
-        px[i] = p.x;
-        py[i] = p.y;
-        pz[i] = p.z;
+        L.px[i] = p.x;
+        L.py[i] = p.y;
+        L.pz[i] = p.z;
     }
     int P = 1;
     while (P < m) P <<= 1;
@@ -216,9 +276,9 @@ __global__ __launch_bounds__(SB) void k_build_small(const float4* __restrict__ p
         // the caller's lists are already sorted (coordinate, original index)
         // per segment, and the points were gathered in x order
         for (int i = t; i < m; i += SB) {
-            lst[0][0][i] = (unsigned short)i;
-            lst[0][1][i] = (unsigned short)(pre.inv0[pre.list1[l0 + i]] - l0);
-            lst[0][2][i] = (unsigned short)(pre.inv0[pre.list2[l0 + i]] - l0);
+            L.lst[0][0][i] = (unsigned short)i;
+            L.lst[0][1][i] = (unsigned short)(pre.inv0[pre.list1[l0 + i]] - l0);
+            L.lst[0][2][i] = (unsigned short)(pre.inv0[pre.list2[l0 + i]] - l0);
         }
     } else {
     // tie-break rank of every point: its order by original index, or its position
@@ -230,43 +290,43 @@ __global__ __launch_bounds__(SB) void k_build_small(const float4* __restrict__ p
             const int i = e * SB + t;
             x[e] = i < m ? (((unsigned long long)orig[l0 + i] << 16) | (unsigned)i) : ~0ull;
         }
-        reg_bitonic<SB, E>(x, P, skey);
+        reg_bitonic<SB, E>(x, P, L.skey);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int i = e * SB + t;
-            if (i < m) rnk[x[e] & 0xffffu] = (unsigned short)i;
+            if (i < m) L.rnk[x[e] & 0xffffu] = (unsigned short)i;
         }
     } else {
-        for (int i = t; i < m; i += SB) rnk[i] = (unsigned short)i;
+        for (int i = t; i < m; i += SB) L.rnk[i] = (unsigned short)i;
     }
-    __syncthreads();
+    build_sync<SB>();
     // three stable sorted index lists: key (coordinate, rank, position)
     for (int a = 0; a < 3; ++a) {
-        const float* c = a == 0 ? px : (a == 1 ? py : pz);
+        const float* c = a == 0 ? L.px : (a == 1 ? L.py : L.pz);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int i = e * SB + t;
-            x[e] = i < m ? (((unsigned long long)float_key(c[i]) << 32) | ((unsigned)rnk[i] << 16) | (unsigned)i)
+            x[e] = i < m ? (((unsigned long long)float_key(c[i]) << 32) | ((unsigned)L.rnk[i] << 16) | (unsigned)i)
                          : ~0ull;
         }
-        reg_bitonic<SB, E>(x, P, skey);
+        reg_bitonic<SB, E>(x, P, L.skey);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int i = e * SB + t;
-            if (i < m) lst[0][a][i] = (unsigned short)(x[e] & 0xffffu);
+            if (i < m) L.lst[0][a][i] = (unsigned short)(x[e] & 0xffffu);
         }
     }
-    __syncthreads();
+    build_sync<SB>();
     }
-    for (int i = t; i < m; i += SB) sid[0][i] = 0;
+    for (int i = t; i < m; i += SB) L.sid[0][i] = 0;
     if (t == 0) {
-        seg_l[0][0] = 0;
-        seg_r[0][0] = (short)(m - 1);
-        seg_node[0][0] = sg.z;
-        seg_par[0][0] = sg.w;
+        L.seg_l[0][0] = 0;
+        L.seg_r[0][0] = (short)(m - 1);
+        L.seg_node[0][0] = sg.z;
+        L.seg_par[0][0] = sg.w;
     }
-    __syncthreads();
-    unsigned long long* run = skey;  // the sort keys' space, reused for running counts
+    build_sync<SB>();
+    unsigned long long* run = L.skey;  // the sort keys' space, reused for running counts
     const int chunk = (m + SB - 1) / SB;
     int ns = 1;
     int cur = 0;
@@ -277,34 +337,34 @@ __global__ __launch_bounds__(SB) void k_build_small(const float4* __restrict__ p
         for (int q = 0; q < per; ++q) {
             const int s = t * per + q;
             if (s >= ns) break;
-            const int l = seg_l[cur][s], r = seg_r[cur][s];
+            const int l = L.seg_l[cur][s], r = L.seg_r[cur][s];
             float ext[3];
-            ext[0] = px[lst[cur][0][r]] - px[lst[cur][0][l]];
-            ext[1] = py[lst[cur][1][r]] - py[lst[cur][1][l]];
-            ext[2] = pz[lst[cur][2][r]] - pz[lst[cur][2][l]];
+            ext[0] = L.px[L.lst[cur][0][r]] - L.px[L.lst[cur][0][l]];
+            ext[1] = L.py[L.lst[cur][1][r]] - L.py[L.lst[cur][1][l]];
+            ext[2] = L.pz[L.lst[cur][2][r]] - L.pz[L.lst[cur][2][l]];
             int axis = 0;
             if (ext[1] > ext[axis]) axis = 1;
             if (ext[2] > ext[axis]) axis = 2;
             const int mid = (l + r) >> 1;
-            seg_axis[s] = (unsigned char)axis;
-            seg_mid[s] = (short)mid;
+            L.seg_axis[s] = (unsigned char)axis;
+            L.seg_mid[s] = (short)mid;
             const int hl = mid > l, hr = mid < r;
             my_pairs += (hl || hr) ? 1 : 0;
             my_children += hl + hr;
         }
         unsigned long long tot2;
         const unsigned long long off2 =
-            block_exscan_u64<SB>((unsigned long long)my_pairs | ((unsigned long long)my_children << 32), wtot, &tot2);
+            block_exscan_u64<SB>((unsigned long long)my_pairs | ((unsigned long long)my_children << 32), L.wtot, &tot2);
         int pair_off = (int)(unsigned)off2, child_off = (int)(off2 >> 32);
         const int tot_pairs = (int)(unsigned)tot2, tot_children = (int)(tot2 >> 32);
         for (int q = 0; q < per; ++q) {
             const int s = t * per + q;
             if (s >= ns) break;
-            const int l = seg_l[cur][s], r = seg_r[cur][s], mid = seg_mid[s], axis = seg_axis[s];
-            const int node = seg_node[cur][s], parent = seg_par[cur][s];
+            const int l = L.seg_l[cur][s], r = L.seg_r[cur][s], mid = L.seg_mid[s], axis = L.seg_axis[s];
+            const int node = L.seg_node[cur][s], parent = L.seg_par[cur][s];
             const int hl = mid > l, hr = mid < r;
             const int pair = (hl || hr) ? next_pair + pair_off++ : 0;
-            const int piv = lst[cur][axis][mid];
+            const int piv = L.lst[cur][axis][mid];
             const uint32_t link = ((uint32_t)pair << LK_PAIR_SHIFT) | (hl ? LK_HASL : 0u) | (hr ? LK_HASR : 0u);
             const float4 P4 = pts[l0 + piv];
             *reinterpret_cast<float4*>(pool.hot[node].f) = make_float4(P4.x, P4.y, P4.z, bitsf(link));
@@ -312,39 +372,39 @@ __global__ __launch_bounds__(SB) void k_build_small(const float4* __restrict__ p
             pool.par[node] = parent;
             pool.cnt[node] = make_int4(r - l + 1, 0, 0, depth);
             pool.meta[node] = (uint32_t)axis;
-            float box[6] = {px[lst[cur][0][l]], py[lst[cur][1][l]], pz[lst[cur][2][l]],
-                            px[lst[cur][0][r]], py[lst[cur][1][r]], pz[lst[cur][2][r]]};
+            float box[6] = {L.px[L.lst[cur][0][l]], L.py[L.lst[cur][1][l]], L.pz[L.lst[cur][2][l]],
+                            L.px[L.lst[cur][0][r]], L.py[L.lst[cur][1][r]], L.pz[L.lst[cur][2][r]]};
             write_child_box_s(pool.hot, parent, node & 1, box);
             int cl = -1, cr = -1;
             if (hl) {
                 cl = child_off++;
-                seg_l[cur ^ 1][cl] = (short)l;
-                seg_r[cur ^ 1][cl] = (short)(mid - 1);
-                seg_node[cur ^ 1][cl] = 2 * pair;
-                seg_par[cur ^ 1][cl] = node;
+                L.seg_l[cur ^ 1][cl] = (short)l;
+                L.seg_r[cur ^ 1][cl] = (short)(mid - 1);
+                L.seg_node[cur ^ 1][cl] = 2 * pair;
+                L.seg_par[cur ^ 1][cl] = node;
             }
             if (hr) {
                 cr = child_off++;
-                seg_l[cur ^ 1][cr] = (short)(mid + 1);
-                seg_r[cur ^ 1][cr] = (short)r;
-                seg_node[cur ^ 1][cr] = 2 * pair + 1;
-                seg_par[cur ^ 1][cr] = node;
+                L.seg_l[cur ^ 1][cr] = (short)(mid + 1);
+                L.seg_r[cur ^ 1][cr] = (short)r;
+                L.seg_node[cur ^ 1][cr] = 2 * pair + 1;
+                L.seg_par[cur ^ 1][cr] = node;
             }
-            seg_cl[s] = (short)cl;
-            seg_cr[s] = (short)cr;
+            L.seg_cl[s] = (short)cl;
+            L.seg_cr[s] = (short)cr;
         }
         if (t == 0) atomicMax(&hdr->max_depth, depth);
         next_pair += tot_pairs;
-        __syncthreads();
+        build_sync<SB>();
         if (tot_children == 0) break;
         // side of every live position, read off its segment's axis list
         for (int j = t; j < m; j += SB) {
-            const int s = sid[cur][j];
+            const int s = L.sid[cur][j];
             if (s < 0) continue;
-            const int mid = seg_mid[s];
-            side[lst[cur][seg_axis[s]][j]] = (unsigned char)(j < mid ? 0 : (j == mid ? 2 : 1));
+            const int mid = L.seg_mid[s];
+            L.side[L.lst[cur][L.seg_axis[s]][j]] = (unsigned char)(j < mid ? 0 : (j == mid ? 2 : 1));
         }
-        __syncthreads();
+        build_sync<SB>();
         // stable partition of the three lists at once: for every position, the
         // numbers of left and right entries of each list before it, as six
         // 10-bit fields of one value (no field reaches 1024: at most m - 1
@@ -353,57 +413,56 @@ __global__ __launch_bounds__(SB) void k_build_small(const float4* __restrict__ p
         for (int q = 0; q < chunk; ++q) {
             const int j = t * chunk + q;
             if (j >= m) break;
-            if (sid[cur][j] < 0) continue;
+            if (L.sid[cur][j] < 0) continue;
 #pragma unroll
             for (int b = 0; b < 3; ++b) {
-                const unsigned char sd = side[lst[cur][b][j]];
+                const unsigned char sd = L.side[L.lst[cur][b][j]];
                 if (sd < 2) cnt6 += 1ull << (20 * b + 10 * sd);
             }
         }
         unsigned long long tot6;
-        unsigned long long acc = block_exscan_u64<SB>(cnt6, wtot, &tot6);
+        unsigned long long acc = block_exscan_u64<SB>(cnt6, L.wtot, &tot6);
         for (int q = 0; q < chunk; ++q) {
             const int j = t * chunk + q;
             if (j >= m) break;
             run[j] = acc;
-            if (sid[cur][j] < 0) continue;
+            if (L.sid[cur][j] < 0) continue;
 #pragma unroll
             for (int b = 0; b < 3; ++b) {
-                const unsigned char sd = side[lst[cur][b][j]];
+                const unsigned char sd = L.side[L.lst[cur][b][j]];
                 if (sd < 2) acc += 1ull << (20 * b + 10 * sd);
             }
         }
-        __syncthreads();
+        build_sync<SB>();
         for (int b = 0; b < 3; ++b) {
             for (int q = 0; q < chunk; ++q) {
                 const int j = t * chunk + q;
                 if (j >= m) break;
-                const int s = sid[cur][j];
+                const int s = L.sid[cur][j];
                 if (s < 0) {
-                    if (b == 0) sid[cur ^ 1][j] = -1;
+                    if (b == 0) L.sid[cur ^ 1][j] = -1;
                     continue;
                 }
-                const int p = lst[cur][b][j];
-                const unsigned char sd = side[p];
+                const int p = L.lst[cur][b][j];
+                const unsigned char sd = L.side[p];
                 if (sd == 2) {
-                    if (b == 0) sid[cur ^ 1][seg_mid[s]] = -1;
+                    if (b == 0) L.sid[cur ^ 1][L.seg_mid[s]] = -1;
                     continue;
                 }
-                const int l = seg_l[cur][s], mid = seg_mid[s];
+                const int l = L.seg_l[cur][s], mid = L.seg_mid[s];
                 // fields only grow along the list, so the packed difference
                 // subtracts field by field without borrows
                 const int before = (int)(((run[j] - run[l]) >> (20 * b + 10 * sd)) & 1023ull);
                 const int np = sd == 0 ? l + before : mid + 1 + before;
-                lst[cur ^ 1][b][np] = (unsigned short)p;
-                if (b == 0) sid[cur ^ 1][np] = sd == 0 ? seg_cl[s] : seg_cr[s];
+                L.lst[cur ^ 1][b][np] = (unsigned short)p;
+                if (b == 0) L.sid[cur ^ 1][np] = sd == 0 ? L.seg_cl[s] : L.seg_cr[s];
             }
         }
-        __syncthreads();
+        build_sync<SB>();
         ns = tot_children;
         cur ^= 1;
     }
-    __syncthreads();  // the next segment of the list reuses the LDS arrays
-    }
+    build_sync<SB>();  // the next segment of the list reuses the LDS arrays
 }
 
 // One lane builds one segment of at most MICRO_MAX points: the median tree of
@@ -414,44 +473,37 @@ __global__ __launch_bounds__(SB) void k_build_small(const float4* __restrict__ p
 // indexed at run time lives in private memory); pairs are taken from the
 // segment's range one internal node at a time.  Larger segments (or every
 // segment when micro is off) go to the size-class lists.
-constexpr int MICRO_BS = 256;
+constexpr int MICRO_BS = SMALL_SB;
 constexpr int MICRO_STACK = 6;  // pending ranges: at most one per level below the current one
+struct MicroLds {
+    // per lane: (lo | hi << 4 | level << 8), slot node, slot parent
+    int stk_r[MICRO_STACK][MICRO_BS], stk_node[MICRO_STACK][MICRO_BS], stk_par[MICRO_STACK][MICRO_BS];
+};
 __device__ __forceinline__ float micro_coord(const float4& q, int axis) {
     return axis == 0 ? q.x : (axis == 1 ? q.y : q.z);
 }
-__global__ __launch_bounds__(MICRO_BS) void k_build_micro(const float4* __restrict__ pts, const int4* __restrict__ seg,
-                                                          const int* __restrict__ seg_depth,
-                                                          const int* __restrict__ pair_scan, int S,
-                                                          const int* __restrict__ count_dev, int micro, Pool pool,
-                                                          DevHdr* hdr, int* __restrict__ tiny_list,
-                                                          int* __restrict__ small_list) {
-    // per lane: (lo | hi << 4 | level << 8), slot node, slot parent
-    __shared__ int stk_r[MICRO_STACK][MICRO_BS], stk_node[MICRO_STACK][MICRO_BS], stk_par[MICRO_STACK][MICRO_BS];
+__device__ void build_micro(MicroLds& L, int g, const float4* __restrict__ pts, const int4* __restrict__ seg,
+                            const int* __restrict__ seg_depth, const int* __restrict__ pair_scan, int S,
+                            const int* __restrict__ count_dev, const Pool& pool, DevHdr* hdr) {
     const int tid = threadIdx.x;
-    const int g = blockIdx.x * blockDim.x + tid;
     if (g >= S || (count_dev && g >= *count_dev)) return;
     const int4 sg = seg[g];
     const int m = sg.y - sg.x + 1;
-    if (m <= 0) return;
-    if (!micro || m > MICRO_MAX) {
-        if (m <= TINY_MAX) tiny_list[atomicAdd(&hdr->small_lists[0], 1)] = g;
-        else small_list[atomicAdd(&hdr->small_lists[1], 1)] = g;
-        return;
-    }
+    if (m <= 0 || m > MICRO_MAX) return;
     const float4* P = pts + sg.x;
     uint64_t perm = 0x76543210ull;  // nibble i: the position at work-order slot i
-    int next_pair = hdr->pair_used + pair_scan[g];
+    int next_pair = hdr->pair_base + pair_scan[g];
     const int depth0 = seg_depth[g];
     int nw = 1;
-    stk_r[0][tid] = m << 4;
-    stk_node[0][tid] = sg.z;
-    stk_par[0][tid] = sg.w;
+    L.stk_r[0][tid] = m << 4;
+    L.stk_node[0][tid] = sg.z;
+    L.stk_par[0][tid] = sg.w;
     int deepest = depth0;
     while (nw > 0) {
         --nw;
-        const int rr = stk_r[nw][tid];
+        const int rr = L.stk_r[nw][tid];
         const int lo = rr & 15, hi = (rr >> 4) & 15, depth = depth0 + (rr >> 8);
-        const int node = stk_node[nw][tid], parent = stk_par[nw][tid];
+        const int node = L.stk_node[nw][tid], parent = L.stk_par[nw][tid];
         const int cnt = hi - lo;
         // bounds in key order, as the sorted lists give them (-0 below +0)
         const float4 q0 = P[(perm >> (4 * lo)) & 15];
@@ -514,46 +566,86 @@ __global__ __launch_bounds__(MICRO_BS) void k_build_micro(const float4* __restri
         deepest = depth > deepest ? depth : deepest;
         const int lv = (rr >> 8) + 1;
         if (hr) {
-            stk_r[nw][tid] = (lo + nl + 1) | (hi << 4) | (lv << 8);
-            stk_node[nw][tid] = 2 * pair + 1;
-            stk_par[nw][tid] = node;
+            L.stk_r[nw][tid] = (lo + nl + 1) | (hi << 4) | (lv << 8);
+            L.stk_node[nw][tid] = 2 * pair + 1;
+            L.stk_par[nw][tid] = node;
             ++nw;
         }
         if (hl) {
-            stk_r[nw][tid] = lo | ((lo + nl) << 4) | (lv << 8);
-            stk_node[nw][tid] = 2 * pair;
-            stk_par[nw][tid] = node;
+            L.stk_r[nw][tid] = lo | ((lo + nl) << 4) | (lv << 8);
+            L.stk_node[nw][tid] = 2 * pair;
+            L.stk_par[nw][tid] = node;
             ++nw;
         }
     }
     atomicMax(&hdr->max_depth, deepest);
 }
 
+// The three shapes in one launch: the workgroups [0, nb_small) share the list
+// of segments above TINY_MAX points, the wavefronts of the next nb_tiny the list
+// of those above MICRO_MAX, and the lanes of the rest take one segment each.
+__global__ __launch_bounds__(SMALL_SB) void k_build_segments(const float4* __restrict__ pts,
+                                                             const int4* __restrict__ seg,
+                                                             const int* __restrict__ seg_depth,
+                                                             const int* __restrict__ pair_scan, int S,
+                                                             const int* __restrict__ count_dev,
+                                                             const int* __restrict__ lists,
+                                                             const uint32_t* __restrict__ orig, SmallLists pre,
+                                                             Pool pool, DevHdr* hdr, int nb_small, int nb_tiny) {
+    __shared__ union {
+        BuildLds<SMALL_SB, SMALL_MAX> small;
+        BuildLds<64, TINY_MAX> tiny[TINY_WAVES];
+        MicroLds micro;
+    } lds;
+    const int b = blockIdx.x;
+    if (b < nb_small) {
+        const int n = hdr->small_lists[1];
+        for (int i = b; i < n; i += nb_small)
+            build_segment<SMALL_SB, SMALL_MAX>(lds.small, lists[S + i], pts, seg, seg_depth, pair_scan, orig, pre, pool,
+                                               hdr);
+    } else if (b < nb_small + nb_tiny) {
+        const int n = hdr->small_lists[0], w = threadIdx.x >> 6;
+        for (int i = (b - nb_small) * TINY_WAVES + w; i < n; i += nb_tiny * TINY_WAVES)
+            build_segment<64, TINY_MAX>(lds.tiny[w], lists[i], pts, seg, seg_depth, pair_scan, orig, pre, pool, hdr);
+    } else {
+        build_micro(lds.micro, (b - nb_small - nb_tiny) * MICRO_BS + (int)threadIdx.x, pts, seg, seg_depth, pair_scan,
+                    S, count_dev, pool, hdr);
+    }
+}
+
 static inline int blocks_for(long long n, int bs) { return (int)((n + bs - 1) / bs); }
 
-void launch_small_pairs(const int4* seg, int S, const int* count_dev, int* pairs, DevHdr* hdr, hipStream_t s) {
+bool small_plan_fits(int S) { return S <= PLAN_MAX; }
+// the lane build follows the position tie rule only: presorted or
+// original-order inputs go to the larger shapes
+static int micro_ok(const uint32_t* orig, const SmallLists& pre) { return (!orig && !pre.inv0) ? 1 : 0; }
+
+void launch_small_plan(const int4* seg, int S, const int* count_dev, const uint32_t* orig, const SmallLists& pre,
+                       int* pair_scan, int* lists, DevHdr* hdr, hipStream_t s) {
     if (S <= 0) return;
-    hipLaunchKernelGGL(k_small_pairs, dim3(blocks_for(S, 256)), dim3(256), 0, s, seg, S, count_dev, pairs, hdr);
+    hipLaunchKernelGGL(k_small_plan, dim3(1), dim3(1024), 0, s, seg, S, count_dev, micro_ok(orig, pre), pair_scan,
+                       lists, hdr);
 }
-void launch_build_small(const float4* pts, const int4* seg, const int* seg_depth, const int* pair_scan, int S,
-                        const int* count_dev, const uint32_t* orig, SmallLists pre, int* lists, Pool pool,
-                        DevHdr* hdr, hipStream_t s) {
+void launch_small_pairs(const int4* seg, int S, const int* count_dev, const uint32_t* orig, const SmallLists& pre,
+                        int* pairs, int* lists, DevHdr* hdr, hipStream_t s) {
     if (S <= 0) return;
-    // the lane build follows the position tie rule only: presorted or
-    // original-order inputs go to the workgroup builds
-    const int micro = (!orig && !pre.inv0) ? 1 : 0;
-    hipLaunchKernelGGL(k_build_micro, dim3(blocks_for(S, MICRO_BS)), dim3(MICRO_BS), 0, s, pts, seg, seg_depth, pair_scan, S,
-                       count_dev, micro, pool, hdr, lists, lists + S);
-    // each workgroup loops over its shape's list; the grids only need to be
-    // wide enough to fill the device when a list is long
-    hipLaunchKernelGGL((k_build_small<64, TINY_MAX>), dim3(std::min(S, 2048)), dim3(64), 0, s, pts, seg, seg_depth,
-                       pair_scan, lists, &hdr->small_lists[0], orig, pre, pool, hdr);
-    hipLaunchKernelGGL((k_build_small<SMALL_SB, SMALL_MAX>), dim3(std::min(S, 512)), dim3(SMALL_SB), 0, s, pts, seg,
-                       seg_depth, pair_scan, lists + S, &hdr->small_lists[1], orig, pre, pool, hdr);
+    launch_fill_i32(hdr->small_lists, 0, 2, s);
+    hipLaunchKernelGGL(k_small_pairs, dim3(blocks_for(S, 256)), dim3(256), 0, s, seg, S, count_dev, micro_ok(orig, pre),
+                       pairs, lists, hdr);
 }
 void launch_small_commit(const int* pairs, const int* pair_scan, int S, DevHdr* hdr, hipStream_t s) {
     if (S <= 0) return;
     hipLaunchKernelGGL(k_small_commit, dim3(1), dim3(1), 0, s, pairs, pair_scan, S, hdr);
+}
+void launch_build_small(const float4* pts, const int4* seg, const int* seg_depth, const int* pair_scan, int S,
+                        const int* count_dev, const uint32_t* orig, SmallLists pre, const int* lists, Pool pool,
+                        DevHdr* hdr, hipStream_t s) {
+    if (S <= 0) return;
+    // wide enough to fill the device when a list is long
+    const int nb_small = std::min(S, 512), nb_tiny = std::min(blocks_for(S, TINY_WAVES), 512);
+    const int nb_micro = micro_ok(orig, pre) ? blocks_for(S, MICRO_BS) : 0;
+    hipLaunchKernelGGL(k_build_segments, dim3(nb_small + nb_tiny + nb_micro), dim3(SMALL_SB), 0, s, pts, seg, seg_depth,
+                       pair_scan, S, count_dev, lists, orig, pre, pool, hdr, nb_small, nb_tiny);
 }
 
 }  // namespace ikd

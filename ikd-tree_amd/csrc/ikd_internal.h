@@ -36,7 +36,8 @@ struct DevHdr {
     float alpha_del;
     int vox_bad;        // downsample: a voxel index of the batch is out of range
     int ins_maxlen;     // insert: points of the largest attach group
-    int small_lists[2]; // small build: segments listed for the 64- and 256-thread workgroup builds
+    int small_lists[2]; // small build: segments listed for the wavefront and workgroup shapes
+    int pair_base;      // small build: the first pair it takes
 };
 static_assert(sizeof(DevHdr) % sizeof(int) == 0, "the header is cleared as ints");
 constexpr int DEFER_CAP = 4096;  // deferred-rebuild list entries
@@ -98,7 +99,6 @@ void launch_build_side(const BuildLevel& L, DevHdr* hdr, hipStream_t s);
 void launch_build_flags(const BuildLevel& L, hipStream_t s);
 void launch_build_scatter(const BuildLevel& L, hipStream_t s);
 
-void launch_small_pairs(const int4* seg, int S, const int* count_dev, int* pairs, DevHdr* hdr, hipStream_t s);
 // Presorted lists for the small build (all null: the kernel sorts): the
 // segments' y- and z-ordered lists of point indices (list1, list2) and, for
 // every point, its position in the x-ordered list the points were gathered in.
@@ -107,13 +107,20 @@ struct SmallLists {
     const uint32_t* list2 = nullptr;
     const int* inv0 = nullptr;
 };
-// lists: 2 S ints of scratch (the size-class lists)
+// The plan of a small build: every segment's first pair and the size-class
+// lists (2 S ints); one launch where small_plan_fits(S), else the pairs, their
+// scan and the commit.
+bool small_plan_fits(int S);
+void launch_small_plan(const int4* seg, int S, const int* count_dev, const uint32_t* orig, const SmallLists& pre,
+                       int* pair_scan, int* lists, DevHdr* hdr, hipStream_t s);
+void launch_small_pairs(const int4* seg, int S, const int* count_dev, const uint32_t* orig, const SmallLists& pre,
+                        int* pairs, int* lists, DevHdr* hdr, hipStream_t s);
+void launch_small_commit(const int* pairs, const int* pair_scan, int S, DevHdr* hdr, hipStream_t s);
 void launch_build_small(const float4* pts, const int4* seg, const int* seg_depth, const int* pair_scan, int S,
-                        const int* count_dev, const uint32_t* orig, SmallLists pre, int* lists, Pool pool,
+                        const int* count_dev, const uint32_t* orig, SmallLists pre, const int* lists, Pool pool,
                         DevHdr* hdr, hipStream_t s);
 void launch_gather_list(const float4* pts, const uint32_t* perm, const int* sid, int m, float4* out, int* inv,
                         hipStream_t s);
-void launch_small_commit(const int* pairs, const int* pair_scan, int S, DevHdr* hdr, hipStream_t s);
 
 // ---------------------------------------------------------------- refit
 void launch_refit_up(Pool pool, Params prm, const int* dirty, int* pend, int* start, DevHdr* hdr, int* viol,
