@@ -12,7 +12,9 @@
 #include <climits>
 #include <cmath>
 #include <cstdio>
+#include <atomic>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -231,6 +233,15 @@ struct Stager {
     bool pending = false;
 };
 
+// A batch's event, kept alive by the batch and by the trees whose next work has
+// to wait for it.
+struct BatchEvent {
+    hipEvent_t ev = nullptr;
+    ~BatchEvent() {
+        if (ev) hipEventDestroy(ev);
+    }
+};
+
 }  // namespace
 
 struct ikd_tree_s {
@@ -262,6 +273,17 @@ struct ikd_tree_s {
     float4* removed = nullptr;  // that record (x, y, z, id bits), hdr->removed_count entries
     long long removed_cap = 0;
     hipEvent_t ev = nullptr;  // orders batch launches against this tree's stream
+    // Order against batches.  A launch has to wait for this tree's work once,
+    // not once per launch: `work` counts the calls that may have queued some,
+    // and the stream of the batch seen_by is already behind seen_work of them.
+    // The tree's work has to wait for the launches only when there is some: the
+    // next call on the tree queues the waits in `after`.  Once a caller has the
+    // stream (ikd_stream), work may be queued behind our back, and every launch
+    // orders itself at once, as it did for every tree before (48 runtime calls
+    // around a launch over 16 trees, 200 us of host time for 350 us of kernel).
+    uint64_t work = 1, seen_by = 0, seen_work = 0;
+    std::vector<std::shared_ptr<BatchEvent>> after;
+    bool stream_shared = false;
     ikd_counters_t ctr{};     // event counts since creation (ikd_get_counters)
     hipMemPool_t mp = nullptr;  // stream-ordered allocations (null: hipMalloc / hipFree)
     Stager stg;                 // pinned staging of small host-to-device copies
@@ -283,7 +305,8 @@ struct ikd_tree_s {
 // of those trees' later work waits for the launch.
 struct ikd_batch_s {
     hipStream_t st = nullptr;
-    hipEvent_t ev = nullptr;
+    std::shared_ptr<BatchEvent> done = std::make_shared<BatchEvent>();  // behind the last launch
+    uint64_t serial = 0;  // names the batch in the trees it read
     std::string err;
     int knn_lanes = -1;
     int knn_stack = 0;
@@ -356,6 +379,17 @@ hipMemPool_t library_pool(int dev) {
         (void)hipGetLastError();
     }
     return pools[dev];
+}
+
+// A call on the tree begins (its lock is held): what it queues runs after the
+// batch launches that read the tree.
+int enter_tree(ikd_tree_t t) {
+    t->work += 1;
+    while (!t->after.empty()) {
+        HIPCHK(hipStreamWaitEvent(t->st, t->after.back()->ev, 0));
+        t->after.pop_back();
+    }
+    return IKD_OK;
 }
 
 // Device memory ordered on the owner's stream: usable by work queued after
@@ -1686,9 +1720,10 @@ int upload(ikd_tree_t t, int slot, const T* h, long long n, T** d) {
 
 // =================================================================== C ABI
 // Every entry point on a tree holds the tree's lock for the whole call.
-#define CHECK_T()                    \
-    if (!t) return IKD_ERR_ARG;      \
-    std::lock_guard<std::recursive_mutex> call_lock_(t->mu)
+#define CHECK_T()                                            \
+    if (!t) return IKD_ERR_ARG;                              \
+    std::lock_guard<std::recursive_mutex> call_lock_(t->mu); \
+    CHK(enter_tree(t))
 
 extern "C" {
 
@@ -1731,6 +1766,7 @@ int ikd_destroy(ikd_tree_t t) {
     {
         // wait for a call still running on another thread
         std::lock_guard<std::recursive_mutex> g(t->mu);
+        if (t->st) enter_tree(t);
     }
     if (t->st) {
         if (t->cap > 0) free_pool(t, &t->pool);
@@ -2224,6 +2260,7 @@ int ikd_synchronize(ikd_tree_t t) {
 int ikd_stream(ikd_tree_t t, void** out) {
     CHECK_T();
     if (!out) return IKD_ERR_ARG;
+    t->stream_shared = true;
     *out = (void*)t->st;
     return IKD_OK;
 }
@@ -2441,6 +2478,17 @@ __global__ void k_store_trees(TreeTable tab, int n, TreeRef* __restrict__ dst) {
     if (i < n) dst[i] = tab.t[i];
 }
 
+// The batch's stream waits for the tree's pending work (the tree's lock is held).
+static int order_after_tree(ikd_batch_t b, ikd_tree_t tr) {
+    auto* t = b;
+    if (!tr->stream_shared && tr->seen_by == b->serial && tr->seen_work == tr->work) return IKD_OK;
+    HIPCHK(hipEventRecord(tr->ev, tr->st));
+    HIPCHK(hipStreamWaitEvent(b->st, tr->ev, 0));
+    tr->seen_by = b->serial;
+    tr->seen_work = tr->work;
+    return IKD_OK;
+}
+
 // shared prologue of batch launches: compact over-deep trees, make the batch
 // stream wait for the trees' pending work, report the deepest tree and the
 // largest pool
@@ -2457,7 +2505,8 @@ static int batch_begin(ikd_batch_t b, const ikd_tree_t* trees, int ntrees, int* 
         std::lock_guard<std::recursive_mutex> g(tr->mu);
         if (tr->max_depth + 2 > MAX_DEPTH) {
             tr->hdr_valid = false;
-            int rc = compact_if_needed(tr, true);
+            int rc = enter_tree(tr);
+            if (rc == IKD_OK) rc = compact_if_needed(tr, true);
             if (rc != IKD_OK) {
                 b->err = "batch: " + tr->err;
                 return rc;
@@ -2465,18 +2514,22 @@ static int batch_begin(ikd_batch_t b, const ikd_tree_t* trees, int ntrees, int* 
         }
         *depth = std::max(*depth, tr->max_depth);
         *steps = std::max(*steps, tr->pool_used + 16);
-        HIPCHK(hipEventRecord(tr->ev, tr->st));
-        HIPCHK(hipStreamWaitEvent(b->st, tr->ev, 0));
+        CHK(order_after_tree(b, tr));
     }
     return IKD_OK;
 }
 
 static int batch_end(ikd_batch_t b, const ikd_tree_t* trees, int ntrees) {
     auto* t = b;
-    HIPCHK(hipEventRecord(b->ev, b->st));
+    HIPCHK(hipEventRecord(b->done->ev, b->st));
     for (int i = 0; i < ntrees; ++i) {
-        std::lock_guard<std::recursive_mutex> g(trees[i]->mu);
-        HIPCHK(hipStreamWaitEvent(trees[i]->st, b->ev, 0));
+        ikd_tree_t tr = trees[i];
+        std::lock_guard<std::recursive_mutex> g(tr->mu);
+        if (tr->stream_shared) {
+            HIPCHK(hipStreamWaitEvent(tr->st, b->done->ev, 0));
+        } else if (std::find(tr->after.begin(), tr->after.end(), b->done) == tr->after.end()) {
+            tr->after.push_back(b->done);
+        }
     }
     return IKD_OK;
 }
@@ -2491,9 +2544,11 @@ int ikd_batch_create(ikd_batch_t* out) {
         delete b;
         return IKD_ERR_HIP;
     }
+    static std::atomic<uint64_t> serials{0};
+    b->serial = ++serials;
     b->mp = library_pool(dev);
     if (hipStreamCreateWithFlags(&b->st, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&b->ev, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&b->done->ev, hipEventDisableTiming) != hipSuccess ||
         hipHostMalloc(&b->h_count, sizeof(long long) + 2 * sizeof(int), hipHostMallocDefault) != hipSuccess) {
         ikd_batch_destroy(b);
         return IKD_ERR_HIP;
@@ -2524,7 +2579,6 @@ int ikd_batch_destroy(ikd_batch_t b) {
     }
     stage_release(b);
     if (b->h_count) hipHostFree(b->h_count);
-    if (b->ev) hipEventDestroy(b->ev);
     if (b->st) hipStreamDestroy(b->st);
     delete b;
     return IKD_OK;
@@ -2678,8 +2732,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
         steps = std::max(steps, tr->pool_used + 16);
         small_pools = small_pools && tr->cap <= (1ll << 24);
         tab.t[i] = TreeRef{tr->pool.hot, tr->pool.ids};
-        HIPCHK(hipEventRecord(tr->ev, tr->st));
-        HIPCHK(hipStreamWaitEvent(b->st, tr->ev, 0));
+        CHK(order_after_tree(b, tr));
     }
     hipLaunchKernelGGL(k_store_trees, dim3(1), dim3(IKD_NOALLOC_MAX_TREES), 0, b->st, tab, ntrees, table);
     launch_fill_i32(ctrl + 8, 0, 1, b->st);
@@ -2860,8 +2913,7 @@ int ikd_batch_knn_graph_launch(ikd_knn_graph_t g) {
             return IKD_ERR_UNSUPPORTED;
         }
         g->h_table[i] = TreeRef{tr->pool.hot, tr->pool.ids};
-        HIPCHK(hipEventRecord(tr->ev, tr->st));
-        HIPCHK(hipStreamWaitEvent(b->st, tr->ev, 0));
+        CHK(order_after_tree(b, tr));
     }
     HIPCHK(hipMemcpyAsync(g->d_table, g->h_table, n * sizeof(TreeRef), hipMemcpyHostToDevice, b->st));
     HIPCHK(hipEventRecord(g->ev_table, b->st));
