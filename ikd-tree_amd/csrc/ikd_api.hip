@@ -326,7 +326,7 @@ namespace {
 
 enum Buf {
     B_TMP = 0, B_PTS, B_PTS2, B_SEGOF, B_KEYA, B_KEYB, B_VALA, B_PERM0, B_PERM1 = B_PERM0 + 3, B_SID = B_PERM1 + 3,
-    B_SID2, B_SIDE, B_SEG0, B_SEG1, B_SEGD0, B_SEGD1, B_SEGAX, B_SEGMID, B_SEGCH, B_SEGFL, B_SEGSC, B_POSFL, B_POSSC,
+    B_SID2, B_SIDE, B_SEG0, B_SEG1, B_SEGD0, B_SEGD1, B_SEGAX, B_SEGMID, B_SEGCH, B_SEGFL, B_SEGSC, B_SEGLRI, B_SEGLR, B_BITS, B_TILELR,
     B_SEEDS, B_DIRTY, B_VIOL, B_TOP, B_INFO, B_FRONT0, B_FRONT1, B_EKEY0, B_EKEY1, B_RECS, B_GFLAG, B_GSCAN, B_ATTACH,
     B_PFLAG, B_PSCAN, B_ISEG, B_ISEGD, B_IO0, B_IO1, B_IO2, B_IO3, B_IO4, B_VSTART, B_DELBOX, B_DELFL, B_INSPT,
     B_INSFL, B_CBOX, B_CPTS, B_MORTK, B_MORTV, B_MORTK2, B_MORTV2, B_CNT64, B_OFF64, B_ADDX, B_ADDI, B_PNEXT, B_SPAIRS, B_SPSCAN,
@@ -777,14 +777,17 @@ int run_build(ikd_tree_t t, const float4* pts, const int* seg_of, int m, const i
     CHK(ensure(t, B_SEGD1, segcap, &segd[1]));
     int *segax, *segmid;
     int2* segch;
-    unsigned long long *segfl, *segsc, *posfl, *possc;
+    unsigned long long *segfl, *segsc, *seglri, *seglr, *bits, *tilelr;
     CHK(ensure(t, B_SEGAX, segcap, &segax));
     CHK(ensure(t, B_SEGMID, segcap, &segmid));
     CHK(ensure(t, B_SEGCH, segcap, &segch));
     CHK(ensure(t, B_SEGFL, segcap, &segfl));
     CHK(ensure(t, B_SEGSC, segcap, &segsc));
-    CHK(ensure(t, B_POSFL, 3ll * m, &posfl));
-    CHK(ensure(t, B_POSSC, 3ll * m, &possc));
+    CHK(ensure(t, B_SEGLRI, segcap, &seglri));
+    CHK(ensure(t, B_SEGLR, segcap, &seglr));
+    const long long words = ((long long)m + 63) / 64;
+    CHK(ensure(t, B_BITS, 6 * words, &bits));
+    CHK(ensure(t, B_TILELR, 3 * build_tiles(m), &tilelr));
 
     const int end_bit = 32 + bits_for(S);
     if (m <= RANK_SORT_MAX) {
@@ -794,7 +797,21 @@ int run_build(ikd_tree_t t, const float4* pts, const int* seg_of, int m, const i
         CHK(ensure(t, B_SORTV, 3ll * m, &tv));
         launch_build_sort3(pts, seg_of, m, tk, tv, perm[0], sid[0], st);
     }
-    for (int a = 0; m > RANK_SORT_MAX && a < 3; ++a) {
+    if (m > RANK_SORT_MAX && S == 1) {
+        // one segment (a Build, a compaction): 32-bit keys, half the sort's traffic
+        // and a digit pass less (2M points: 188 us a list with 64-bit keys, 134 with these)
+        uint32_t *k32 = reinterpret_cast<uint32_t*>(keya), *k32s = reinterpret_cast<uint32_t*>(keyb);
+        launch_fill_i32(sid[0], 0, m, st);
+        for (int a = 0; a < 3; ++a) {
+            launch_build_keys32(pts, m, a, k32, vala, st);
+            size_t bytes = 0;
+            HIPCHK(prim_sort_pairs_u32(nullptr, bytes, k32, k32s, vala, perm[0][a], m, st));
+            void* tmp;
+            CHK(prim_tmp<char>(t, bytes, &tmp));
+            HIPCHK(prim_sort_pairs_u32(tmp, bytes, k32, k32s, vala, perm[0][a], m, st));
+        }
+    }
+    for (int a = 0; m > RANK_SORT_MAX && S > 1 && a < 3; ++a) {
         launch_build_keys(pts, seg_of, m, a, keya, vala, st);
         CHK(sort_pairs(t, keya, keyb, vala, perm[0][a], m, end_bit));
         if (a == 0) launch_build_init_sid(keyb, m, sid[0], st);
@@ -832,19 +849,23 @@ int run_build(ikd_tree_t t, const float4* pts, const int* seg_of, int m, const i
         BL.seg_child = segch;
         BL.seg_flags = segfl;
         BL.seg_scan = segsc;
-        BL.pos_flags = posfl;
-        BL.pos_scan = possc;
+        BL.seg_lr_in = seglri;
+        BL.seg_lr = seglr;
+        BL.bits_l = bits;
+        BL.bits_r = bits + 3 * words;
+        BL.tile_lr = tilelr;
         BL.m = m;
         BL.cur = cur;
-        launch_build_seg_a(BL, (int)bound, t->d_hdr, st);
-        CHK(exscan_u64(t, segfl, segsc, (int)bound));
-        launch_build_seg_b(BL, (int)bound, t->pool, t->d_hdr, st);
-        launch_build_side(BL, t->d_hdr, st);
-        if (L + 1 < levels) {
-            launch_build_flags(BL, st);
-            CHK(exscan_u64(t, posfl, possc, 3 * m));
-            launch_build_scatter(BL, st);
+        if (build_seg_one_fits((int)bound)) {
+            launch_build_seg_one(BL, t->pool, t->d_hdr, st);
+        } else {
+            launch_build_seg_a(BL, (int)bound, t->d_hdr, st);
+            CHK(exscan_u64(t, segfl, segsc, (int)bound));
+            CHK(exscan_u64(t, seglri, seglr, (int)bound));
+            launch_build_seg_b(BL, (int)bound, t->pool, t->d_hdr, st);
         }
+        launch_build_side(BL, t->d_hdr, st);
+        if (L + 1 < levels) launch_build_partition(BL, st);
     }
     if (Ls < levels) {
         // level Ls: its segments (count on the device) and its x-ordered list

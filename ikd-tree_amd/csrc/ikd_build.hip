@@ -33,6 +33,16 @@ __global__ void k_build_keys(const float4* __restrict__ pts, const int* __restri
     vals[i] = (uint32_t)i;
 }
 
+// one segment: the coordinate alone
+__global__ void k_build_keys32(const float4* __restrict__ pts, int m, int axis, uint32_t* __restrict__ keys,
+                               uint32_t* __restrict__ vals) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= m) return;
+    float4 p = pts[i];
+    keys[i] = float_key(axis == 0 ? p.x : (axis == 1 ? p.y : p.z));
+    vals[i] = (uint32_t)i;
+}
+
 __global__ void k_build_init_sid(const unsigned long long* __restrict__ k0, int m, int* __restrict__ sid) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= m) return;
@@ -274,34 +284,27 @@ void launch_build_sort3(const float4* pts, const int* seg_of, int n, unsigned lo
 __device__ __forceinline__ float coord_of(float4 p, int a) { return a == 0 ? p.x : (a == 1 ? p.y : p.z); }
 
 // Per segment: longest axis, mid, and what it allocates (one pair if it has a
-// child; one next-level segment per non-empty side).
-__global__ void k_build_seg_a(BuildLevel L, int bound, DevHdr* hdr) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s == 0) hdr->seg_count[L.cur ^ 1] = 0;
-    if (s >= bound) return;
-    int count = hdr->seg_count[L.cur];
-    if (s >= count) {
-        L.seg_flags[s] = 0ull;
-        return;
-    }
-    int4 sg = L.seg[s];
-    int l = sg.x, r = sg.y;
+// child; one next-level segment per non-empty side): pairs | segments << 32.
+// lr: the points it sends left | right << 32.
+__device__ __forceinline__ unsigned long long seg_decide(const BuildLevel& L, int s, unsigned long long& lr) {
+    const int4 sg = L.seg[s];
+    const int l = sg.x, r = sg.y;
     float ext[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        float lo = coord_of(L.pts[L.perm[a][l]], a);
-        float hi = coord_of(L.pts[L.perm[a][r]], a);
+        const float lo = coord_of(L.pts[L.perm[a][l]], a);
+        const float hi = coord_of(L.pts[L.perm[a][r]], a);
         ext[a] = hi - lo;
     }
     int axis = 0;
     if (ext[1] > ext[axis]) axis = 1;
     if (ext[2] > ext[axis]) axis = 2;
-    int mid = (l + r) >> 1;
-    int has_l = mid > l, has_r = mid < r;
+    const int mid = (l + r) >> 1;
+    const int has_l = mid > l, has_r = mid < r;
     L.seg_axis[s] = axis;
     L.seg_mid[s] = mid;
-    unsigned long long need_pair = (has_l || has_r) ? 1ull : 0ull;
-    L.seg_flags[s] = need_pair | ((unsigned long long)(has_l + has_r) << 32);
+    lr = (unsigned long long)(uint32_t)(mid - l) | ((unsigned long long)(uint32_t)(r - mid) << 32);
+    return ((has_l || has_r) ? 1ull : 0ull) | ((unsigned long long)(has_l + has_r) << 32);
 }
 
 __device__ __forceinline__ void write_child_box(NodeHot* hot, int parent, int side, const float* b) {
@@ -315,28 +318,20 @@ __device__ __forceinline__ void write_child_box(NodeHot* hot, int parent, int si
     }
 }
 
-// Per segment: write the node and emit the child segments.
-__global__ void k_build_seg_b(BuildLevel L, int bound, Pool pool, DevHdr* hdr) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= bound) return;
-    int count = hdr->seg_count[L.cur];
-    if (s >= count) return;
-    unsigned long long sc = L.seg_scan[s];
-    unsigned long long fl = L.seg_flags[s];
-    int pairs_before = (int)(uint32_t)sc;
-    int child_before = (int)(sc >> 32);
-    int need_pair = (int)(fl & 1ull);
-    int nch = (int)(fl >> 32);
-    int4 sg = L.seg[s];
-    int l = sg.x, r = sg.y, node = sg.z, parent = sg.w;
-    int depth = L.seg_depth[s];
-    int axis = L.seg_axis[s];
-    int mid = L.seg_mid[s];
-    int has_l = mid > l, has_r = mid < r;
-    int pair = need_pair ? hdr->pair_used + pairs_before : 0;
+// Per segment: write the node and emit the child segments.  before: the pairs and
+// segments of the segments before it; first_pair: the level's first pair.
+__device__ __forceinline__ void seg_emit(const BuildLevel& L, int s, unsigned long long before, int first_pair,
+                                         const Pool& pool, DevHdr* hdr) {
+    const int4 sg = L.seg[s];
+    const int l = sg.x, r = sg.y, node = sg.z, parent = sg.w;
+    const int depth = L.seg_depth[s];
+    const int axis = L.seg_axis[s];
+    const int mid = L.seg_mid[s];
+    const int has_l = mid > l, has_r = mid < r;
+    const int pair = (has_l || has_r) ? first_pair + (int)(uint32_t)before : 0;
 
-    float4 P = L.pts[L.perm[axis][mid]];
-    uint32_t link = ((uint32_t)pair << LK_PAIR_SHIFT) | (has_l ? LK_HASL : 0u) | (has_r ? LK_HASR : 0u);
+    const float4 P = L.pts[L.perm[axis][mid]];
+    const uint32_t link = ((uint32_t)pair << LK_PAIR_SHIFT) | (has_l ? LK_HASL : 0u) | (has_r ? LK_HASR : 0u);
     *reinterpret_cast<float4*>(pool.hot[node].f) = make_float4(P.x, P.y, P.z, bitsf(link));
     pool.ids[node] = fbits(P.w);
     pool.par[node] = parent;
@@ -353,7 +348,7 @@ __global__ void k_build_seg_b(BuildLevel L, int bound, Pool pool, DevHdr* hdr) {
     box[5] = L.pts[L.perm[2][r]].z;
     write_child_box(pool.hot, parent, node & 1, box);
 
-    int c = child_before;
+    int c = (int)(before >> 32);
     int2 ch = make_int2(-1, -1);
     if (has_l) {
         L.seg_next[c] = make_int4(l, mid - 1, 2 * pair, node);
@@ -366,9 +361,78 @@ __global__ void k_build_seg_b(BuildLevel L, int bound, Pool pool, DevHdr* hdr) {
         ch.y = c++;
     }
     L.seg_child[s] = ch;
+}
+
+// A level's segments by one workgroup (up to SEG_ONE_MAX of them: decide, scan
+// and emit in one launch; each was one of the 8 launches of a level).
+__device__ __forceinline__ unsigned long long wave_inclusive_u64(unsigned long long x, int lane) {
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int src = (lane - d) & 63;  // lanes below d ignore what they read
+        const unsigned lo = (unsigned)__shfl((int)(unsigned)x, src);
+        const unsigned hi = (unsigned)__shfl((int)(unsigned)(x >> 32), src);
+        if (lane >= d) x += ((unsigned long long)hi << 32) | lo;
+    }
+    return x;
+}
+constexpr int SEG_ONE_MAX = 8192;
+__global__ __launch_bounds__(1024) void k_build_seg_one(BuildLevel L, Pool pool, DevHdr* hdr) {
+    __shared__ unsigned long long tot_f[16], tot_lr[16];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int count = hdr->seg_count[L.cur], first_pair = hdr->pair_used;
+    const int chunk = (count + 1023) >> 10;
+    const int b = min(t * chunk, count), e = min(b + chunk, count);
+    unsigned long long f = 0, lr = 0;
+    for (int s = b; s < e; ++s) {
+        unsigned long long x;
+        f += seg_decide(L, s, x);
+        lr += x;
+    }
+    const unsigned long long inc_f = wave_inclusive_u64(f, lane), inc_lr = wave_inclusive_u64(lr, lane);
+    if (lane == 63) {
+        tot_f[w] = inc_f;
+        tot_lr[w] = inc_lr;
+    }
+    __syncthreads();
+    unsigned long long run_f = inc_f - f, run_lr = inc_lr - lr;
+    for (int i = 0; i < w; ++i) {
+        run_f += tot_f[i];
+        run_lr += tot_lr[i];
+    }
+    for (int s = b; s < e; ++s) {
+        const int4 sg = L.seg[s];
+        const int mid = L.seg_mid[s];
+        const int has_l = mid > sg.x, has_r = mid < sg.y;
+        L.seg_lr[s] = run_lr;
+        seg_emit(L, s, run_f, first_pair, pool, hdr);
+        run_f += ((has_l || has_r) ? 1ull : 0ull) | ((unsigned long long)(has_l + has_r) << 32);
+        run_lr += (unsigned long long)(uint32_t)(mid - sg.x) | ((unsigned long long)(uint32_t)(sg.y - mid) << 32);
+    }
+    if (t == 1023) {
+        hdr->seg_count[L.cur ^ 1] = (int)(run_f >> 32);
+        hdr->pair_used = first_pair + (int)(uint32_t)run_f;
+    }
+}
+
+// More segments: decide, two scans, emit.
+__global__ void k_build_seg_a(BuildLevel L, int bound, DevHdr* hdr) {
+    int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0) hdr->seg_count[L.cur ^ 1] = 0;
+    if (s >= bound) return;
+    unsigned long long f = 0, lr = 0;
+    if (s < hdr->seg_count[L.cur]) f = seg_decide(L, s, lr);
+    L.seg_flags[s] = f;
+    L.seg_lr_in[s] = lr;
+}
+__global__ void k_build_seg_b(BuildLevel L, int bound, Pool pool, DevHdr* hdr) {
+    int s = blockIdx.x * blockDim.x + threadIdx.x;
+    const int count = hdr->seg_count[L.cur];
+    if (s >= bound || s >= count) return;
+    seg_emit(L, s, L.seg_scan[s], hdr->pair_used, pool, hdr);
     if (s == count - 1) {
-        hdr->seg_count[L.cur ^ 1] = child_before + nch;
-        hdr->pair_pending = pairs_before + need_pair;
+        const unsigned long long all = L.seg_scan[s] + L.seg_flags[s];
+        hdr->seg_count[L.cur ^ 1] = (int)(all >> 32);
+        hdr->pair_pending = (int)(uint32_t)all;
     }
 }
 
@@ -387,43 +451,100 @@ __global__ void k_build_side(BuildLevel L, DevHdr* hdr) {
     L.side[p] = (uint8_t)(j < mid ? 0 : (j == mid ? 2 : 1));
 }
 
-__global__ void k_build_flags(BuildLevel L) {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    int b = blockIdx.y;
-    if (j >= L.m) return;
-    int s = L.sid[j];
-    unsigned long long v = 0ull;
-    if (s >= 0) {
-        uint8_t sd = L.side[L.perm[b][j]];
-        v = sd == 0 ? 1ull : (sd == 1 ? (1ull << 32) : 0ull);
+// The stable partition of the three lists, PART_TILE positions to a workgroup.
+// k_build_bits: which positions go left and right, as one bit each, and the
+// tile's counts of both.  k_build_scatter: a position's rank among the lefts (or
+// rights) of its segment is the tile's prefix (the counts of the tiles before
+// it), the bits before it in the tile, less the lefts of the segments before
+// its own, which the segments' sizes give (seg_lr).  The bits are 1/4 byte a
+// position where a flag and its scan moved 24: a level of 2M points took 25 us
+// of flags, 45 of scan and 37 of scatter (now 24 of bits and 31 of scatter).
+constexpr int PART_TILE = 1024, PART_SB = 256, PART_WORDS = PART_TILE / 64;
+
+__global__ __launch_bounds__(PART_SB) void k_build_bits(BuildLevel L) {
+    __shared__ int cl[PART_SB / 64], cr[PART_SB / 64];
+    const int t = threadIdx.x, b = blockIdx.y, lane = t & 63, w = t >> 6;
+    const int words = (L.m + 63) >> 6, tiles = gridDim.x;
+    int nl = 0, nr = 0;
+#pragma unroll
+    for (int it = 0; it < PART_TILE / PART_SB; ++it) {
+        const int j = blockIdx.x * PART_TILE + it * PART_SB + t;
+        int sd = 2;
+        if (j < L.m && L.sid[j] >= 0) sd = L.side[L.perm[b][j]];
+        const unsigned long long ml = __ballot(sd == 0), mr = __ballot(sd == 1);
+        if (lane == 0 && j < L.m) {
+            L.bits_l[(size_t)b * words + (j >> 6)] = ml;
+            L.bits_r[(size_t)b * words + (j >> 6)] = mr;
+        }
+        nl += __popcll(ml);
+        nr += __popcll(mr);
     }
-    L.pos_flags[(size_t)b * L.m + j] = v;
+    if (lane == 0) {
+        cl[w] = nl;
+        cr[w] = nr;
+    }
+    __syncthreads();
+    if (t == 0) {
+        unsigned long long c = 0;
+        for (int i = 0; i < PART_SB / 64; ++i) c += (unsigned long long)(uint32_t)cl[i] | ((unsigned long long)(uint32_t)cr[i] << 32);
+        L.tile_lr[(size_t)b * tiles + blockIdx.x] = c;
+    }
 }
 
-__global__ void k_build_scatter(BuildLevel L) {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    int b = blockIdx.y;
-    if (j >= L.m) return;
-    int s = L.sid[j];
-    if (s < 0) {
-        if (b == 0) L.sid_next[j] = -1;
-        return;
+__global__ __launch_bounds__(PART_SB) void k_build_scatter(BuildLevel L) {
+    __shared__ unsigned long long part[PART_SB / 64];
+    __shared__ unsigned long long wl[PART_WORDS], wr[PART_WORDS];
+    __shared__ unsigned long long pre[PART_WORDS];  // lefts | rights << 32 before each word, in the list
+    const int t = threadIdx.x, b = blockIdx.y, lane = t & 63, w = t >> 6;
+    const int words = (L.m + 63) >> 6, tiles = gridDim.x;
+    const unsigned long long* __restrict__ counts = L.tile_lr + (size_t)b * tiles;
+    unsigned long long sum = 0;
+    for (int i = t; i < (int)blockIdx.x; i += PART_SB) sum += counts[i];
+    sum = wave_inclusive_u64(sum, lane);
+    if (lane == 63) part[w] = sum;
+    if (t < PART_WORDS) {
+        const int q = blockIdx.x * PART_WORDS + t;
+        wl[t] = q < words ? L.bits_l[(size_t)b * words + q] : 0ull;
+        wr[t] = q < words ? L.bits_r[(size_t)b * words + q] : 0ull;
     }
-    int l = L.seg[s].x;
-    int mid = L.seg_mid[s];
-    uint32_t p = L.perm[b][j];
-    uint8_t sd = L.side[p];
-    if (sd == 2) {
-        if (b == 0) L.sid_next[mid] = -1;
-        return;
+    __syncthreads();
+    if (t == 0) {
+        unsigned long long run = 0;
+        for (int i = 0; i < PART_SB / 64; ++i) run += part[i];
+        for (int i = 0; i < PART_WORDS; ++i) {
+            pre[i] = run;
+            run += (unsigned long long)(uint32_t)__popcll(wl[i]) | ((unsigned long long)(uint32_t)__popcll(wr[i]) << 32);
+        }
     }
-    size_t base = (size_t)b * L.m;
-    unsigned long long ex = L.pos_scan[base + j] - L.pos_scan[base + l];
-    int np = sd == 0 ? l + (int)(uint32_t)ex : mid + 1 + (int)(ex >> 32);
-    L.perm_next[b][np] = p;
-    if (b == 0) {
-        int2 ch = L.seg_child[s];
-        L.sid_next[np] = sd == 0 ? ch.x : ch.y;
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < PART_TILE / PART_SB; ++it) {
+        const int k = it * PART_SB + t, j = blockIdx.x * PART_TILE + k;
+        if (j >= L.m) continue;
+        const int s = L.sid[j];
+        if (s < 0) {
+            if (b == 0) L.sid_next[j] = -1;
+            continue;
+        }
+        const int q = k >> 6;
+        const unsigned long long below = (1ull << (k & 63)) - 1ull, bit = 1ull << (k & 63);
+        const unsigned long long p = pre[q], base = L.seg_lr[s];
+        const int mid = L.seg_mid[s];
+        int np;
+        bool left = (wl[q] & bit) != 0;
+        if (left) {
+            np = L.seg[s].x + (int)((uint32_t)p - (uint32_t)base) + __popcll(wl[q] & below);
+        } else if (wr[q] & bit) {
+            np = mid + 1 + (int)((uint32_t)(p >> 32) - (uint32_t)(base >> 32)) + __popcll(wr[q] & below);
+        } else {
+            if (b == 0) L.sid_next[mid] = -1;  // the segment's node
+            continue;
+        }
+        L.perm_next[b][np] = L.perm[b][j];
+        if (b == 0) {
+            const int2 ch = L.seg_child[s];
+            L.sid_next[np] = left ? ch.x : ch.y;
+        }
     }
 }
 
@@ -458,9 +579,17 @@ void launch_build_keys(const float4* pts, const int* seg_of, int m, int axis, un
     if (m <= 0) return;
     hipLaunchKernelGGL(k_build_keys, dim3(blocks_for(m, 256)), dim3(256), 0, s, pts, seg_of, m, axis, keys, vals);
 }
+void launch_build_keys32(const float4* pts, int m, int axis, uint32_t* keys, uint32_t* vals, hipStream_t s) {
+    if (m <= 0) return;
+    hipLaunchKernelGGL(k_build_keys32, dim3(blocks_for(m, 256)), dim3(256), 0, s, pts, m, axis, keys, vals);
+}
 void launch_build_init_sid(const unsigned long long* k0, int m, int* sid, hipStream_t s) {
     if (m <= 0) return;
     hipLaunchKernelGGL(k_build_init_sid, dim3(blocks_for(m, 256)), dim3(256), 0, s, k0, m, sid);
+}
+bool build_seg_one_fits(int bound) { return bound <= SEG_ONE_MAX; }
+void launch_build_seg_one(const BuildLevel& L, Pool pool, DevHdr* hdr, hipStream_t s) {
+    hipLaunchKernelGGL(k_build_seg_one, dim3(1), dim3(1024), 0, s, L, pool, hdr);
 }
 void launch_build_seg_a(const BuildLevel& L, int bound, DevHdr* hdr, hipStream_t s) {
     hipLaunchKernelGGL(k_build_seg_a, dim3(blocks_for(bound > 0 ? bound : 1, 256)), dim3(256), 0, s, L, bound, hdr);
@@ -472,13 +601,12 @@ void launch_build_seg_b(const BuildLevel& L, int bound, Pool pool, DevHdr* hdr, 
 void launch_build_side(const BuildLevel& L, DevHdr* hdr, hipStream_t s) {
     hipLaunchKernelGGL(k_build_side, dim3(blocks_for(L.m > 0 ? L.m : 1, 256)), dim3(256), 0, s, L, hdr);
 }
-void launch_build_flags(const BuildLevel& L, hipStream_t s) {
+long long build_tiles(long long m) { return (m + PART_TILE - 1) / PART_TILE; }
+void launch_build_partition(const BuildLevel& L, hipStream_t s) {
     if (L.m <= 0) return;
-    hipLaunchKernelGGL(k_build_flags, dim3(blocks_for(L.m, 256), 3), dim3(256), 0, s, L);
-}
-void launch_build_scatter(const BuildLevel& L, hipStream_t s) {
-    if (L.m <= 0) return;
-    hipLaunchKernelGGL(k_build_scatter, dim3(blocks_for(L.m, 256), 3), dim3(256), 0, s, L);
+    const dim3 grid((unsigned)build_tiles(L.m), 3);
+    hipLaunchKernelGGL(k_build_bits, grid, dim3(PART_SB), 0, s, L);
+    hipLaunchKernelGGL(k_build_scatter, grid, dim3(PART_SB), 0, s, L);
 }
 
 }  // namespace ikd

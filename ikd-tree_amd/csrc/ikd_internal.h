@@ -75,14 +75,18 @@ struct BuildLevel {
     int2* seg_child;       // next-level indices of the two children, -1 if none
     unsigned long long* seg_flags;  // scan input: pairs | children<<32
     unsigned long long* seg_scan;
-    unsigned long long* pos_flags;  // 3m: isL | isR<<32
-    unsigned long long* pos_scan;
+    unsigned long long* seg_lr_in;  // scan input: points sent left | right<<32
+    unsigned long long* seg_lr;     // the same of the segments before each
+    unsigned long long* bits_l;     // 3 lists of ceil(m / 64) words: positions that go left
+    unsigned long long* bits_r;     // and right
+    unsigned long long* tile_lr;    // 3 lists of build_tiles(m): lefts | rights<<32 of a tile
     int m;
     int cur;               // 0/1: which DevHdr::seg_count holds this level's count
 };
 
 void launch_build_keys(const float4* pts, const int* seg_of, int m, int axis, unsigned long long* keys,
                        uint32_t* vals, hipStream_t s);
+void launch_build_keys32(const float4* pts, int m, int axis, uint32_t* keys, uint32_t* vals, hipStream_t s);
 void launch_build_init_sid(const unsigned long long* sorted_keys0, int m, int* sid, hipStream_t s);
 // Stable sorts of lists of at most RANK_SORT_MAX keys below 2^64 - 1, in two
 // launches (tmp_key, tmp_val: scratch as long as all lists together): the
@@ -96,8 +100,11 @@ void launch_build_sort3(const float4* pts, const int* seg_of, int n, unsigned lo
 void launch_build_seg_a(const BuildLevel& L, int bound, DevHdr* hdr, hipStream_t s);
 void launch_build_seg_b(const BuildLevel& L, int bound, Pool pool, DevHdr* hdr, hipStream_t s);
 void launch_build_side(const BuildLevel& L, DevHdr* hdr, hipStream_t s);
-void launch_build_flags(const BuildLevel& L, hipStream_t s);
-void launch_build_scatter(const BuildLevel& L, hipStream_t s);
+// one launch for a level's segments where build_seg_one_fits(bound), else a, two scans, b
+bool build_seg_one_fits(int bound);
+void launch_build_seg_one(const BuildLevel& L, Pool pool, DevHdr* hdr, hipStream_t s);
+long long build_tiles(long long m);
+void launch_build_partition(const BuildLevel& L, hipStream_t s);
 
 // Presorted lists for the small build (all null: the kernel sorts): the
 // segments' y- and z-ordered lists of point indices (list1, list2) and, for
@@ -298,6 +305,8 @@ void launch_pack_points(const float* xyz, const uint32_t* ids, uint32_t id_base,
 hipError_t prim_sort_pairs_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* kin,
                                unsigned long long* kout, const uint32_t* vin, uint32_t* vout, int n,
                                int begin_bit, int end_bit, hipStream_t s);
+hipError_t prim_sort_pairs_u32(void* tmp, size_t& tmp_bytes, const uint32_t* kin, uint32_t* kout, const uint32_t* vin,
+                               uint32_t* vout, int n, hipStream_t s);
 hipError_t prim_sort_keys_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* kin,
                               unsigned long long* kout, int n, int begin_bit, int end_bit, hipStream_t s);
 hipError_t prim_exscan_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* in,

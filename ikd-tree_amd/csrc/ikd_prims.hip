@@ -16,6 +16,11 @@ hipError_t prim_sort_pairs_u64(void* tmp, size_t& tmp_bytes, const unsigned long
                                      (unsigned int)end_bit, s);
 }
 
+hipError_t prim_sort_pairs_u32(void* tmp, size_t& tmp_bytes, const uint32_t* kin, uint32_t* kout, const uint32_t* vin,
+                               uint32_t* vout, int n, hipStream_t s) {
+    return rocprim::radix_sort_pairs(tmp, tmp_bytes, kin, kout, vin, vout, (unsigned int)n, 0u, 32u, s);
+}
+
 hipError_t prim_sort_keys_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* kin, unsigned long long* kout,
                               int n, int begin_bit, int end_bit, hipStream_t s) {
     return rocprim::radix_sort_keys(tmp, tmp_bytes, kin, kout, (unsigned int)n, (unsigned int)begin_bit,

@@ -14,6 +14,23 @@ static unsigned long long bits(unsigned long long k, int b0, int b1) {
     return w >= 64 ? v : (v & ((1ull << w) - 1));
 }
 
+hipError_t prim_sort_pairs_u32(void* tmp, size_t& tmp_bytes, const uint32_t* kin, uint32_t* kout, const uint32_t* vin,
+                               uint32_t* vout, int n, hipStream_t) {
+    if (!tmp) {
+        tmp_bytes = 16;
+        return hipSuccess;
+    }
+    emu_tally("prim:sort_pairs_u32");
+    std::vector<int> idx(n);
+    std::iota(idx.begin(), idx.end(), 0);
+    std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return kin[a] < kin[b]; });
+    for (int i = 0; i < n; ++i) {
+        kout[i] = kin[idx[i]];
+        vout[i] = vin[idx[i]];
+    }
+    return hipSuccess;
+}
+
 hipError_t prim_sort_pairs_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* kin, unsigned long long* kout,
                                const uint32_t* vin, uint32_t* vout, int n, int begin_bit, int end_bit, hipStream_t) {
     if (!tmp) {

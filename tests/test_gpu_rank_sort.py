@@ -39,7 +39,7 @@ def _median_tree(p):
     return np.array(out, np.uint32)
 
 
-@pytest.mark.parametrize("n,kind", [(1025, "uniform"), (2047, "grid"), (2048, "uniform"), (2049, "same"),
+@pytest.mark.parametrize("n,kind", [(1025, "uniform"), (200001, "uniform"), (131072, "grid"), (2047, "grid"), (2048, "uniform"), (2049, "same"),
                                     (4097, "grid"), (30001, "uniform"), (65535, "grid"), (65536, "uniform"),
                                     (65537, "uniform")])
 def test_build_order(n, kind):
