@@ -1252,26 +1252,31 @@ int insert_points(ikd_tree_t t, const float4* pts, int m, const int* extra_seeds
     CHK(ensure(t, B_IO3, m, &vb));
     launch_insert_descend(t->pool, pts, m, ka, va, t->d_hdr, st);
     CHK(sort_pairs(t, ka, kb, va, vb, m, 1 + bits_for(t->pool_used)));
-    int *gflag, *gscan, *attach, *pflag, *pscan, *segof, *segd;
+    int *attach, *segof, *segd;
     int4* seg;
-    CHK(ensure(t, B_GFLAG, m, &gflag));
-    CHK(ensure(t, B_GSCAN, m, &gscan));
+    float4* spts;
     CHK(ensure(t, B_ATTACH, m, &attach));
-    CHK(ensure(t, B_PFLAG, m, &pflag));
-    CHK(ensure(t, B_PSCAN, m, &pscan));
     CHK(ensure(t, B_SEGOF, m, &segof));
     CHK(ensure(t, B_ISEG, m, &seg));
     CHK(ensure(t, B_ISEGD, m, &segd));
-    launch_insert_groups(kb, m, gflag, st);
-    CHK(exscan_i32(t, gflag, gscan, m));
-    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(1), 0, st, t->d_hdr, 16);
-    launch_insert_segments2(t->pool, kb, gscan, gflag, m, seg, segd, segof, attach, pflag, t->d_hdr, st);
-    CHK(exscan_i32(t, pflag, pscan, m));
-    launch_insert_pairs(t->pool, attach, pflag, pscan, t->d_hdr, m, seg, st);
-    hipLaunchKernelGGL(k_group_maxlen, dim3(nblk(m)), dim3(BS), 0, st, seg, t->d_hdr, m);
-    float4* spts;
     CHK(ensure(t, B_PTS2, m, &spts));
-    hipLaunchKernelGGL(k_gather_pts, dim3(nblk(m)), dim3(BS), 0, st, pts, vb, m, spts);
+    if (insert_plan_fits(m)) {
+        launch_insert_plan(t->pool, kb, m, pts, vb, seg, segd, segof, attach, spts, t->d_hdr, st);
+    } else {
+        int *gflag, *gscan, *pflag, *pscan;
+        CHK(ensure(t, B_GFLAG, m, &gflag));
+        CHK(ensure(t, B_GSCAN, m, &gscan));
+        CHK(ensure(t, B_PFLAG, m, &pflag));
+        CHK(ensure(t, B_PSCAN, m, &pscan));
+        launch_insert_groups(kb, m, gflag, st);
+        CHK(exscan_i32(t, gflag, gscan, m));
+        hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(1), 0, st, t->d_hdr, 16);
+        launch_insert_segments2(t->pool, kb, gscan, gflag, m, seg, segd, segof, attach, pflag, t->d_hdr, st);
+        CHK(exscan_i32(t, pflag, pscan, m));
+        launch_insert_pairs(t->pool, attach, pflag, pscan, t->d_hdr, m, seg, st);
+        hipLaunchKernelGGL(k_group_maxlen, dim3(nblk(m)), dim3(BS), 0, st, seg, t->d_hdr, m);
+        hipLaunchKernelGGL(k_gather_pts, dim3(nblk(m)), dim3(BS), 0, st, pts, vb, m, spts);
+    }
     CHK(sync_hdr(t));
     const int S = t->h_hdr->group_count, maxlen = t->h_hdr->ins_maxlen;
     CHK(check_count(t, "insert: attach groups", S, 1, m));

@@ -158,6 +158,12 @@ void launch_enum_groups(Pool pool, const int4* roots, const int4* groups, int n_
 // ---------------------------------------------------------------- insert
 void launch_insert_descend(Pool pool, const float4* pts, int n, unsigned long long* keys, uint32_t* vals,
                            DevHdr* hdr, hipStream_t s);
+// groups, segments, pairs, largest group and the points in slot order in one
+// launch where insert_plan_fits(n), else the launches below
+bool insert_plan_fits(int n);
+void launch_insert_plan(Pool pool, const unsigned long long* keys, int n, const float4* pts, const uint32_t* order,
+                        int4* seg, int* seg_depth, int* seg_of, int* attach, float4* out_pts, DevHdr* hdr,
+                        hipStream_t s);
 void launch_insert_groups(const unsigned long long* sorted_keys, int n, int* grp_flag, hipStream_t s);
 void launch_insert_segments2(Pool pool, const unsigned long long* keys, const int* gscan, const int* gflag, int n,
                              int4* seg, int* seg_depth, int* seg_of, int* attach, int* pair_flag, DevHdr* hdr,

@@ -625,6 +625,102 @@ __global__ void k_insert_descend(Pool pool, const float4* __restrict__ pts, int 
     keys[i] = ((unsigned long long)(uint32_t)u << 1) | (unsigned long long)side;
 }
 
+// The plan of an insert of up to INSERT_PLAN_MAX points by one workgroup: the
+// groups of points that share an attach slot, their segments, the sibling pairs
+// they need, the largest group, and the points in slot order.  A wavefront
+// marks 64 sorted keys at a time in two words of LDS, so a point's group and a
+// group's pair are a count of the words before and of the bits below, and every
+// pass reads memory in order with its loads independent: 17 us for a mapped
+// scan's 2-4k kept points (29 us with a run of consecutive keys per thread,
+// whose loads wait for one another).  That is about the time of the nine
+// launches it replaces (flags, scan, segments, scan, pairs, commit, largest,
+// gather, header), but eight fewer to enqueue: 20 mapped scans 16.30-17.02 ->
+// 16.21-16.22 ms, from host memory 10.95-11.44 -> 10.86-11.30.  One workgroup
+// takes longer than the chip from some ten thousand points, so longer inserts
+// keep the nine.
+constexpr int INSERT_PLAN_MAX = 8192;
+__global__ __launch_bounds__(1024) void k_insert_plan(Pool pool, const unsigned long long* __restrict__ keys, int n,
+                                                      const float4* __restrict__ pts,
+                                                      const uint32_t* __restrict__ order, int4* __restrict__ seg,
+                                                      int* __restrict__ seg_depth, int* __restrict__ seg_of,
+                                                      int* __restrict__ attach, float4* __restrict__ out_pts,
+                                                      DevHdr* hdr) {
+    constexpr int WORDS = INSERT_PLAN_MAX / 64;
+    __shared__ unsigned long long heads[WORDS], fresh[WORDS];  // first of a group; of one that takes a new pair
+    __shared__ int2 before[WORDS];                             // groups and new pairs in the words before
+    __shared__ int longest;
+    const int t = threadIdx.x, lane = t & 63;
+    const int words = (n + 63) >> 6;
+    const int first_pair = hdr->pair_used;
+    if (t == 0) longest = 0;
+    for (int w0 = 0; w0 < words; w0 += 16) {  // as often in every wavefront
+        const int w = w0 + (t >> 6), i = w * 64 + lane;
+        bool head = false, needs = false;
+        if (i < n) {
+            const unsigned long long key = keys[i], prev = i > 0 ? keys[i - 1] : ~key;
+            out_pts[i] = pts[order[i]];
+            head = key != prev;
+            // the node's first group takes a pair for both, unless it has one
+            needs = (key >> 1) != (prev >> 1) && lk_pair(load_link(pool.hot, (int)(key >> 1))) == 0;
+        }
+        const unsigned long long h = __ballot(head), f = __ballot(needs);
+        if (lane == 0 && w < words) {
+            heads[w] = h;
+            fresh[w] = f;
+        }
+    }
+    __syncthreads();
+    if (t < WORDS) {
+        int g = 0, p = 0;
+        for (int w = 0; w < min(t, words); ++w) {
+            g += __popcll(heads[w]);
+            p += __popcll(fresh[w]);
+        }
+        before[t] = make_int2(g, p);
+    }
+    __syncthreads();
+    int most = 0;
+    for (int w = t >> 6; w < words; w += 16) {
+        const int i = w * 64 + lane;
+        if (i >= n) continue;
+        const unsigned long long key = keys[i], upto = ~0ull >> (63 - lane);
+        const unsigned long long h = heads[w];
+        const int g = before[w].x + __popcll(h & upto) - 1;
+        seg_of[i] = g;
+        if ((h >> lane) & 1ull) {
+            const int X = (int)(key >> 1);
+            int pair = (int)lk_pair(load_link(pool.hot, X));
+            // a new one is this group's, or its sibling group's just before it
+            if (pair == 0) pair = first_pair + before[w].y + __popcll(fresh[w] & upto) - 1;
+            // up to the next group's first point
+            int u = w;
+            unsigned long long hu = h & ~upto;
+            while (hu == 0 && ++u < words) hu = heads[u];
+            const int end = hu ? u * 64 + __ffsll((long long)hu) - 2 : n - 1;
+            seg[g] = make_int4(i, end, 2 * pair + (int)(key & 1ull), X);
+            attach[g] = (int)key;
+            seg_depth[g] = X == SENTINEL ? 0 : pool.cnt[X].w + 1;
+            most = max(most, end - i + 1);
+        }
+    }
+    if (most > 0) atomicMax(&longest, most);
+    __syncthreads();
+    if (t == 0) {
+        const int w = words - 1;
+        hdr->group_count = before[w].x + __popcll(heads[w]);
+        hdr->ins_maxlen = longest;
+        hdr->pair_used = first_pair + before[w].y + __popcll(fresh[w]);
+    }
+}
+bool insert_plan_fits(int n) { return n <= INSERT_PLAN_MAX; }
+void launch_insert_plan(Pool pool, const unsigned long long* keys, int n, const float4* pts, const uint32_t* order,
+                        int4* seg, int* seg_depth, int* seg_of, int* attach, float4* out_pts, DevHdr* hdr,
+                        hipStream_t s) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_insert_plan, dim3(1), dim3(1024), 0, s, pool, keys, n, pts, order, seg, seg_depth, seg_of,
+                       attach, out_pts, hdr);
+}
+
 __global__ void k_insert_groups(const unsigned long long* __restrict__ keys, int n, int* __restrict__ flag) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
