@@ -269,6 +269,9 @@ struct ikd_tree_s {
     int fold_lanes = 0;   // lanes per voxel in the downsample fold: 0 picks by map size; else 1, 4, 8, 16
     int knn_stage = 0;    // one-lane kNN: tree levels staged in each workgroup's LDS (0: none)
     int knn_compact = 1;  // one-lane kNN: 4-byte LDS stack entries when the pool has <= 2^24 slots
+    // Add_Point_Boxes has restored points since the pool was last built anew:
+    // stored ranges may miss some of them (knn_lanes_for)
+    bool ranges_miss = false;
     int record_removed = 0;     // 1: rebuilds record the deleted points they drop (acquire_removed_points)
     float4* removed = nullptr;  // that record (x, y, z, id bits), hdr->removed_count entries
     long long removed_cap = 0;
@@ -713,6 +716,7 @@ int reserve_nodes(ikd_tree_t t, long long extra) {
 int reset_pool(ikd_tree_t t) {
     t->pool_used = 4;
     t->max_depth = 0;
+    t->ranges_miss = false;
     CHK(reserve_nodes(t, 4));
     hipLaunchKernelGGL(k_init_pool, dim3(1), dim3(1), 0, t->st, t->pool, t->d_hdr);
     HIPCHK(hipGetLastError());
@@ -1384,6 +1388,7 @@ int add_boxes_dev(ikd_tree_t t, const float* d_boxes, int nb) {
         }
         CHK(check_count(t, "box re-insertion: records", nrec, 0, cap));
         if (nrec == 0) continue;
+        t->ranges_miss = true;
         int* seeds;
         CHK(ensure(t, B_SEEDS, nrec, &seeds));
         const int levels = t->max_depth + 2;
@@ -1556,6 +1561,13 @@ int auto_lanes(int nq) {
     return nq < (1 << 17) ? 4 : 1;
 }
 
+// Lanes per query for a launch that was to take `lanes`.  Where a stored range
+// misses points below it, what a walk finds depends on when it gets there: a
+// team, whose bound has points of several branches in it early, can pass over
+// a subtree that the reference's order enters.  One lane per query walks in
+// that order and enters all of them.
+int knn_lanes_for(int lanes, bool ranges_miss) { return ranges_miss && lanes > 1 ? 1 : lanes; }
+
 float max_dist_threshold(double max_dist) {
     double m = max_dist * max_dist;
     if (std::isnan(m)) return -INFINITY;
@@ -1612,7 +1624,7 @@ int knn_dev(ikd_tree_t t, const float* d_q, int nq, int k, double max_dist, floa
     int stack = t->max_depth + 2;
     if (t->knn_stack > stack) stack = t->knn_stack;
     if (stack > MAX_DEPTH) stack = MAX_DEPTH;
-    int lanes = t->knn_lanes >= 0 ? t->knn_lanes : auto_lanes(nq);
+    const int lanes = knn_lanes_for(t->knn_lanes >= 0 ? t->knn_lanes : auto_lanes(nq), t->ranges_miss);
     if (t->knn_stage > 0 && lanes == 1) {
         // the staged levels, capped so that one workgroup's LDS (stacks and
         // table) stays within 64 KiB
@@ -2658,8 +2670,9 @@ int ikd_batch_nearest_search_device(ikd_batch_t b, const ikd_tree_t* trees, int 
     long long steps;
     CHK(batch_begin(b, trees, ntrees, &depth, &steps));
     std::vector<TreeRef> refs((size_t)ntrees);
-    bool small_pools = true;
+    bool small_pools = true, ranges_miss = false;
     for (int i = 0; i < ntrees; ++i) {
+        ranges_miss = ranges_miss || trees[i]->ranges_miss;
         refs[i] = TreeRef{trees[i]->pool.hot, trees[i]->pool.ids};
         small_pools = small_pools && trees[i]->cap <= (1ll << 24);
     }
@@ -2693,7 +2706,7 @@ int ikd_batch_nearest_search_device(ikd_batch_t b, const ikd_tree_t* trees, int 
     a.overflow = flag;
     a.max_steps = (int)std::min<long long>(steps, INT_MAX);
     int stack = std::min(std::max(depth + 2, b->knn_stack), MAX_DEPTH);
-    int lanes = b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq);
+    const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq), ranges_miss);
     if (launch_knn(a, k_max, lanes, stack, b->st, next, 256 * 10) != 0) {
         b->err = "batch: unsupported launch shape";
         return IKD_ERR_UNSUPPORTED;
@@ -2741,7 +2754,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
     TreeTable tab;
     int depth = 0;
     long long steps = 16;
-    bool small_pools = true;
+    bool small_pools = true, ranges_miss = false;
     for (int i = 0; i < ntrees; ++i) {
         ikd_tree_t tr = trees[i];
         if (!tr) {
@@ -2757,6 +2770,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
         depth = std::max(depth, tr->max_depth);
         steps = std::max(steps, tr->pool_used + 16);
         small_pools = small_pools && tr->cap <= (1ll << 24);
+        ranges_miss = ranges_miss || tr->ranges_miss;
         tab.t[i] = TreeRef{tr->pool.hot, tr->pool.ids};
         CHK(order_after_tree(b, tr));
     }
@@ -2784,7 +2798,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
     a.overflow = ctrl + 8;
     a.max_steps = (int)std::min<long long>(steps, INT_MAX);
     const int stack = std::min(std::max(depth + 2, b->knn_stack), MAX_DEPTH);
-    const int lanes = b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq);
+    const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq), ranges_miss);
     if (launch_knn(a, k_max, lanes, stack, b->st, ctrl, 256 * 10) != 0) {
         b->err = "batch (no-alloc): unsupported launch shape";
         return IKD_ERR_UNSUPPORTED;
@@ -2804,8 +2818,10 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
 struct ikd_knn_graph_s {
     ikd_batch_t b = nullptr;
     std::vector<ikd_tree_t> trees;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    // the launch, and where it takes teams the same with one lane per query,
+    // for replays over trees whose ranges may miss points
+    hipGraph_t graph[2] = {nullptr, nullptr};
+    hipGraphExec_t exec[2] = {nullptr, nullptr};
     TreeRef* d_table = nullptr;
     TreeRef* h_table = nullptr;     // pinned staging of the table refresh
     hipEvent_t ev_table = nullptr;  // behind the last refresh's copy
@@ -2818,8 +2834,10 @@ struct ikd_knn_graph_s {
 static void knn_graph_free(ikd_knn_graph_t g) {
     if (!g) return;
     if (g->table_pending) hipEventSynchronize(g->ev_table);
-    if (g->exec) hipGraphExecDestroy(g->exec);
-    if (g->graph) hipGraphDestroy(g->graph);
+    for (int v = 0; v < 2; ++v) {
+        if (g->exec[v]) hipGraphExecDestroy(g->exec[v]);
+        if (g->graph[v]) hipGraphDestroy(g->graph[v]);
+    }
     if (g->b && g->b->st) hipStreamSynchronize(g->b->st);  // no replay still reads the buffers
     if (g->d_table) hipFree(g->d_table);
     if (g->h_table) hipHostFree(g->h_table);
@@ -2900,23 +2918,25 @@ int ikd_batch_knn_graph_create(ikd_batch_t b, const ikd_tree_t* trees, int ntree
     // outlive the trees' growth
     a.max_steps = 1 << 30;
     const int lanes = b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq);
-    if (hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal) != hipSuccess) {
-        (void)hipGetLastError();
-        knn_graph_free(g);
-        b->err = "recorded kNN: stream capture could not begin";
-        return IKD_ERR_HIP;
-    }
-    launch_fill_i32(flag, 0, 1, b->st);
-    if (d_max_dist) launch_thresholds(d_max_dist, (int)nq, g->d_thr, b->st);
-    const int lrc = launch_knn(a, k_max, lanes, g->stack, b->st, g->d_ctrl, 256 * 10);
-    const hipError_t le = hipGetLastError();
-    const hipError_t ce = hipStreamEndCapture(b->st, &g->graph);
-    if (lrc != 0 || le != hipSuccess || ce != hipSuccess || !g->graph ||
-        hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0) != hipSuccess) {
-        (void)hipGetLastError();
-        knn_graph_free(g);
-        b->err = lrc != 0 ? "recorded kNN: unsupported launch shape" : "recorded kNN: recording the launch failed";
-        return lrc != 0 ? IKD_ERR_UNSUPPORTED : IKD_ERR_HIP;
+    for (int v = 0; v < (knn_lanes_for(lanes, true) != lanes ? 2 : 1); ++v) {
+        if (hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal) != hipSuccess) {
+            (void)hipGetLastError();
+            knn_graph_free(g);
+            b->err = "recorded kNN: stream capture could not begin";
+            return IKD_ERR_HIP;
+        }
+        launch_fill_i32(flag, 0, 1, b->st);
+        if (d_max_dist) launch_thresholds(d_max_dist, (int)nq, g->d_thr, b->st);
+        const int lrc = launch_knn(a, k_max, knn_lanes_for(lanes, v == 1), g->stack, b->st, g->d_ctrl, 256 * 10);
+        const hipError_t le = hipGetLastError();
+        const hipError_t ce = hipStreamEndCapture(b->st, &g->graph[v]);
+        if (lrc != 0 || le != hipSuccess || ce != hipSuccess || !g->graph[v] ||
+            hipGraphInstantiate(&g->exec[v], g->graph[v], nullptr, nullptr, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            knn_graph_free(g);
+            b->err = lrc != 0 ? "recorded kNN: unsupported launch shape" : "recorded kNN: recording the launch failed";
+            return lrc != 0 ? IKD_ERR_UNSUPPORTED : IKD_ERR_HIP;
+        }
     }
     *out = g;
     return IKD_OK;
@@ -2931,6 +2951,7 @@ int ikd_batch_knn_graph_launch(ikd_knn_graph_t g) {
     if (g->table_pending) HIPCHK(hipEventSynchronize(g->ev_table));
     g->table_pending = false;
     const int n = (int)g->trees.size();
+    bool ranges_miss = false;
     for (int i = 0; i < n; ++i) {
         ikd_tree_t tr = g->trees[i];
         std::lock_guard<std::recursive_mutex> lk(tr->mu);
@@ -2938,13 +2959,14 @@ int ikd_batch_knn_graph_launch(ikd_knn_graph_t g) {
             b->err = "recorded kNN: a tree grew deeper than the recorded launch allows; record it again";
             return IKD_ERR_UNSUPPORTED;
         }
+        ranges_miss = ranges_miss || tr->ranges_miss;
         g->h_table[i] = TreeRef{tr->pool.hot, tr->pool.ids};
         CHK(order_after_tree(b, tr));
     }
     HIPCHK(hipMemcpyAsync(g->d_table, g->h_table, n * sizeof(TreeRef), hipMemcpyHostToDevice, b->st));
     HIPCHK(hipEventRecord(g->ev_table, b->st));
     g->table_pending = true;
-    HIPCHK(hipGraphLaunch(g->exec, b->st));
+    HIPCHK(hipGraphLaunch(g->exec[ranges_miss && g->exec[1] ? 1 : 0], b->st));
     return batch_end(b, g->trees.data(), n);
 }
 
