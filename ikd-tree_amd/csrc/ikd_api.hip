@@ -569,15 +569,6 @@ int sort_pairs(ikd_tree_t t, const unsigned long long* kin, unsigned long long* 
     HIPCHK(prim_sort_pairs_u64(tmp, bytes, kin, kout, vin, vout, n, 0, end_bit, t->st));
     return IKD_OK;
 }
-int sort_keys(ikd_tree_t t, const unsigned long long* kin, unsigned long long* kout, int n, int end_bit) {
-    if (n <= 0) return IKD_OK;
-    size_t bytes = 0;
-    HIPCHK(prim_sort_keys_u64(nullptr, bytes, kin, kout, n, 0, end_bit, t->st));
-    void* tmp;
-    CHK(prim_tmp<char>(t, bytes, &tmp));
-    HIPCHK(prim_sort_keys_u64(tmp, bytes, kin, kout, n, 0, end_bit, t->st));
-    return IKD_OK;
-}
 // Exclusive scans of up to SCAN_ONE_MAX values run as one workgroup in one
 // launch: each of the 1024 threads sums a run of consecutive values, the run
 // totals are scanned across the wavefronts, then each thread rewrites its run.

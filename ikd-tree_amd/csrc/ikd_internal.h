@@ -207,8 +207,6 @@ void launch_voxel_fold2(Pool pool, const float4* pts, const uint32_t* order, con
                         const int* vstart, int n, int bound, float ds, int check, float* del_boxes, int* del_flag,
                         float4* ins_pts, int* ins_flag, DevHdr* hdr, long long max_steps, int* del_out, int del_cap,
                         int stack_cap, int lanes, const int* bad, hipStream_t s);
-void launch_compact_boxes(const int* flag, const int* scan, const float* in, int bound, DevHdr* hdr, float* out,
-                          int* out_count, hipStream_t s);
 void launch_compact_pts(const int* flag, const int* scan, const float4* in, int bound, DevHdr* hdr, float4* out,
                         int* out_count, hipStream_t s);
 
@@ -313,8 +311,6 @@ hipError_t prim_sort_pairs_u64(void* tmp, size_t& tmp_bytes, const unsigned long
                                int begin_bit, int end_bit, hipStream_t s);
 hipError_t prim_sort_pairs_u32(void* tmp, size_t& tmp_bytes, const uint32_t* kin, uint32_t* kout, const uint32_t* vin,
                                uint32_t* vout, int n, hipStream_t s);
-hipError_t prim_sort_keys_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* kin,
-                              unsigned long long* kout, int n, int begin_bit, int end_bit, hipStream_t s);
 hipError_t prim_exscan_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* in,
                            unsigned long long* out, int n, hipStream_t s);
 hipError_t prim_exscan_i32(void* tmp, size_t& tmp_bytes, const int* in, int* out, int n, hipStream_t s);

@@ -21,12 +21,6 @@ hipError_t prim_sort_pairs_u32(void* tmp, size_t& tmp_bytes, const uint32_t* kin
     return rocprim::radix_sort_pairs(tmp, tmp_bytes, kin, kout, vin, vout, (unsigned int)n, 0u, 32u, s);
 }
 
-hipError_t prim_sort_keys_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* kin, unsigned long long* kout,
-                              int n, int begin_bit, int end_bit, hipStream_t s) {
-    return rocprim::radix_sort_keys(tmp, tmp_bytes, kin, kout, (unsigned int)n, (unsigned int)begin_bit,
-                                    (unsigned int)end_bit, s);
-}
-
 hipError_t prim_exscan_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* in, unsigned long long* out, int n,
                            hipStream_t s) {
     return rocprim::exclusive_scan(tmp, tmp_bytes, in, out, 0ull, (size_t)n, rocprim::plus<unsigned long long>(), s);

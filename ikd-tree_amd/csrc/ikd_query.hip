@@ -266,7 +266,6 @@ static inline int xcd_grid(int nchunks) {
 // distance would, and at most one visit more than the 16-bit key (the visit
 // evaluates the children's boxes exactly, and a child's box lies inside the
 // node's).  Two thirds of the LDS per lane keep more wavefronts resident.
-constexpr int COMPACT_NODE_BITS = 24;
 __device__ __forceinline__ uint32_t compact_entry(int n, float d) {
     return ((uint32_t)n << 8) | (fbits(d) >> 23);
 }

@@ -535,19 +535,7 @@ __global__ __launch_bounds__(64) void k_voxel_fold_team(Pool pool, const float4*
     });
 }
 
-// stream compaction of the flagged voxel boxes / points
-__global__ void k_compact_boxes(const int* __restrict__ flag, const int* __restrict__ scan, const float* __restrict__ in,
-                                int bound, DevHdr* hdr, float* __restrict__ out, int* __restrict__ out_count) {
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    int nv = hdr->group_count;
-    if (v >= bound || v >= nv) return;
-    if (v == nv - 1) *out_count = scan[v] + flag[v];
-    if (!flag[v]) return;
-    int o = scan[v];
-#pragma unroll
-    for (int a = 0; a < 6; ++a) out[6 * o + a] = in[6 * v + a];
-}
-
+// stream compaction of the flagged voxels' points
 __global__ void k_compact_pts(const int* __restrict__ flag, const int* __restrict__ scan, const float4* __restrict__ in,
                               int bound, DevHdr* hdr, float4* __restrict__ out, int* __restrict__ out_count) {
     int v = blockIdx.x * blockDim.x + threadIdx.x;
@@ -592,12 +580,6 @@ void launch_voxel_fold2(Pool pool, const float4* pts, const uint32_t* order, con
                                del_out, del_cap, stack_cap, bad);
     }
 #undef IKD_FOLD_TEAM
-}
-void launch_compact_boxes(const int* flag, const int* scan, const float* in, int bound, DevHdr* hdr, float* out,
-                          int* out_count, hipStream_t s) {
-    if (bound <= 0) return;
-    hipLaunchKernelGGL(k_compact_boxes, dim3(blocks_for(bound, 256)), dim3(256), 0, s, flag, scan, in, bound, hdr, out,
-                       out_count);
 }
 void launch_compact_pts(const int* flag, const int* scan, const float4* in, int bound, DevHdr* hdr, float4* out,
                         int* out_count, hipStream_t s) {

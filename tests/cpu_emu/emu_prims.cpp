@@ -53,21 +53,6 @@ hipError_t prim_sort_pairs_u64(void* tmp, size_t& tmp_bytes, const unsigned long
     return hipSuccess;
 }
 
-hipError_t prim_sort_keys_u64(void* tmp, size_t& tmp_bytes, const unsigned long long* kin, unsigned long long* kout,
-                              int n, int begin_bit, int end_bit, hipStream_t) {
-    if (!tmp) {
-        tmp_bytes = 16;
-        return hipSuccess;
-    }
-    emu_tally("prim:sort_keys_u64");
-    std::vector<unsigned long long> k2(kin, kin + n);
-    std::stable_sort(k2.begin(), k2.end(), [&](unsigned long long a, unsigned long long b) {
-        return bits(a, begin_bit, end_bit) < bits(b, begin_bit, end_bit);
-    });
-    std::copy(k2.begin(), k2.end(), kout);
-    return hipSuccess;
-}
-
 template <class T>
 static hipError_t exscan(void* tmp, size_t& tmp_bytes, const T* in, T* out, int n) {
     if (!tmp) {
