@@ -765,12 +765,13 @@ def knn_kernel_name(k, lanes, lds_levels=0, compact=1):
     if lanes == 1:
         if lds_levels > 0:
             return f"ikd::k_knn_staged<{knn_bucket(k)}>"
-        return f"ikd::k_knn<{knn_bucket(k)}, {'true' if compact else 'false'}>"
+        return f"ikd::k_knn<{knn_bucket(k)}, {'true' if compact else 'false'}, false>"
     if lanes == 0:
         return f"ikd::k_knn_persist<{knn_bucket(k)}>"
     if lanes < 0:
         return f"ikd::k_knn*<{knn_bucket(k)}> (lanes per query from the batch size)"
-    return f"ikd::k_knn_team<{knn_bucket(k)}, {lanes}, {'true' if compact else 'false'}>"
+    slots = next(s for s in (1, 2, 3, 5, 8, 16, 32) if -(-k // lanes) <= s)  # of the team's list, per lane
+    return f"ikd::k_knn_team<{slots}, {lanes}, {'true' if compact else 'false'}>"
 
 
 def knn_bucket(k):
