@@ -257,6 +257,10 @@ def _result_arrays(lib, parts):
     return out
 
 
+# Result points a range search makes room for before it knows their number (64 MB).
+ROOM_MAX = 1 << 22
+
+
 class KD_TREE:
     """``KD_TREE<PointType>`` (ikd-Tree/ikd_Tree.h:59-249) on one MI355X."""
 
@@ -345,18 +349,25 @@ class KD_TREE:
         off = np.zeros(n + 1, np.int64)
         # room for a quarter more points per query than the last call of this kind
         # found, so that one call usually finds and delivers them; without
-        # enough room the call still gives the offsets
-        room = int(self._room.get(fn.__name__, 0.0) * n)
+        # enough room the call still gives the offsets.  A guess above ROOM_MAX
+        # (few queries with much, then many) is not tried.
+        room = int(min(self._room.get(fn.__name__, 0.0) * n, ROOM_MAX + 1))
+        if room > ROOM_MAX:
+            room = 0
         xyz, ids = _result_arrays(self._lib, (((room, 3), np.float32), ((room,), np.uint32)))
         rc = fn(self._h, *args, n, _ptr(off), _ptr(xyz) if room else None, _ptr(ids) if room else None, room)
         if rc not in (IKD_OK, IKD_ERR_CAPACITY):
             self._check(rc)
         total = int(off[n])
+        if n > 0:
+            self._room[fn.__name__] = 1.25 * total / n
         if total > room:
             xyz, ids = _result_arrays(self._lib, (((total, 3), np.float32), ((total,), np.uint32)))
             self._check(fn(self._h, *args, n, _ptr(off), _ptr(xyz), _ptr(ids), total))
-        if n > 0:
-            self._room[fn.__name__] = min(1.25 * total / n, (1 << 24) / n)
+        elif 2 * total < room:  # results keep no more than twice their size alive
+            big = xyz, ids
+            xyz, ids = _result_arrays(self._lib, (((total, 3), np.float32), ((total,), np.uint32)))
+            xyz[:], ids[:] = big[0][:total], big[1][:total]
         return off, xyz[:total], ids[:total]
 
     def box_search_batch(self, boxes):
