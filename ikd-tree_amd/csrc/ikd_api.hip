@@ -2507,9 +2507,17 @@ __global__ void k_store_trees(TreeTable tab, int n, TreeRef* __restrict__ dst) {
     if (i < n) dst[i] = tab.t[i];
 }
 
-// The batch's stream waits for the tree's pending work (the tree's lock is held).
-static int order_after_tree(ikd_batch_t b, ikd_tree_t tr) {
+// The batch's stream waits for the tree's pending work and for other batches'
+// launches that read the tree (the tree's lock is held): launches with a tree in
+// common run one behind the other, so one may read what the other wrote, and
+// they can share the no-alloc scratch.  waited: the launches this call is behind.
+static int order_after_tree(ikd_batch_t b, ikd_tree_t tr, std::vector<const BatchEvent*>& waited) {
     auto* t = b;
+    for (const auto& e : tr->after) {
+        if (e == b->done || std::find(waited.begin(), waited.end(), e.get()) != waited.end()) continue;
+        HIPCHK(hipStreamWaitEvent(b->st, e->ev, 0));
+        waited.push_back(e.get());
+    }
     if (!tr->stream_shared && tr->seen_by == b->serial && tr->seen_work == tr->work) return IKD_OK;
     HIPCHK(hipEventRecord(tr->ev, tr->st));
     HIPCHK(hipStreamWaitEvent(b->st, tr->ev, 0));
@@ -2525,6 +2533,7 @@ static int batch_begin(ikd_batch_t b, const ikd_tree_t* trees, int ntrees, int* 
     auto* t = b;
     *depth = 0;
     *steps = 16;
+    std::vector<const BatchEvent*> waited;
     for (int i = 0; i < ntrees; ++i) {
         ikd_tree_t tr = trees[i];
         if (!tr) {
@@ -2543,7 +2552,7 @@ static int batch_begin(ikd_batch_t b, const ikd_tree_t* trees, int ntrees, int* 
         }
         *depth = std::max(*depth, tr->max_depth);
         *steps = std::max(*steps, tr->pool_used + 16);
-        CHK(order_after_tree(b, tr));
+        CHK(order_after_tree(b, tr, waited));
     }
     return IKD_OK;
 }
@@ -2746,6 +2755,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
     int depth = 0;
     long long steps = 16;
     bool small_pools = true, ranges_miss = false;
+    std::vector<const BatchEvent*> waited;
     for (int i = 0; i < ntrees; ++i) {
         ikd_tree_t tr = trees[i];
         if (!tr) {
@@ -2763,7 +2773,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
         small_pools = small_pools && tr->cap <= (1ll << 24);
         ranges_miss = ranges_miss || tr->ranges_miss;
         tab.t[i] = TreeRef{tr->pool.hot, tr->pool.ids};
-        CHK(order_after_tree(b, tr));
+        CHK(order_after_tree(b, tr, waited));
     }
     hipLaunchKernelGGL(k_store_trees, dim3(1), dim3(IKD_NOALLOC_MAX_TREES), 0, b->st, tab, ntrees, table);
     launch_fill_i32(ctrl + 8, 0, 1, b->st);
@@ -2943,6 +2953,7 @@ int ikd_batch_knn_graph_launch(ikd_knn_graph_t g) {
     g->table_pending = false;
     const int n = (int)g->trees.size();
     bool ranges_miss = false;
+    std::vector<const BatchEvent*> waited;
     for (int i = 0; i < n; ++i) {
         ikd_tree_t tr = g->trees[i];
         std::lock_guard<std::recursive_mutex> lk(tr->mu);
@@ -2952,7 +2963,7 @@ int ikd_batch_knn_graph_launch(ikd_knn_graph_t g) {
         }
         ranges_miss = ranges_miss || tr->ranges_miss;
         g->h_table[i] = TreeRef{tr->pool.hot, tr->pool.ids};
-        CHK(order_after_tree(b, tr));
+        CHK(order_after_tree(b, tr, waited));
     }
     HIPCHK(hipMemcpyAsync(g->d_table, g->h_table, n * sizeof(TreeRef), hipMemcpyHostToDevice, b->st));
     HIPCHK(hipEventRecord(g->ev_table, b->st));
