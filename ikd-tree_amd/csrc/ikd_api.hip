@@ -2507,12 +2507,24 @@ __global__ void k_store_trees(TreeTable tab, int n, TreeRef* __restrict__ dst) {
     if (i < n) dst[i] = tab.t[i];
 }
 
+// The launch being queued on the batch's stream.
+struct LaunchOrder {
+    bool captured = false;  // into a graph of the caller's: it runs when the caller replays it, nothing is ordered now
+    std::vector<const BatchEvent*> waited;  // other batches' launches it is behind
+    explicit LaunchOrder(ikd_batch_t b) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        captured = hipStreamIsCapturing(b->st, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+    }
+};
+
 // The batch's stream waits for the tree's pending work and for other batches'
 // launches that read the tree (the tree's lock is held): launches with a tree in
 // common run one behind the other, so one may read what the other wrote, and
-// they can share the no-alloc scratch.  waited: the launches this call is behind.
-static int order_after_tree(ikd_batch_t b, ikd_tree_t tr, std::vector<const BatchEvent*>& waited) {
+// they can share the no-alloc scratch.
+static int order_after_tree(ikd_batch_t b, ikd_tree_t tr, LaunchOrder& order) {
     auto* t = b;
+    if (order.captured) return IKD_OK;
+    auto& waited = order.waited;
     for (const auto& e : tr->after) {
         if (e == b->done || std::find(waited.begin(), waited.end(), e.get()) != waited.end()) continue;
         HIPCHK(hipStreamWaitEvent(b->st, e->ev, 0));
@@ -2529,11 +2541,11 @@ static int order_after_tree(ikd_batch_t b, ikd_tree_t tr, std::vector<const Batc
 // shared prologue of batch launches: compact over-deep trees, make the batch
 // stream wait for the trees' pending work, report the deepest tree and the
 // largest pool
-static int batch_begin(ikd_batch_t b, const ikd_tree_t* trees, int ntrees, int* depth, long long* steps) {
+static int batch_begin(ikd_batch_t b, const ikd_tree_t* trees, int ntrees, LaunchOrder& order, int* depth,
+                       long long* steps) {
     auto* t = b;
     *depth = 0;
     *steps = 16;
-    std::vector<const BatchEvent*> waited;
     for (int i = 0; i < ntrees; ++i) {
         ikd_tree_t tr = trees[i];
         if (!tr) {
@@ -2552,13 +2564,14 @@ static int batch_begin(ikd_batch_t b, const ikd_tree_t* trees, int ntrees, int* 
         }
         *depth = std::max(*depth, tr->max_depth);
         *steps = std::max(*steps, tr->pool_used + 16);
-        CHK(order_after_tree(b, tr, waited));
+        CHK(order_after_tree(b, tr, order));
     }
     return IKD_OK;
 }
 
-static int batch_end(ikd_batch_t b, const ikd_tree_t* trees, int ntrees) {
+static int batch_end(ikd_batch_t b, const ikd_tree_t* trees, int ntrees, const LaunchOrder& order) {
     auto* t = b;
+    if (order.captured) return IKD_OK;
     HIPCHK(hipEventRecord(b->done->ev, b->st));
     for (int i = 0; i < ntrees; ++i) {
         ikd_tree_t tr = trees[i];
@@ -2668,7 +2681,8 @@ int ikd_batch_nearest_search_device(ikd_batch_t b, const ikd_tree_t* trees, int 
     auto* t = b;  // HIPCHK reports into b->err
     int depth;
     long long steps;
-    CHK(batch_begin(b, trees, ntrees, &depth, &steps));
+    LaunchOrder order(b);
+    CHK(batch_begin(b, trees, ntrees, order, &depth, &steps));
     std::vector<TreeRef> refs((size_t)ntrees);
     bool small_pools = true, ranges_miss = false;
     for (int i = 0; i < ntrees; ++i) {
@@ -2712,7 +2726,7 @@ int ikd_batch_nearest_search_device(ikd_batch_t b, const ikd_tree_t* trees, int 
         return IKD_ERR_UNSUPPORTED;
     }
     HIPCHK(hipGetLastError());
-    return batch_end(b, trees, ntrees);
+    return batch_end(b, trees, ntrees, order);
 }
 
 int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int ntrees,
@@ -2755,7 +2769,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
     int depth = 0;
     long long steps = 16;
     bool small_pools = true, ranges_miss = false;
-    std::vector<const BatchEvent*> waited;
+    LaunchOrder order(b);
     for (int i = 0; i < ntrees; ++i) {
         ikd_tree_t tr = trees[i];
         if (!tr) {
@@ -2773,7 +2787,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
         small_pools = small_pools && tr->cap <= (1ll << 24);
         ranges_miss = ranges_miss || tr->ranges_miss;
         tab.t[i] = TreeRef{tr->pool.hot, tr->pool.ids};
-        CHK(order_after_tree(b, tr, waited));
+        CHK(order_after_tree(b, tr, order));
     }
     hipLaunchKernelGGL(k_store_trees, dim3(1), dim3(IKD_NOALLOC_MAX_TREES), 0, b->st, tab, ntrees, table);
     launch_fill_i32(ctrl + 8, 0, 1, b->st);
@@ -2806,7 +2820,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
     }
     HIPCHK(hipGetLastError());
     b->na_flag = ctrl + 8;
-    return batch_end(b, trees, ntrees);
+    return batch_end(b, trees, ntrees, order);
 }
 
 // ------------------------------------------------------- recorded kNN launch
@@ -2953,7 +2967,7 @@ int ikd_batch_knn_graph_launch(ikd_knn_graph_t g) {
     g->table_pending = false;
     const int n = (int)g->trees.size();
     bool ranges_miss = false;
-    std::vector<const BatchEvent*> waited;
+    LaunchOrder order(b);
     for (int i = 0; i < n; ++i) {
         ikd_tree_t tr = g->trees[i];
         std::lock_guard<std::recursive_mutex> lk(tr->mu);
@@ -2963,13 +2977,13 @@ int ikd_batch_knn_graph_launch(ikd_knn_graph_t g) {
         }
         ranges_miss = ranges_miss || tr->ranges_miss;
         g->h_table[i] = TreeRef{tr->pool.hot, tr->pool.ids};
-        CHK(order_after_tree(b, tr, waited));
+        CHK(order_after_tree(b, tr, order));
     }
     HIPCHK(hipMemcpyAsync(g->d_table, g->h_table, n * sizeof(TreeRef), hipMemcpyHostToDevice, b->st));
     HIPCHK(hipEventRecord(g->ev_table, b->st));
     g->table_pending = true;
     HIPCHK(hipGraphLaunch(g->exec[ranges_miss && g->exec[1] ? 1 : 0], b->st));
-    return batch_end(b, g->trees.data(), n);
+    return batch_end(b, g->trees.data(), n, order);
 }
 
 int ikd_batch_knn_graph_destroy(ikd_knn_graph_t g) {
@@ -2997,7 +3011,8 @@ int ikd_batch_radius_search_device(ikd_batch_t b, const ikd_tree_t* trees, int n
     auto* t = b;
     int depth;
     long long steps;
-    CHK(batch_begin(b, trees, ntrees, &depth, &steps));
+    LaunchOrder order(b);
+    CHK(batch_begin(b, trees, ntrees, order, &depth, &steps));
     std::vector<Pool> pools((size_t)ntrees);
     for (int i = 0; i < ntrees; ++i) pools[i] = trees[i]->pool;
     Pool* d_pools;
@@ -3031,7 +3046,7 @@ int ikd_batch_radius_search_device(ikd_batch_t b, const ikd_tree_t* trees, int n
         launch_range_item_fill(a, ntask, a.item_offsets, b->st);
         HIPCHK(hipGetLastError());
     }
-    CHK(batch_end(b, trees, ntrees));
+    CHK(batch_end(b, trees, ntrees, order));
     if (d_out_xyz && capacity < total) {
         b->err = "batch: output capacity below the result count";
         return IKD_ERR_CAPACITY;

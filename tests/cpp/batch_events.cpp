@@ -26,13 +26,23 @@ hipError_t hipEventDestroy(hipEvent_t e) {
     --g_live_events;
     return hipSuccess;
 }
+static bool captured(hipStream_t s) {
+    hipStreamCaptureStatus st;
+    hipStreamIsCapturing(s, &st);
+    return st != hipStreamCaptureStatusNone;
+}
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+    if (captured(s)) {  // part of the graph: orders nothing outside
+        g_at[e].clear();
+        return hipSuccess;
+    }
     ++g_now[s][s];
     g_at[e] = g_now[s];
     return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
     ++g_waits;
+    if (captured(s)) return hipSuccess;
     for (auto& kv : g_at[e]) g_now[s][kv.first] = std::max(g_now[s][kv.first], kv.second);
     return hipSuccess;
 }
@@ -108,6 +118,43 @@ static int two_batches() {
     return 0;
 }
 
+// a launch that the caller captures from the batch's stream runs when the caller
+// replays it: the order of what runs now does not change
+static int captured_launch() {
+    ikd_tree_t t = make_tree();
+    ikd_batch_t b;
+    REQUIRE(t && ikd_batch_create(&b) == IKD_OK);
+    const hipStream_t bs = stream_of(b);
+    for (int round = 0; round < 2; ++round) {
+        REQUIRE(launch(b, &t, 1) == IKD_OK);
+        const long first = g_now[bs][bs];
+        hipGraph_t g = nullptr;
+        REQUIRE(hipStreamBeginCapture(bs, hipStreamCaptureModeThreadLocal) == hipSuccess);
+        REQUIRE(launch_noalloc(b, &t, 1) == IKD_OK);
+        REQUIRE(hipStreamEndCapture(bs, &g) == hipSuccess);
+        REQUIRE(hipGraphDestroy(g) == hipSuccess);
+        // the tree's next work is behind the launch before the capture
+        int32_t n = 0;
+        REQUIRE(ikd_add_points(t, g_q, nullptr, 3, 0, &n) == IKD_OK);
+        long most = 0;
+        for (auto& kv : g_now)
+            if (kv.first != bs) most = std::max(most, kv.second[bs]);
+        REQUIRE(most >= first);
+        // a launch after a captured one is behind the tree's work
+        REQUIRE(hipStreamBeginCapture(bs, hipStreamCaptureModeThreadLocal) == hipSuccess);
+        REQUIRE(launch_noalloc(b, &t, 1) == IKD_OK);
+        REQUIRE(hipStreamEndCapture(bs, &g) == hipSuccess);
+        REQUIRE(hipGraphDestroy(g) == hipSuccess);
+        const Clock before = g_now[bs];
+        REQUIRE(launch(b, &t, 1) == IKD_OK);
+        bool waited = false;
+        for (auto& kv : g_now[bs])
+            if (kv.first != bs) waited = waited || !before.count(kv.first) || kv.second > before.at(kv.first);
+        REQUIRE(waited);
+    }
+    return 0;
+}
+
 int main(int argc, char** argv) {
     unsigned x = 1;
     auto rnd = [&] {
@@ -120,6 +167,7 @@ int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     int rc = 2;
     if (!std::strcmp(what, "two_batches")) rc = two_batches();
+    if (!std::strcmp(what, "captured_launch")) rc = captured_launch();
     if (rc == 0) std::printf("ok\n");
     return rc;
 }

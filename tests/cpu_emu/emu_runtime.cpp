@@ -191,10 +191,16 @@ struct emu_graph_exec {
     std::vector<emu_node> nodes;
 };
 static thread_local emu_graph* t_capture = nullptr;
+static thread_local hipStream_t t_capture_stream = nullptr;
 
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) {
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* status) {
+    *status = t_capture && s == t_capture_stream ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
     if (t_capture) return hipErrorInvalidValue;
     t_capture = new emu_graph();
+    t_capture_stream = s;
     return hipSuccess;
 }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {

@@ -169,6 +169,9 @@ typedef emu_graph* hipGraph_t;
 typedef emu_graph_exec* hipGraphExec_t;
 enum hipStreamCaptureMode { hipStreamCaptureModeGlobal = 0, hipStreamCaptureModeThreadLocal = 1,
                             hipStreamCaptureModeRelaxed = 2 };
+enum hipStreamCaptureStatus { hipStreamCaptureStatusNone = 0, hipStreamCaptureStatusActive = 1,
+                              hipStreamCaptureStatusInvalidated = 2 };
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* status);
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode mode);
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g);
 hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, void* error_node, char* log, size_t log_size);
