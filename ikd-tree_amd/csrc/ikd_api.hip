@@ -237,6 +237,7 @@ struct Stager {
 // to wait for it.
 struct BatchEvent {
     hipEvent_t ev = nullptr;
+    std::atomic<bool> over{false};  // the batch is closed and its launches are done: nothing to wait for
     ~BatchEvent() {
         if (ev) hipEventDestroy(ev);
     }
@@ -389,7 +390,7 @@ hipMemPool_t library_pool(int dev) {
 int enter_tree(ikd_tree_t t) {
     t->work += 1;
     while (!t->after.empty()) {
-        HIPCHK(hipStreamWaitEvent(t->st, t->after.back()->ev, 0));
+        if (!t->after.back()->over) HIPCHK(hipStreamWaitEvent(t->st, t->after.back()->ev, 0));
         t->after.pop_back();
     }
     return IKD_OK;
@@ -2525,6 +2526,9 @@ static int order_after_tree(ikd_batch_t b, ikd_tree_t tr, LaunchOrder& order) {
     auto* t = b;
     if (order.captured) return IKD_OK;
     auto& waited = order.waited;
+    // a tree that is only searched keeps no event of a closed batch
+    tr->after.erase(std::remove_if(tr->after.begin(), tr->after.end(), [](const auto& e) { return e->over.load(); }),
+                    tr->after.end());
     for (const auto& e : tr->after) {
         if (e == b->done || std::find(waited.begin(), waited.end(), e.get()) != waited.end()) continue;
         HIPCHK(hipStreamWaitEvent(b->st, e->ev, 0));
@@ -2626,7 +2630,7 @@ int ikd_batch_destroy(ikd_batch_t b) {
     if (!b) return IKD_ERR_ARG;
     if (b->st) {
         for (auto& d : b->b) dev_free(b, d.p);
-        hipStreamSynchronize(b->st);
+        if (hipStreamSynchronize(b->st) == hipSuccess) b->done->over = true;
     }
     stage_release(b);
     if (b->h_count) hipHostFree(b->h_count);

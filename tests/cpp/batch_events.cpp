@@ -155,6 +155,29 @@ static int captured_launch() {
     return 0;
 }
 
+// a batch per request over a tree that is only searched: a closed batch leaves
+// nothing behind
+static int closed_batches() {
+    ikd_tree_t t = make_tree();
+    ikd_batch_t keep;
+    REQUIRE(t && ikd_batch_create(&keep) == IKD_OK && launch(keep, &t, 1) == IKD_OK);
+    const long events = g_live_events;
+    for (int i = 0; i < 50; ++i) {
+        ikd_batch_t b;
+        REQUIRE(ikd_batch_create(&b) == IKD_OK);
+        REQUIRE(launch(b, &t, 1) == IKD_OK && launch(keep, &t, 1) == IKD_OK);
+        REQUIRE(ikd_batch_destroy(b) == IKD_OK);
+        REQUIRE(g_live_events <= events + 1);
+    }
+    const long waits = g_waits;
+    int32_t n = 0;
+    REQUIRE(ikd_add_points(t, g_q, nullptr, 3, 0, &n) == IKD_OK);
+    REQUIRE(g_waits - waits <= 2);
+    REQUIRE(ikd_batch_destroy(keep) == IKD_OK && ikd_destroy(t) == IKD_OK);
+    REQUIRE(g_live_events == 0);
+    return 0;
+}
+
 int main(int argc, char** argv) {
     unsigned x = 1;
     auto rnd = [&] {
@@ -168,6 +191,7 @@ int main(int argc, char** argv) {
     int rc = 2;
     if (!std::strcmp(what, "two_batches")) rc = two_batches();
     if (!std::strcmp(what, "captured_launch")) rc = captured_launch();
+    if (!std::strcmp(what, "closed_batches")) rc = closed_batches();
     if (rc == 0) std::printf("ok\n");
     return rc;
 }

@@ -25,7 +25,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("scenario", ["two_batches", "captured_launch"])
+@pytest.mark.parametrize("scenario", ["two_batches", "captured_launch", "closed_batches"])
 def test_order_between_launches_and_trees(exe, scenario):
     r = subprocess.run([str(exe), scenario], capture_output=True, text=True, timeout=300,
                        env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
