@@ -275,7 +275,7 @@ struct RangeArgs {
     uint32_t* out_ids;
     int* overflow;
     long long max_steps;
-    int stack;            // item walks: LDS stack entries per lane (>= tree depth + 2)
+    int stack;            // walks of one lane: LDS stack entries (>= tree depth + 2)
     const Pool* pools;    // multi-tree launch: pool table with qtree[q] per query (else null)
     const int* qtree;
     int ntrees;           // a query naming no valid tree finds nothing
@@ -291,6 +291,9 @@ struct RangeArgs {
     int4* tasks;
     const long long* item_offsets;
 };
+// Above this many queries one lane walks each, below a wavefront.
+constexpr int RANGE_WAVES_MAX = 1 << 15;
+inline bool range_by_lanes(int nq) { return nq > RANGE_WAVES_MAX; }
 // list 0: tcounts[q] = items of query q, the first of them kept in raw; list 1: the items at toffsets[q]
 void launch_range_top(const RangeArgs& a, int list, hipStream_t s);
 // counts[i] = points of item i

@@ -983,7 +983,8 @@ __device__ __forceinline__ int classify(const RangeArgs& a, int qi, const float*
     return 2;
 }
 
-// Range search in items.  One wavefront walks each query; the walk goes down
+// Range search in items.  One wavefront (one lane, when there are very many
+// queries) walks each query; the walk goes down
 // only through subtrees of more than task_nodes nodes, and everything at or
 // below that size, and the own point of every node it walks, becomes an item
 // of the query's list, in pre-order:
@@ -1073,11 +1074,11 @@ __device__ __forceinline__ int4 range_item_of(int e, int qi) {
                      0);
 }
 
-__global__ __launch_bounds__(64) void k_range_top(RangeArgs a, int list, int qbase) {
+__global__ __launch_bounds__(64) void k_range_top(RangeArgs a, int list) {
     extern __shared__ int lds_dyn[];
     int* stk = lds_dyn;
     const int lane = threadIdx.x;
-    const int qi = qbase + (int)blockIdx.x;
+    const int qi = blockIdx.x;
     bool ok;
     const Pool P = range_pool(a, qi, &ok);
     if (!ok) {
@@ -1188,6 +1189,94 @@ __global__ __launch_bounds__(64) void k_range_top(RangeArgs a, int list, int qba
     if (!list && lane == 0) a.tcounts[qi] = items;
 }
 
+// One lane per query, depth-first: the items of the same walk in the same order
+// (stack entries as [stack][64] in LDS), for launches of more than RANGE_WAVES_MAX
+// queries.  Those fill the device with lanes, and a walk to a small ball has a
+// frontier of a few nodes, so a wavefront per query leaves most of its lanes idle:
+// 1M balls of 0.05 m on a LiDAR map of 1M points take 5109 us with it and 810 with
+// lanes, 80k 472 and 250; 10k, whose lanes would not fill the device, 157 and 208,
+// and 20k balls of 1 m 685 and 890.  The two cross between 20k and 60k queries.
+__global__ __launch_bounds__(64) void k_range_top_lanes(RangeArgs a, int list) {
+    extern __shared__ int lds_dyn[];
+    int* stk = lds_dyn;
+    const int lane = threadIdx.x;
+    const int qi = blockIdx.x * 64 + lane;
+    if (qi >= a.nq) return;
+    bool ok;
+    const Pool P = range_pool(a, qi, &ok);
+    if (!ok) {
+        if (!list) a.tcounts[qi] = 0;
+        return;
+    }
+    int* const raw = a.raw + (size_t)qi * a.raw_cap;
+    int4* dst = nullptr;
+    long long cap = a.raw_cap;
+    if (list) {
+        dst = a.tasks + a.toffsets[qi];
+        cap = a.toffsets[qi + 1] - a.toffsets[qi];
+        if (cap <= a.raw_cap) {
+            for (int i = 0; i < (int)cap; ++i) dst[i] = range_item_of(raw[i], qi);
+            return;
+        }
+    }
+    const NodeHot* __restrict__ hot = P.hot;
+    const int G = a.task_nodes;
+    const RangeQuery q = range_query(a, qi);
+    long long items = 0;
+    auto item = [&](int e) {
+        if (list) {
+            if (items < cap) dst[items] = range_item_of(e, qi);
+            else atomicOr(a.overflow, 8);  // more items than the first walk counted
+        } else if (items < cap) {
+            raw[items] = e;
+        }
+        ++items;
+    };
+    // the entry of node c of class cls (1 covered, 2 cut)
+    auto entry = [&](int c, int cls) -> int {
+        if (P.cnt[c].x <= G) return c | RANGE_TASK | (cls == 2 ? RANGE_CUT : 0);
+        return c | (cls == 1 ? RANGE_WHOLE : 0);
+    };
+    int sp = 0;
+    const uint32_t lk0 = fbits(hot[SENTINEL].f[3]);
+    if ((lk0 & LK_HASL) && !(lk0 & LK_TDL)) {
+        const int c0 = classify(a, qi, hot[SENTINEL].f + 4, q.qx, q.qy, q.qz, q.r);
+        if (c0 != 0) {
+            stk[lane] = entry(ROOT, c0);
+            sp = 1;
+        }
+    }
+    long long steps = 0;
+    while (sp > 0) {
+        if (++steps > a.max_steps) {
+            atomicOr(a.overflow, 8);
+            break;
+        }
+        const int e = stk[--sp * 64 + lane];
+        if (e & RANGE_TASK) {
+            item(e);
+            continue;
+        }
+        const int u = e & RANGE_NODE;
+        const bool whole = (e & RANGE_WHOLE) != 0;
+        float f[16];
+        load_record(hot[u].f, f);
+        const uint32_t lk = fbits(f[3]);
+        if (!(lk & LK_PDEL) && (whole || range_takes(a, qi, q, f))) item(u | RANGE_TASK | RANGE_WHOLE);
+        const int pair = (int)lk_pair(lk);
+#pragma unroll
+        for (int s = 1; s >= 0; --s) {
+            if (!(lk & lk_has(s)) || (lk & lk_td(s))) continue;
+            const int c = 2 * pair + s;
+            const int cls = whole ? 1 : classify(a, qi, f + 4 + 6 * s, q.qx, q.qy, q.qz, q.r);
+            if (cls == 0) continue;
+            if (sp < a.stack) stk[sp++ * 64 + lane] = entry(c, cls);
+            else atomicOr(a.overflow, 8);
+        }
+    }
+    if (!list) a.tcounts[qi] = items;
+}
+
 // The points one item holds: counted (fill false) or written from pos on in
 // pre-order (fill true, at most lim).  Returns the count / the end position.
 __device__ long long range_item(const RangeArgs& a, const Pool& P, int qi, int u, int kind, int* stk, int lane,
@@ -1287,14 +1376,16 @@ __global__ __launch_bounds__(64) void k_range_item_fill(RangeArgs a, long long n
 
 void launch_range_top(const RangeArgs& a, int list, hipStream_t s) {
     if (a.nq <= 0) return;
+    if (range_by_lanes(a.nq)) {
+        hipLaunchKernelGGL(k_range_top_lanes, dim3(blocks_for(a.nq, 64)), dim3(64), (size_t)a.stack * 64 * sizeof(int),
+                           s, a, list);
+        return;
+    }
     // 16 KB of stack a wavefront while the queries do not fill the device (the
     // widest frontiers then still go 64 at a time), 4 KB when occupancy counts
     RangeArgs b = a;
     b.stack = a.nq <= RANGE_FEW_QUERIES ? 4096 : 1024;
-    constexpr int STEP = 1 << 25;  // a grid holds fewer than 2^32 lanes
-    for (int q0 = 0; q0 < a.nq; q0 += std::min(STEP, a.nq - q0))
-        hipLaunchKernelGGL(k_range_top, dim3(std::min(STEP, a.nq - q0)), dim3(64), (size_t)b.stack * sizeof(int), s, b,
-                           list, q0);
+    hipLaunchKernelGGL(k_range_top, dim3(a.nq), dim3(64), (size_t)b.stack * sizeof(int), s, b, list);
 }
 void launch_range_item_count(const RangeArgs& a, long long ntask, long long* counts, hipStream_t s) {
     if (ntask <= 0) return;

@@ -36,6 +36,8 @@ def test_noalloc_launches_of_two_batches():
         qt = torch.from_numpy(rng.integers(0, len(tl), nq).astype(np.int32)).to(dev)
         md = torch.from_numpy(rng.choice(np.array([1.0, 4.0, np.inf]), nq)).to(dev)
         calls.append((tl, qt, q, md, _outs(torch, nq, k, dev), _outs(torch, nq, k, dev)))
+    if dev.type == "cuda":
+        torch.cuda.synchronize()  # batches have streams of their own
     one = ikd.Batch()
     for tl, qt, q, md, want, _ in calls:  # everything waited for
         one.nearest_search_device(tl, qt, q, k, *want, max_dist=md)
