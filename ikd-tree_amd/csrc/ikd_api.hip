@@ -783,7 +783,9 @@ int run_build(ikd_tree_t t, const float4* pts, const int* seg_of, int m, const i
     CHK(ensure(t, B_SEGLR, segcap, &seglr));
     const long long words = ((long long)m + 63) / 64;
     CHK(ensure(t, B_BITS, 6 * words, &bits));
-    CHK(ensure(t, B_TILELR, 3 * build_tiles(m), &tilelr));
+    const long long tiles = 3 * build_tiles(m);
+    const bool scanned = build_tiles_scanned(m);
+    CHK(ensure(t, B_TILELR, (scanned ? 2 : 1) * tiles, &tilelr));
 
     const int end_bit = 32 + bits_for(S);
     if (m <= RANK_SORT_MAX) {
@@ -850,6 +852,7 @@ int run_build(ikd_tree_t t, const float4* pts, const int* seg_of, int m, const i
         BL.bits_l = bits;
         BL.bits_r = bits + 3 * words;
         BL.tile_lr = tilelr;
+        BL.tile_pre = scanned ? tilelr + tiles : nullptr;
         BL.m = m;
         BL.cur = cur;
         if (build_seg_one_fits((int)bound)) {
@@ -861,7 +864,11 @@ int run_build(ikd_tree_t t, const float4* pts, const int* seg_of, int m, const i
             launch_build_seg_b(BL, (int)bound, t->pool, t->d_hdr, st);
         }
         launch_build_side(BL, t->d_hdr, st);
-        if (L + 1 < levels) launch_build_partition(BL, st);
+        if (L + 1 < levels) {
+            launch_build_bits(BL, st);
+            if (scanned) CHK(exscan_u64(t, BL.tile_lr, BL.tile_pre, (int)tiles));
+            launch_build_scatter(BL, st);
+        }
     }
     if (Ls < levels) {
         // level Ls: its segments (count on the device) and its x-ordered list

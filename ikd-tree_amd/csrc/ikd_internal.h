@@ -80,6 +80,7 @@ struct BuildLevel {
     unsigned long long* bits_l;     // 3 lists of ceil(m / 64) words: positions that go left
     unsigned long long* bits_r;     // and right
     unsigned long long* tile_lr;    // 3 lists of build_tiles(m): lefts | rights<<32 of a tile
+    unsigned long long* tile_pre;   // their exclusive scan where build_tiles_scanned(m), else null
     int m;
     int cur;               // 0/1: which DevHdr::seg_count holds this level's count
 };
@@ -104,7 +105,10 @@ void launch_build_side(const BuildLevel& L, DevHdr* hdr, hipStream_t s);
 bool build_seg_one_fits(int bound);
 void launch_build_seg_one(const BuildLevel& L, Pool pool, DevHdr* hdr, hipStream_t s);
 long long build_tiles(long long m);
-void launch_build_partition(const BuildLevel& L, hipStream_t s);
+bool build_tiles_scanned(long long m);
+// a level's partition: bits, the scan of tile_lr where it is asked for, scatter
+void launch_build_bits(const BuildLevel& L, hipStream_t s);
+void launch_build_scatter(const BuildLevel& L, hipStream_t s);
 
 // Presorted lists for the small build (all null: the kernel sorts): the
 // segments' y- and z-ordered lists of point indices (list1, list2) and, for
