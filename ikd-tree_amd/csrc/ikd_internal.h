@@ -251,6 +251,9 @@ struct KnnArgs {
     // one-lane launches: 4-byte LDS stack entries (every tree of the launch
     // has at most 2^24 node slots)
     int compact_stack;
+    // one-lane launches over a tree whose stored ranges may miss points: deferred
+    // children keep their exact box distance
+    int exact_stack;
 };
 // Copies the tree's first `levels` levels into a complete binary layout (slot 0
 // the root, slot s's children at 2s+1 and 2s+2): top[s] the node's record,

@@ -272,6 +272,14 @@ __device__ __forceinline__ uint32_t compact_entry(int n, float d) {
 __device__ __forceinline__ float compact_dist(uint32_t e) { return bitsf((e & 0xffu) << 23); }
 static inline size_t lds_compact_bytes(int stack) { return (size_t)stack * 64 * sizeof(uint32_t); }
 
+// Exact stacks (trees whose stored ranges may miss points below them,
+// KnnArgs::exact_stack): node index and the 32-bit distance.  There a subtree
+// that a rounded distance admits may hold points nearer than its box, which the
+// reference, comparing the exact distance, leaves out; 64 entries of a lane take
+// 32 KB, so such launches run fewer wavefronts on deep trees.
+enum StackForm { STACK_KEY16 = 0, STACK_COMPACT = 1, STACK_EXACT = 2 };
+static inline size_t lds_exact_bytes(int stack) { return (size_t)stack * 64 * (sizeof(int) + sizeof(float)); }
+
 // The node a lane starts at: the root, if it is live and within the bound.
 __device__ __forceinline__ int knn_root(const QueryCtx& c) {
     const uint32_t lk0 = fbits(c.hot[SENTINEL].f[3]);
@@ -282,21 +290,33 @@ __device__ __forceinline__ int knn_root(const QueryCtx& c) {
 // The lane's next deferred child that can still improve (-1: none left).
 // Entries were within max_dist's threshold when they were pushed, and a stored
 // distance never exceeds the exact one.
-template <bool COMPACT>
+template <int FORM>
+__device__ __forceinline__ void knn_push(const LdsStack& st, uint32_t* cst, int at, int n, float d) {
+    if (FORM == STACK_COMPACT) {
+        cst[at] = compact_entry(n, d);
+    } else {
+        st.n[at] = n;
+        if (FORM == STACK_EXACT) reinterpret_cast<float*>(st.d)[at] = d;
+        else st.d[at] = dist_key(d);
+    }
+}
+template <int FORM>
 __device__ __forceinline__ int knn_pop(const LdsStack& st, const uint32_t* cst, int lane, int& sp, float kth) {
     while (sp > 0) {
         --sp;
-        if (COMPACT) {
-            const uint32_t e = cst[sp * 64 + lane];
+        const int at = sp * 64 + lane;
+        if (FORM == STACK_COMPACT) {
+            const uint32_t e = cst[at];
             if (compact_dist(e) <= kth) return (int)(e >> 8);
         } else {
-            if (dist_val(st.d[sp * 64 + lane]) <= kth) return st.n[sp * 64 + lane];
+            const float d = FORM == STACK_EXACT ? reinterpret_cast<const float*>(st.d)[at] : dist_val(st.d[at]);
+            if (d <= kth) return st.n[at];
         }
     }
     return -1;
 }
 
-template <int KM, bool COMPACT, bool COUNT>
+template <int KM, int FORM, bool COUNT>
 __global__ __launch_bounds__(64) void k_knn(KnnArgs a) {
     const LdsStack st = lds_stack(a.stack);
     extern __shared__ int lds_dyn[];
@@ -320,12 +340,7 @@ __global__ __launch_bounds__(64) void k_knn(KnnArgs a) {
         visit_node<KM, COUNT>(c, best, n, c.thr, lim, nn, dn, fn, df, boxes);
         if (fn >= 0) {
             if (sp < a.stack) {
-                if (COMPACT) {
-                    cst[sp * 64 + lane] = compact_entry(fn, df);
-                } else {
-                    st.n[sp * 64 + lane] = fn;
-                    st.d[sp * 64 + lane] = dist_key(df);
-                }
+                knn_push<FORM>(st, cst, sp * 64 + lane, fn, df);
                 ++sp;
             } else {
                 atomicOr(a.overflow, 1);
@@ -337,7 +352,7 @@ __global__ __launch_bounds__(64) void k_knn(KnnArgs a) {
             sp = 0;
             n = -1;
         }
-        if (n < 0) n = knn_pop<COMPACT>(st, cst, lane, sp, best.d[0]);
+        if (n < 0) n = knn_pop<FORM>(st, cst, lane, sp, best.d[0]);
     }
 
     finish_query<KM>(a, c, best, visits, boxes);
@@ -762,12 +777,7 @@ __global__ __launch_bounds__(64) void k_knn_persist(KnnArgs a, int* __restrict__
             visit_node<KM, true>(c, best, n, c.thr, lim, nn, dn, fn, df, boxes);
             if (fn >= 0) {
                 if (sp < a.stack) {
-                    if (COMPACT) {
-                        cst[sp * 64 + lane] = compact_entry(fn, df);
-                    } else {
-                        st.n[sp * 64 + lane] = fn;
-                        st.d[sp * 64 + lane] = dist_key(df);
-                    }
+                    knn_push<COMPACT ? STACK_COMPACT : STACK_KEY16>(st, cst, sp * 64 + lane, fn, df);
                     ++sp;
                 } else {
                     atomicOr(a.overflow, 1);
@@ -776,7 +786,7 @@ __global__ __launch_bounds__(64) void k_knn_persist(KnnArgs a, int* __restrict__
             n = nn;
             if (n >= 0) continue;
         }
-        n = knn_pop<COMPACT>(st, cst, lane, sp, best.d[0]);
+        n = knn_pop<COMPACT ? STACK_COMPACT : STACK_KEY16>(st, cst, lane, sp, best.d[0]);
         if (n >= 0) continue;
         finish_query<KM>(a, c, best, visits, boxes);
         has = false;
@@ -805,15 +815,20 @@ static int launch_knn_km(const KnnArgs& a0, int lanes, int stack, hipStream_t s,
     dim3 block(64);
     a.stack = stack;
     const size_t lds = lds_stack_bytes(stack);
+    const dim3 grid(xcd_grid(blocks_for(a.nq, 64)));
     switch (lanes) {
         case 1:
             if (a.top_slots > 0 && a.top && !a.trees) {
                 const size_t lds_t = lds_stack_bytes16(stack) + lds_top_bytes(a.top_slots);
-                hipLaunchKernelGGL((k_knn_staged<KM>), dim3(xcd_grid(blocks_for(a.nq, 64))), block, lds_t, s, a);
+                hipLaunchKernelGGL((k_knn_staged<KM>), grid, block, lds_t, s, a);
                 return 0;
             }
             if (a.visits) {
-                hipLaunchKernelGGL((k_knn<KM, false, true>), dim3(xcd_grid(blocks_for(a.nq, 64))), block, lds, s, a);
+                hipLaunchKernelGGL((k_knn<KM, STACK_KEY16, true>), grid, block, lds, s, a);
+                return 0;
+            }
+            if (a.exact_stack) {
+                hipLaunchKernelGGL((k_knn<KM, STACK_EXACT, false>), grid, block, lds_exact_bytes(stack), s, a);
                 return 0;
             }
             if (a.compact_stack) {
@@ -822,11 +837,10 @@ static int launch_knn_km(const KnnArgs& a0, int lanes, int stack, hipStream_t s,
                 // queries each, k = 5) evict each other's nodes from L2, 446 us a launch
                 // against 433; one map alone takes 447 against 452.
                 const size_t lb = lds_compact_bytes(std::max(stack, KNN_STACK_FLOOR));
-                hipLaunchKernelGGL((k_knn<KM, true, false>), dim3(xcd_grid(blocks_for(a.nq, 64))), block,
-                                   lb, s, a);
+                hipLaunchKernelGGL((k_knn<KM, STACK_COMPACT, false>), grid, block, lb, s, a);
                 return 0;
             }
-            hipLaunchKernelGGL((k_knn<KM, false, false>), dim3(xcd_grid(blocks_for(a.nq, 64))), block, lds, s, a);
+            hipLaunchKernelGGL((k_knn<KM, STACK_KEY16, false>), grid, block, lds, s, a);
             return 0;
         case 0: {  // persistent lanes; the 8 per-XCD query counters were zeroed by the caller
             // as many single-wavefront workgroups as the LDS stacks let each CU hold
