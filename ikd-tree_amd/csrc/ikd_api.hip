@@ -908,7 +908,8 @@ constexpr long long ENUM_GROUP_ROOT_MAX = 16384;
 // ones: more items than a lane keeps cost it a second walk, and there are items
 // enough (80k balls of 1 m on a 1M LiDAR map: items of 32 nodes 3061 us, 64 2640,
 // 128 2462, 256 2407; balls of 0.3 m 649, 551, 555, 653).
-constexpr int RANGE_TASK_NODES = 32, RANGE_TASK_NODES_LANES = 128;
+// More than INT_MAX - 1 items take larger ones (an item is 32 bytes of scratch).
+constexpr int RANGE_TASK_NODES = 32, RANGE_TASK_NODES_LANES = 128, RANGE_TASK_NODES_MOST = 256;
 // Items the first walk of a range search keeps for all queries together (16 MB):
 // 200 boxes keep up to 20k each, half a million balls 7.
 constexpr int RANGE_RAW_ITEMS = 1 << 22;
@@ -1684,12 +1685,17 @@ int range_plan(Owner* t, RangeArgs& a, int nq, long long* d_offsets, const int (
     a.tcounts = tcnt;
     a.raw_cap = (int)std::max<long long>(1, std::min<long long>(pool_bound, RANGE_RAW_ITEMS / nq));
     CHK(ensure(t, slots[5], (long long)nq * a.raw_cap, &a.raw));
-    launch_range_top(a, 0, st);
-    CHK(exscan_i64(t, tcnt, toff, nq + 1));
-    hipLaunchKernelGGL(k_publish_count, dim3(1), dim3(1), 0, st, toff + nq, t->h_count);
-    HIPCHK(hipGetLastError());
-    HIPCHK(owner_wait(t));
-    const long long ntask = *t->h_count;
+    long long ntask;
+    while (true) {
+        launch_range_top(a, 0, st);
+        CHK(exscan_i64(t, tcnt, toff, nq + 1));
+        hipLaunchKernelGGL(k_publish_count, dim3(1), dim3(1), 0, st, toff + nq, t->h_count);
+        HIPCHK(hipGetLastError());
+        HIPCHK(owner_wait(t));
+        ntask = *t->h_count;
+        if (ntask < INT_MAX || a.task_nodes >= RANGE_TASK_NODES_MOST) break;
+        a.task_nodes = RANGE_TASK_NODES_MOST;
+    }
     CHK(check_count(t, "range search: items", ntask, 0, std::min<long long>((long long)nq * pool_bound, INT_MAX - 1)));
     CHK(ensure(t, slots[2], std::max<long long>(ntask, 1), &items));
     CHK(ensure(t, slots[3], ntask + 1, &icnt));
