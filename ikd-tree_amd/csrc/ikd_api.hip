@@ -1617,6 +1617,7 @@ int knn_dev(ikd_tree_t t, const float* d_q, int nq, int k, double max_dist, floa
     a.boxes = d_boxes;
     a.overflow = &t->d_hdr->overflow;
     a.max_steps = (int)std::min<long long>(t->pool_used + 16, INT_MAX);
+    a.nodes = t->pool_used;
     a.compact_stack = (t->knn_compact && t->cap <= (1ll << 24)) ? 1 : 0;
     a.exact_stack = t->ranges_miss ? 1 : 0;
     if (t->query_order && nq >= 4096) {
@@ -2711,8 +2712,10 @@ int ikd_batch_nearest_search_device(ikd_batch_t b, const ikd_tree_t* trees, int 
     CHK(batch_begin(b, trees, ntrees, order, &depth, &steps));
     std::vector<TreeRef> refs((size_t)ntrees);
     bool small_pools = true, ranges_miss = false;
+    long long nodes = 0;
     for (int i = 0; i < ntrees; ++i) {
         ranges_miss = ranges_miss || trees[i]->ranges_miss;
+        nodes += trees[i]->pool_used;
         refs[i] = TreeRef{trees[i]->pool.hot, trees[i]->pool.ids};
         small_pools = small_pools && trees[i]->cap <= (1ll << 24);
     }
@@ -2746,6 +2749,7 @@ int ikd_batch_nearest_search_device(ikd_batch_t b, const ikd_tree_t* trees, int 
     a.out_counts = d_out_counts;
     a.overflow = flag;
     a.max_steps = (int)std::min<long long>(steps, INT_MAX);
+    a.nodes = nodes;
     int stack = std::min(std::max(depth + 2, b->knn_stack), MAX_DEPTH);
     const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq), ranges_miss);
     if (launch_knn(a, k_max, lanes, stack, b->st, next, 256 * 10) != 0) {
@@ -2796,6 +2800,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
     int depth = 0;
     long long steps = 16;
     bool small_pools = true, ranges_miss = false;
+    long long nodes = 0;
     LaunchOrder order(b);
     for (int i = 0; i < ntrees; ++i) {
         ikd_tree_t tr = trees[i];
@@ -2813,6 +2818,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
         steps = std::max(steps, tr->pool_used + 16);
         small_pools = small_pools && tr->cap <= (1ll << 24);
         ranges_miss = ranges_miss || tr->ranges_miss;
+        nodes += tr->pool_used;
         tab.t[i] = TreeRef{tr->pool.hot, tr->pool.ids};
         CHK(order_after_tree(b, tr, order));
     }
@@ -2840,6 +2846,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
     a.out_counts = d_out_counts;
     a.overflow = ctrl + 8;
     a.max_steps = (int)std::min<long long>(steps, INT_MAX);
+    a.nodes = nodes;
     const int stack = std::min(std::max(depth + 2, b->knn_stack), MAX_DEPTH);
     const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq), ranges_miss);
     if (launch_knn(a, k_max, lanes, stack, b->st, ctrl, 256 * 10) != 0) {

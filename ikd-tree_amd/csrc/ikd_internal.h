@@ -241,6 +241,7 @@ struct KnnArgs {
     unsigned int* visits;   // optional instrumentation: visited nodes per query
     unsigned int* boxes;    // optional: child boxes evaluated per query
     int* overflow;
+    long long nodes;        // node slots of the trees searched, 0: not known
     int max_steps;          // visit bound per query (the pool size): a corrupt tree cannot hang a lane
     int stack;              // LDS stack entries per lane (set by launch_knn)
     // optional, one-lane single-tree launches: the tree's top levels staged in

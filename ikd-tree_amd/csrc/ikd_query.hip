@@ -806,7 +806,19 @@ static int device_cus() {
     return v;
 }
 
+// Compact stacks of at least KNN_STACK_FLOOR entries hold a CU at 24 wavefronts
+// where a balanced tree of a few million points would let it have 28.  With 28,
+// walks whose node records outgrow the caches evict each other's: launches over
+// three LiDAR maps in turn, queued without waits (k = 5, 24 against 28, us):
+// 2M points each, 1.18M queries 520 and 529, 3M queries 1040 and 1051; 4M points
+// 612 and 625, 1212 and 1236; 1M points, 1.18M queries 437 and 437; 300k points,
+// 3M queries 732 and 701.  And a launch that 28 a CU would take at once must not
+// be cut in two: 400k queries of a 1M map 258 and 222, of 300k points 195 and 158.
 constexpr int KNN_STACK_FLOOR = 26;
+constexpr long long KNN_WIDE_NODES = 1500000;  // 96 MB of records
+static bool knn_fewer_waves(const KnnArgs& a) {
+    return a.nodes >= KNN_WIDE_NODES && blocks_for(a.nq, 64) > 28 * device_cus();
+}
 
 template <int KM>
 static int launch_knn_km(const KnnArgs& a0, int lanes, int stack, hipStream_t s, int* persist_next,
@@ -832,11 +844,7 @@ static int launch_knn_km(const KnnArgs& a0, int lanes, int stack, hipStream_t s,
                 return 0;
             }
             if (a.compact_stack) {
-                // At least KNN_STACK_FLOOR entries of LDS, so that a CU holds at most 24
-                // wavefronts: with 28 the walks of three 2M-point maps in turn (1.18M
-                // queries each, k = 5) evict each other's nodes from L2, 446 us a launch
-                // against 433; one map alone takes 447 against 452.
-                const size_t lb = lds_compact_bytes(std::max(stack, KNN_STACK_FLOOR));
+                const size_t lb = lds_compact_bytes(knn_fewer_waves(a) ? std::max(stack, KNN_STACK_FLOOR) : stack);
                 hipLaunchKernelGGL((k_knn<KM, STACK_COMPACT, false>), grid, block, lb, s, a);
                 return 0;
             }
