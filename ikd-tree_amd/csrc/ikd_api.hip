@@ -1561,10 +1561,22 @@ int add_points_dev(ikd_tree_t t, const float* d_xyz, const uint32_t* d_ids, int 
 // 68/59/70/105/100, 40k 101/84/80/114/127, 80k 163/119/110/125/131, 160k
 // 292/196/158/162/142; the same side wins for k = 1, 10 and 20 and in
 // multi-map launches.
-int auto_lanes(int nq) {
+//
+// Teams of 4 fill the device at 73728 queries (18 wavefronts a CU of 8 KB deques);
+// above, on maps whose walks are long, the rest waits for a second turn, and two
+// lanes or one are ahead (us, lanes 4 / 2 / 1; 300k uniform points, 131k queries:
+// k = 1 97/74/85, k = 5 173/127/132, k = 20 460/432/423; 1M LiDAR points, 100k
+// queries: 73/66/87, 134/116/127, 338/399/292).  One lane is ahead of 4 only from
+// about 90k queries on (1M LiDAR points, 78k queries, k = 7 138/141/147), and maps
+// of up to 100k points are not slower with 4 (20k points, 100k queries: 49/52/58,
+// 91/92/85, 235/346/238).
+int auto_lanes(int nq, int k, long long nodes) {
     if (nq <= (1 << 14)) return 16;
     if (nq <= (1 << 15)) return 8;
-    return nq < (1 << 17) ? 4 : 1;
+    if (nq >= (1 << 17)) return 1;
+    if (nq <= (9 << 13) || nodes <= (1 << 17)) return 4;
+    if (k <= 5) return 2;
+    return nq <= (11 << 13) ? 4 : 1;
 }
 
 // Lanes per query for a launch that was to take `lanes`.  Where a stored range
@@ -1635,7 +1647,7 @@ int knn_dev(ikd_tree_t t, const float* d_q, int nq, int k, double max_dist, floa
     int stack = t->max_depth + 2;
     if (t->knn_stack > stack) stack = t->knn_stack;
     if (stack > MAX_DEPTH) stack = MAX_DEPTH;
-    const int lanes = knn_lanes_for(t->knn_lanes >= 0 ? t->knn_lanes : auto_lanes(nq), t->ranges_miss);
+    const int lanes = knn_lanes_for(t->knn_lanes >= 0 ? t->knn_lanes : auto_lanes(nq, k, t->pool_used), t->ranges_miss);
     if (t->knn_stage > 0 && lanes == 1 && !t->ranges_miss) {
         // the staged levels, capped so that one workgroup's LDS (stacks and
         // table) stays within 64 KiB
@@ -2751,7 +2763,7 @@ int ikd_batch_nearest_search_device(ikd_batch_t b, const ikd_tree_t* trees, int 
     a.max_steps = (int)std::min<long long>(steps, INT_MAX);
     a.nodes = nodes;
     int stack = std::min(std::max(depth + 2, b->knn_stack), MAX_DEPTH);
-    const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq), ranges_miss);
+    const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq, k_max, nodes), ranges_miss);
     if (launch_knn(a, k_max, lanes, stack, b->st, next, 256 * 10) != 0) {
         b->err = "batch: unsupported launch shape";
         return IKD_ERR_UNSUPPORTED;
@@ -2848,7 +2860,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
     a.max_steps = (int)std::min<long long>(steps, INT_MAX);
     a.nodes = nodes;
     const int stack = std::min(std::max(depth + 2, b->knn_stack), MAX_DEPTH);
-    const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq), ranges_miss);
+    const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq, k_max, nodes), ranges_miss);
     if (launch_knn(a, k_max, lanes, stack, b->st, ctrl, 256 * 10) != 0) {
         b->err = "batch (no-alloc): unsupported launch shape";
         return IKD_ERR_UNSUPPORTED;
@@ -2920,6 +2932,7 @@ int ikd_batch_knn_graph_create(ikd_batch_t b, const ikd_tree_t* trees, int ntree
         return IKD_ERR_ARG;
     }
     int depth = 0;
+    long long nodes = 0;
     for (int i = 0; i < ntrees; ++i) {
         if (!trees[i]) {
             b->err = "recorded kNN: null tree handle";
@@ -2931,6 +2944,7 @@ int ikd_batch_knn_graph_create(ikd_batch_t b, const ikd_tree_t* trees, int ntree
             return IKD_ERR_UNSUPPORTED;
         }
         depth = std::max(depth, trees[i]->max_depth);
+        nodes += trees[i]->pool_used;
     }
     ikd_knn_graph_t g = new ikd_knn_graph_s();
     g->b = b;
@@ -2966,7 +2980,7 @@ int ikd_batch_knn_graph_create(ikd_batch_t b, const ikd_tree_t* trees, int ntree
     // the visit bound only stops a walk on a corrupt tree; the recording must
     // outlive the trees' growth
     a.max_steps = 1 << 30;
-    const int lanes = b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq);
+    const int lanes = b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq, k_max, nodes);
     for (int v = 0; v < 2; ++v) {
         a.exact_stack = v;
         if (hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal) != hipSuccess) {
