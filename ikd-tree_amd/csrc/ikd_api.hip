@@ -1574,7 +1574,7 @@ int auto_lanes(int nq, int k, long long nodes) {
     if (nq <= (1 << 14)) return 16;
     if (nq <= (1 << 15)) return 8;
     if (nq >= (1 << 17)) return 1;
-    if (nq <= (9 << 13) || nodes <= (1 << 17)) return 4;
+    if (nq <= (9 << 13) || nodes <= (3 << 16)) return 4;  // slots: about 4 for 3 points
     if (k <= 5) return 2;
     return nq <= (11 << 13) ? 4 : 1;
 }

@@ -1,5 +1,5 @@
 """GPU: kNN launches around the sizes where the lanes per query change on a map of
-more than 2^17 nodes (73728 and 90112 queries, k 5 and 6): the bits of one lane per query,
+more than 3 * 2^16 node slots (73728 and 90112 queries, k 5 and 6): the bits of one lane per query,
 from the tree, a batch and a recorded launch."""
 import importlib
 
@@ -18,7 +18,7 @@ def test_lanes_above_a_full_device(k):
     dev = torch.device("cuda" if torch.cuda.is_available() else "cpu")
     rng = np.random.default_rng(k)
     t = ikd.KD_TREE(0.5, 0.6, 0.5)
-    t.Build(uniform_cloud(rng, 140000))
+    t.Build(uniform_cloud(rng, 200000))
     b = ikd.Batch()
     for nq in (73728, 73729, 90112, 90113):
         q = torch.from_numpy(uniform_cloud(rng, nq)).to(dev)
