@@ -1570,6 +1570,7 @@ int add_points_dev(ikd_tree_t t, const float* d_xyz, const uint32_t* d_ids, int 
 // about 90k queries on (1M LiDAR points, 78k queries, k = 7 138/141/147), and maps
 // of up to 100k points are not slower with 4 (20k points, 100k queries: 49/52/58,
 // 91/92/85, 235/346/238).
+// nodes: slots of the largest map (the walks of many small ones are short).
 int auto_lanes(int nq, int k, long long nodes) {
     if (nq <= (1 << 14)) return 16;
     if (nq <= (1 << 15)) return 8;
@@ -2763,7 +2764,7 @@ int ikd_batch_nearest_search_device(ikd_batch_t b, const ikd_tree_t* trees, int 
     a.max_steps = (int)std::min<long long>(steps, INT_MAX);
     a.nodes = nodes;
     int stack = std::min(std::max(depth + 2, b->knn_stack), MAX_DEPTH);
-    const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq, k_max, nodes), ranges_miss);
+    const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq, k_max, steps), ranges_miss);
     if (launch_knn(a, k_max, lanes, stack, b->st, next, 256 * 10) != 0) {
         b->err = "batch: unsupported launch shape";
         return IKD_ERR_UNSUPPORTED;
@@ -2860,7 +2861,7 @@ int ikd_batch_nearest_search_noalloc(ikd_batch_t b, const ikd_tree_t* trees, int
     a.max_steps = (int)std::min<long long>(steps, INT_MAX);
     a.nodes = nodes;
     const int stack = std::min(std::max(depth + 2, b->knn_stack), MAX_DEPTH);
-    const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq, k_max, nodes), ranges_miss);
+    const int lanes = knn_lanes_for(b->knn_lanes >= 0 ? b->knn_lanes : auto_lanes((int)nq, k_max, steps), ranges_miss);
     if (launch_knn(a, k_max, lanes, stack, b->st, ctrl, 256 * 10) != 0) {
         b->err = "batch (no-alloc): unsupported launch shape";
         return IKD_ERR_UNSUPPORTED;
@@ -2944,7 +2945,7 @@ int ikd_batch_knn_graph_create(ikd_batch_t b, const ikd_tree_t* trees, int ntree
             return IKD_ERR_UNSUPPORTED;
         }
         depth = std::max(depth, trees[i]->max_depth);
-        nodes += trees[i]->pool_used;
+        nodes = std::max(nodes, trees[i]->pool_used);
     }
     ikd_knn_graph_t g = new ikd_knn_graph_s();
     g->b = b;
