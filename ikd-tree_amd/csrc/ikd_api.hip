@@ -311,6 +311,7 @@ struct ikd_batch_s {
     hipStream_t st = nullptr;
     std::shared_ptr<BatchEvent> done = std::make_shared<BatchEvent>();  // behind the last launch
     uint64_t serial = 0;  // names the batch in the trees it read
+    bool stream_shared = false;  // the caller has the stream (ikd_batch_stream) and may capture it
     std::string err;
     int knn_lanes = -1;
     int knn_stack = 0;
@@ -2550,6 +2551,7 @@ struct LaunchOrder {
     bool captured = false;  // into a graph of the caller's: it runs when the caller replays it, nothing is ordered now
     std::vector<const BatchEvent*> waited;  // other batches' launches it is behind
     explicit LaunchOrder(ikd_batch_t b) {
+        if (!b->stream_shared) return;
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
         captured = hipStreamIsCapturing(b->st, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
     }
@@ -2563,13 +2565,20 @@ static int order_after_tree(ikd_batch_t b, ikd_tree_t tr, LaunchOrder& order) {
     auto* t = b;
     if (order.captured) return IKD_OK;
     auto& waited = order.waited;
-    // a tree that is only searched keeps no event of a closed batch
-    tr->after.erase(std::remove_if(tr->after.begin(), tr->after.end(), [](const auto& e) { return e->over.load(); }),
-                    tr->after.end());
-    for (const auto& e : tr->after) {
-        if (e == b->done || std::find(waited.begin(), waited.end(), e.get()) != waited.end()) continue;
-        HIPCHK(hipStreamWaitEvent(b->st, e->ev, 0));
-        waited.push_back(e.get());
+    for (size_t i = 0; i < tr->after.size();) {
+        const BatchEvent* e = tr->after[i].get();
+        if (e != b->done.get()) {
+            if (e->over) {  // a tree that is only searched keeps no event of a closed batch
+                tr->after[i].swap(tr->after.back());
+                tr->after.pop_back();
+                continue;
+            }
+            if (std::find(waited.begin(), waited.end(), e) == waited.end()) {
+                HIPCHK(hipStreamWaitEvent(b->st, e->ev, 0));
+                waited.push_back(e);
+            }
+        }
+        ++i;
     }
     if (!tr->stream_shared && tr->seen_by == b->serial && tr->seen_work == tr->work) return IKD_OK;
     HIPCHK(hipEventRecord(tr->ev, tr->st));
@@ -3125,6 +3134,8 @@ int ikd_batch_synchronize(ikd_batch_t b) {
 
 int ikd_batch_stream(ikd_batch_t b, void** out_stream) {
     if (!b || !out_stream) return IKD_ERR_ARG;
+    std::lock_guard<std::mutex> batch_lock_(b->mu);
+    b->stream_shared = true;
     *out_stream = (void*)b->st;
     return IKD_OK;
 }
