@@ -765,7 +765,7 @@ def knn_kernel_name(k, lanes, lds_levels=0, compact=1):
     if lanes == 1:
         if lds_levels > 0:
             return f"ikd::k_knn_staged<{knn_bucket(k)}>"
-        return f"ikd::k_knn<{knn_bucket(k)}, {'true' if compact else 'false'}, false>"
+        return f"ikd::k_knn<{knn_bucket(k)}, {1 if compact else 0}, false>"
     if lanes == 0:
         return f"ikd::k_knn_persist<{knn_bucket(k)}>"
     if lanes < 0:

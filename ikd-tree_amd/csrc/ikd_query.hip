@@ -13,7 +13,11 @@
 // (d2, x, y, z, id), and a child is pruned only when its box distance is
 // strictly greater than the k-th d2.  The result is therefore the k smallest
 // live points under that order, whatever the tree's shape: identical for any
-// layout, batch composition or launch configuration.  Against the reference
+// layout, batch composition or launch configuration.  (Where Add_Point_Boxes has
+// left stored ranges that miss points below them, that does not hold, and what a
+// walk finds depends on its order: such trees are walked by one lane per query in
+// the reference's order with exact distances, k_knn with STACK_EXACT, whatever
+// entry point or configuration asks.)  Against the reference
 // the squared distances agree bit for bit; only which of several points tied
 // at the k-th distance is returned can differ (its choice follows its
 // traversal order).  Output is ascending in the same order, which on exact
@@ -208,7 +212,7 @@ __device__ __forceinline__ void children(const QueryCtx& c, float link, const gv
 // around, and an offer is medians and selects: about 85 vector instructions a
 // visit where it was 154, with the vector units 86 % busy (2M points, 1.18M
 // queries, k = 5: one launch alone 492 -> 447 us; what is left is the latency
-// of gathers that miss L1 (18 %) and L2 (19 %)).
+// of gathers that miss L1 (18 %) and L2 (18 % of those)).
 template <int KM, bool COUNT>
 __device__ __forceinline__ void visit_node(const QueryCtx& c, BestList<KM>& best, int n, float cap, float& lim,
                                            int& near_n, float& dn, int& far_n, float& df, unsigned int& boxes) {
@@ -287,9 +291,6 @@ __device__ __forceinline__ int knn_root(const QueryCtx& c) {
     return calc_box_dist(c.hot[SENTINEL].f + 4, c.qx, c.qy, c.qz) <= c.thr ? ROOT : -1;
 }
 
-// The lane's next deferred child that can still improve (-1: none left).
-// Entries were within max_dist's threshold when they were pushed, and a stored
-// distance never exceeds the exact one.
 template <int FORM>
 __device__ __forceinline__ void knn_push(const LdsStack& st, uint32_t* cst, int at, int n, float d) {
     if (FORM == STACK_COMPACT) {
@@ -300,6 +301,9 @@ __device__ __forceinline__ void knn_push(const LdsStack& st, uint32_t* cst, int 
         else st.d[at] = dist_key(d);
     }
 }
+// The lane's next deferred child that can still improve (-1: none left).
+// Entries were within max_dist's threshold when they were pushed, and a stored
+// distance never exceeds the exact one.
 template <int FORM>
 __device__ __forceinline__ int knn_pop(const LdsStack& st, const uint32_t* cst, int lane, int& sp, float kth) {
     while (sp > 0) {

@@ -180,7 +180,10 @@ int ikd_device_bytes(ikd_tree_t t, int64_t* out_bytes);
  *  IKD_TUNE_LANES_PER_QUERY -1 (default: from the batch size); 0 persistent
  *                       lanes (one query per lane at a time, idle lanes fetch
  *                       the next query); or 1, 2, 4, 8, 16 lanes sharing one
- *                       query's traversal (64 / lanes queries per wavefront). */
+ *                       query's traversal (64 / lanes queries per wavefront).
+ *                       A tree that Add_Point_Boxes has restored points in is
+ *                       searched by one lane per query, in the reference's
+ *                       order, until its root is rebuilt or it is built anew. */
 #define IKD_TUNE_QUERY_ORDER 1
 #define IKD_TUNE_KNN_STACK 2
 #define IKD_TUNE_LANES_PER_QUERY 3
@@ -254,7 +257,10 @@ const char* ikd_last_error(ikd_tree_t t);
 /* ---- Multi-tree batches (no counterpart in the reference: the batched form
  * of Nearest_Search, ikd_Tree.cpp:366-397, over many trees in one launch). ---
  * A batch owns a stream.  A launch waits for the pending work of every tree
- * it reads, and every such tree's later work waits for the launch. */
+ * it reads and for launches of other batches that read one of them, and every
+ * such tree's later work waits for the launch.  A launch that the caller
+ * captures from the batch's stream orders nothing: its replays are the
+ * caller's to order. */
 typedef struct ikd_batch_s* ikd_batch_t;
 int ikd_batch_create(ikd_batch_t* out);
 int ikd_batch_destroy(ikd_batch_t b);
