@@ -1588,7 +1588,10 @@ int auto_lanes(int nq, int k, long long nodes) {
 // distance can admit one that it leaves out.  There one lane per query walks in
 // the reference's order with exact distances (KnnArgs::exact_stack).  It costs what
 // the team saves: 3000 queries of a 1M LiDAR map take 81 us for k = 1 and 152 for
-// k = 5 (teams 29 and 43), 400k queries, which have a lane each anyway, 163 and 291.
+// k = 5 (teams 29 and 43), 400k queries, which have a lane each anyway, 163 and 291.  A launch over several trees with one
+// such takes one lane for all (16 maps of 100k points, 3000 queries, k = 5: 92 us,
+// 50 without it): teams for the others' queries in a launch of their own before it
+// took 127, since each of the two lasts as long as its longest walk.
 int knn_lanes_for(int lanes, bool ranges_miss) { return ranges_miss ? 1 : lanes; }
 
 float max_dist_threshold(double max_dist) {
@@ -2928,7 +2931,6 @@ int ikd_batch_knn_graph_create(ikd_batch_t b, const ikd_tree_t* trees, int ntree
     if (!b || !out) return IKD_ERR_ARG;
     *out = nullptr;
     std::lock_guard<std::mutex> batch_lock_(b->mu);
-    auto* t = b;  // HIPCHK reports into b->err
     if (!trees || ntrees <= 0 || nq <= 0 || nq >= (1ll << 31)) {
         b->err = "recorded kNN: bad tree list or query count";
         return IKD_ERR_ARG;

@@ -12,7 +12,12 @@ extern "C" long long emu_dispatch_tally(char* buf, int len);
 
 static char g_buf[1 << 16];
 
-// 't': a team walked, 'e': one lane with exact distances, '?': neither or both
+// 't': a team walked, 'e': one lane with exact distances, 'b': both, '?': neither
+static char walked() {
+    emu_dispatch_tally(g_buf, sizeof(g_buf));
+    const bool team = std::strstr(g_buf, "k_knn_team") != nullptr, exact = std::strstr(g_buf, "STACK_EXACT") != nullptr;
+    return team ? (exact ? 'b' : 't') : (exact ? 'e' : '?');
+}
 static char walk(ikd_tree_t t) {
     const float q[3] = {1, 2, 3};
     float xyz[15], d2[5];
@@ -20,9 +25,18 @@ static char walk(ikd_tree_t t) {
     int32_t cnt;
     emu_dispatch_reset();
     if (ikd_nearest_search(t, q, 1, 5, 1e9, xyz, d2, ids, &cnt) != IKD_OK) return '?';
-    emu_dispatch_tally(g_buf, sizeof(g_buf));
-    const bool team = std::strstr(g_buf, "k_knn_team") != nullptr, exact = std::strstr(g_buf, "STACK_EXACT") != nullptr;
-    return team == exact ? '?' : (team ? 't' : 'e');
+    return walked();
+}
+// the same of a launch over n trees
+static char walk_batch(ikd_batch_t b, const ikd_tree_t* trees, int n) {
+    static float q[30], xyz[150], d2[50];
+    static uint32_t ids[50];
+    static int32_t cnt[10], which[10];
+    for (int i = 0; i < 10; ++i) which[i] = i % n;
+    emu_dispatch_reset();
+    if (ikd_batch_nearest_search_device(b, trees, n, which, q, 10, nullptr, 5, nullptr, 1e9, xyz, d2, ids, cnt) != IKD_OK)
+        return 'x';
+    return walked();
 }
 
 #define REQUIRE(x)                                      \
@@ -52,6 +66,14 @@ int main() {
     REQUIRE(ikd_add_point_boxes(t, away, 1) == IKD_OK && walk(t) == 't');  // restores nothing
     REQUIRE(ikd_add_point_boxes(t, back, 1) == IKD_OK && walk(t) == 'e');
     REQUIRE(ikd_add_points(t, p.data(), nullptr, 1, 0, &n) == IKD_OK && walk(t) == 'e');
+    // a launch over several trees with one such
+    ikd_tree_t other;
+    ikd_batch_t b;
+    REQUIRE(ikd_create(0.5f, 0.6f, 0.2f, &other) == IKD_OK && ikd_build(other, p.data(), nullptr, 600) == IKD_OK);
+    REQUIRE(ikd_batch_create(&b) == IKD_OK);
+    const ikd_tree_t both[2] = {other, t};
+    REQUIRE(walk_batch(b, both, 1) == 't' && walk_batch(b, both + 1, 1) == 'e' && walk_batch(b, both, 2) == 'e');
+    REQUIRE(ikd_batch_destroy(b) == IKD_OK && ikd_destroy(other) == IKD_OK);
     // far more points on one side: the root is rebuilt
     REQUIRE(ikd_add_points(t, far.data(), nullptr, 3000, 0, &n) == IKD_OK && walk(t) == 't');
     REQUIRE(ikd_delete_point_boxes(t, del, 1, &n) == IKD_OK && ikd_add_point_boxes(t, back, 1) == IKD_OK && walk(t) == 'e');

@@ -79,3 +79,52 @@ def test_default_tuning_against_the_oracle(seed):
             assert np.array_equal(res[2].cpu().numpy().view(np.uint32), ids), what
             assert np.array_equal(res[3].cpu().numpy(), cnt), what
     graph.close()
+
+
+@pytest.mark.parametrize("nq", [700, 20000])
+def test_one_such_tree_among_others(nq):
+    """A call over several trees of which none, one or all are such trees."""
+    import torch
+
+    ikd = importlib.import_module("ikd-tree_amd")
+    dev = torch.device("cuda" if torch.cuda.is_available() else "cpu")
+    rng = np.random.default_rng(nq)
+    trees = []
+    for n in (3000, 5000, 400):
+        t = ikd.KD_TREE(1.0, 1.0, 0.5)
+        t.Build(uniform_cloud(rng, n, -8, 8))
+        trees.append(t)
+    k = 5
+    q = uniform_cloud(rng, nq, -9, 9)
+    qt = rng.integers(-1, 4, nq).astype(np.int32)  # -1 and 3 name no tree
+    dq, dt = torch.from_numpy(q).to(dev), torch.from_numpy(qt).to(dev)
+    outs = [(torch.zeros((nq, k, 3), device=dev), torch.zeros((nq, k), device=dev),
+             torch.zeros((nq, k), dtype=torch.int32, device=dev), torch.zeros(nq, dtype=torch.int32, device=dev))
+            for _ in range(3)]
+    if dev.type == "cuda":
+        torch.cuda.synchronize()
+    b = ikd.Batch()
+    graph = b.knn_graph(trees, dt, dq, k, *outs[2])
+    for lists in ((), (1,), (0, 1, 2)):  # the trees whose ranges miss points
+        for i in lists:
+            trees[i].Delete_Point_Boxes(random_boxes(rng, 1, -8, 8, 3, 8))
+            trees[i].Add_Point_Boxes(random_boxes(rng, 2, -8, 8, 3, 10))
+        for o in outs:
+            for x in o:
+                x.fill_(-7)
+        if dev.type == "cuda":
+            torch.cuda.synchronize()
+        b.nearest_search_device(trees, dt, dq, k, *outs[0])
+        b.nearest_search_noalloc(trees, dt, dq, k, *outs[1])
+        graph.launch()
+        b.synchronize()
+        for what, o in zip(("batch", "no-alloc", "recorded"), outs):
+            d2, ids, cnt = (x.cpu().numpy() for x in o[1:])
+            assert np.all(cnt[(qt < 0) | (qt > 2)] == 0), what
+            for i, t in enumerate(trees):
+                at = np.nonzero(qt == i)[0]
+                _, wd2, wids, wcnt = t.knn(q[at], k)
+                assert np.array_equal(cnt[at], wcnt), f"{what} {lists}"
+                assert np.array_equal(d2[at].view(np.uint32), wd2.view(np.uint32)), f"{what} {lists}"
+                assert np.array_equal(ids[at].view(np.uint32), wids), f"{what} {lists}"
+    graph.close()
